@@ -36,112 +36,12 @@
 #include <mutex>
 #include <type_traits>
 
-#include "rhip_internal.hpp"
+#include "conv_thin.hpp"
 
 namespace rhip {
 
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef uint32_t v2u __attribute__((ext_vector_type(2)));
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-
-// LDS transpose read: within a 16-lane group, lane i receives the (i % 4)-th
-// 16-bit element at the address of lane 4e + i/4 as element e.
-typedef short v4s __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) v4s lds_v4s;
-
-__device__ __forceinline__ v4s ds_read_tr16(const void *p) {
-  // generic LDS pointer -> LDS address space (the low 32 bits are the offset)
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      reinterpret_cast<lds_v4s *>(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p))));
-}
-
-constexpr int kThreads = 256;
-constexpr int kWaves = kThreads / kWave;
 constexpr int kMaskWords = 4; // the MFMA paths handle K <= 128 offsets
 constexpr int kWideRG = 2;    // row groups per wave of conv_os_lds_kernel's bf16 128-column tiles
-
-template <typename T> struct Mfma;
-
-// v_mfma_f32_16x16x4_f32: lane l supplies A[l%16][l/16], B[l/16][l%16];
-// D[4*(l/16)+e][l%16] lands in element e. A 16-byte lane load covers four
-// consecutive channels, consumed by four MFMAs.
-template <> struct Mfma<float> {
-  static constexpr int kCh = 16; // channels per wave-wide 16-byte load
-  using Frag = v4f;
-  __device__ static __forceinline__ Frag load(const float *p) {
-    return *reinterpret_cast<const v4f *>(p);
-  }
-  __device__ static __forceinline__ Frag zero() { return v4f{0.f, 0.f, 0.f, 0.f}; }
-  // v where keep, else zeros (bitwise, so the load it masks stays unconditional)
-  __device__ static __forceinline__ Frag mask(const Frag &v, bool keep) {
-    const uint32_t m = keep ? ~0u : 0u;
-    uint4 u = __builtin_bit_cast(uint4, v);
-    u.x &= m, u.y &= m, u.z &= m, u.w &= m;
-    return __builtin_bit_cast(Frag, u);
-  }
-  __device__ static __forceinline__ void mma(const Frag &a, const Frag &b, v4f &c) {
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[0], b[0], c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[1], b[1], c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[2], b[2], c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[3], b[3], c, 0, 0, 0);
-  }
-};
-
-// v_mfma_f32_16x16x32_bf16 (gfx950): lane l supplies eight consecutive
-// reduction elements of row l%16 (A) / column l%16 (B), group l/16.
-template <> struct Mfma<__bf16> {
-  static constexpr int kCh = 32;
-  using Frag = v8bf;
-  __device__ static __forceinline__ Frag load(const __bf16 *p) {
-    return *reinterpret_cast<const v8bf *>(p);
-  }
-  __device__ static __forceinline__ Frag zero() {
-    return __builtin_bit_cast(v8bf, uint4{0u, 0u, 0u, 0u});
-  }
-  __device__ static __forceinline__ void mma(const Frag &a, const Frag &b, v4f &c) {
-    c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-  }
-  // v where keep, else zeros (bitwise, so the load it masks stays unconditional)
-  __device__ static __forceinline__ Frag mask(const Frag &v, bool keep) {
-    const uint32_t m = keep ? ~0u : 0u;
-    uint4 u = __builtin_bit_cast(uint4, v);
-    u.x &= m, u.y &= m, u.z &= m, u.w &= m;
-    return __builtin_bit_cast(Frag, u);
-  }
-};
-
-__device__ __forceinline__ float to_f32(float v) { return v; }
-__device__ __forceinline__ float to_f32(__bf16 v) { return static_cast<float>(v); }
-template <typename T> __device__ __forceinline__ T from_f32(float v);
-template <> __device__ __forceinline__ float from_f32<float>(float v) { return v; }
-template <> __device__ __forceinline__ __bf16 from_f32<__bf16>(float v) {
-  return static_cast<__bf16>(v);
-}
-
-// Raw buffer loads (stride 0): a load at a byte offset at or past the
-// buffer's size returns zero without a memory access, so an absent row needs
-// no predicate. Kernels put such offsets at kBufOob, past every buffer they
-// make (host code keeps buffers below kBufMaxBytes).
-constexpr uint32_t kBufOob = 0x80000000u;
-constexpr int64_t kBufMaxBytes = (int64_t(1) << 31) - 256; // offsets stay below kBufOob
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *p, int64_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, static_cast<int>(bytes),
-                                           0x00020000);
-}
-
-// A value the optimiser cannot see through: keeps `load | mask` a bitwise
-// OR instead of a select that would become a branch around the load.
-__device__ __forceinline__ int32_t opaque(int32_t v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
-
-// off where keep is all ones, else kBufOob (keep is 0 or -1)
-__device__ __forceinline__ uint32_t pick_off(uint32_t off, int32_t keep) {
-  return (off & static_cast<uint32_t>(keep)) | (kBufOob & ~static_cast<uint32_t>(keep));
-}
 
 // Gathered rows in quad order. The L1 serves a vector load four lanes at a
 // time and looks up one cache line per distinct line among them; in the MFMA
@@ -2704,10 +2604,6 @@ __global__ __launch_bounds__(kThreads) void colsum_final_kernel(const float *__r
   out[c] = v;
 }
 
-static bool aligned16(const void *p) {
-  return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
-}
-
 template <typename T> constexpr int kChOf = Mfma<T>::kCh;
 template <typename T> constexpr bool kIsF32 = std::is_same<T, float>::value;
 
@@ -2810,13 +2706,27 @@ static void pick_csub(const T *x, int cred, const T *wt, int credw, int ncols,
                            partial, s);
 }
 
+// Whether the tiled MFMA kernels take a reduction of cred channels (credw
+// with its padding) to ncols columns over K offsets.
+template <typename T> static bool os_shape(int cred, int credw, int ncols, int K) {
+  const bool red = cred == credw ? cred % kChOf<T> == 0
+                                 : (!kIsF32<T> && credw == cred + 16 && credw % kChOf<T> == 0);
+  return red && ncols % 16 == 0 && K <= 32 * kMaskWords;
+}
+
 // Whether run_os takes the MFMA kernel for these operands (a padded bf16
 // reduction needs 16-byte aligned rows of 16 channels at least).
 template <typename T>
 static bool os_fast(const T *x, int cred, const T *wt, int credw, int ncols, int K) {
-  const bool red = cred == credw ? cred % kChOf<T> == 0
-                                 : (!kIsF32<T> && credw == cred + 16 && credw % kChOf<T> == 0);
-  return red && ncols % 16 == 0 && K <= 32 * kMaskWords && aligned16(x) && aligned16(wt);
+  return os_shape<T>(cred, credw, ncols, K) && aligned16(x) && aligned16(wt);
+}
+
+// The thin kernels' part: shapes the tiled kernels do not take, up to
+// kThinMaxCols im2col columns (a 3^3 layer of 37 channels).
+template <typename T>
+static bool os_thin(int64_t n_x, int cred, int ncols, int K) {
+  const int32_t dt = kIsF32<T> ? RHIP_F32 : RHIP_BF16;
+  return !os_shape<T>(cred, red_width(dt, cred), ncols, K) && conv_thin_takes(K, cred, n_x, sizeof(T));
 }
 
 // Splits of the offset axis for the MFMA kernel: a map with few rows and
@@ -3231,6 +3141,14 @@ static int dw_width(int c) { return c % 64 == 0 ? 4 : (c % 32 == 0 ? 2 : 1); }
 // counts (most workgroups idle), 15.5 at 3 waves per SIMD, 15.9-18.7 with
 // rows 2 to 4 steps ahead, and 36.3 for conv_dw_kernel.
 constexpr int kDwPairsD = 1, kDwPairsWaves = 2;
+// dW's: channel counts that neither the table's nor the pair lists' tiled
+// kernels take.
+static bool dw_thin(int32_t dtype, int cin, int cout, int K, int64_t n_in, int64_t n_out) {
+  const int s = dtype == RHIP_F32 ? 4 : 2;
+  return !(cin % 16 == 0 && cout % 16 == 0) && cout <= kThinMaxCols &&
+         conv_thin_takes(K, cin, n_in, s) && n_out * cout * s <= kBufMaxBytes;
+}
+
 static DwPlan dw_plan(int32_t dtype, int cin, int cout, int K, int64_t n_pairs, int64_t n_in,
                       int64_t n_out, int wgs = 0) {
   DwPlan p;
@@ -3679,8 +3597,12 @@ static ConvWs carve_conv_front(Carve &cv, int32_t K, int32_t cin, int32_t cout, 
 static ConvWs carve_conv(Carve &cv, int32_t K, int32_t cin, int32_t cout, int32_t dtype,
                          int64_t n_in, int64_t n_out, const DwPlan &p) {
   ConvWs w = carve_conv_front(cv, K, cin, cout, dtype, n_in, n_out);
+  const size_t thin = dw_thin(dtype, cin, cout, K, n_in, n_out)
+                          ? static_cast<size_t>(conv_dw_thin_ranges(K, cin, cout, n_out)) * K *
+                                cin * cout
+                          : 0;
   w.partial = cv.take<float>(std::max<size_t>(
-      {1, p.partial_floats() * K, dw_table_floats(dtype, cin, cout, K, n_in, n_out)}));
+      {1, p.partial_floats() * K, dw_table_floats(dtype, cin, cout, K, n_in, n_out), thin}));
   w.acc = cv.take<float>(static_cast<size_t>(K) * cin * cout);
   return w;
 }
@@ -3691,6 +3613,18 @@ static void conv_forward_into(const void *x, int64_t n_in, int32_t cin, const vo
                               int32_t K, int32_t cout, const float *bias, const int32_t *nbr,
                               const int32_t *out_order, int64_t n_out, void *y, int32_t dtype,
                               void *wt, float *os_partial, hipStream_t stream) {
+  auto thin = [&](auto *xt) {
+    using T = std::remove_const_t<std::remove_pointer_t<decltype(xt)>>;
+    if (!os_thin<T>(n_in, cin, cout, K))
+      return false;
+    conv_thin<T>(xt, n_in, cin, static_cast<const T *>(weight), static_cast<int64_t>(cin) * cout,
+                 cout, 1, nullptr, cout, bias, nbr, n_out, K, out_order, static_cast<T *>(y),
+                 stream);
+    return true;
+  };
+  if (dtype == RHIP_F32 ? thin(static_cast<const float *>(x))
+                        : thin(static_cast<const __bf16 *>(x)))
+    return;
   // the MFMA path reads W[k] column-wise: stage the [K, cout, credw] copy
   const int credw = red_width(dtype, cin);
   const int64_t nw = static_cast<int64_t>(K) * cout * credw;
@@ -3916,6 +3850,18 @@ extern "C" int rhip_conv_backward_input(const void *grad_y, int64_t n_out,
       return;
     RHIP_CHECK_ARG(grad_x && weight && nbr_t, "grad_x, weight and nbr_t are required");
     RHIP_CHECK_ARG(n_out == 0 || grad_y != nullptr, "grad_y is null");
+    auto thin = [&](auto *gy) {
+      using T = std::remove_const_t<std::remove_pointer_t<decltype(gy)>>;
+      if (workspace == nullptr || !os_thin<T>(n_out, cout, cin, K))
+        return false;
+      conv_thin<T>(gy, n_out, cout, static_cast<const T *>(weight),
+                   static_cast<int64_t>(cin) * cout, 1, cout, weight_perm, cin, nullptr, nbr_t,
+                   n_in, K, in_order, static_cast<T *>(grad_x), stream);
+      return true;
+    };
+    if (dtype == RHIP_F32 ? thin(static_cast<const float *>(grad_y))
+                          : thin(static_cast<const __bf16 *>(grad_y)))
+      return;
     // without a workspace the offset axis is not split, and a reduction the
     // MFMA kernels would pad goes to the one-lane-per-output kernel
     float *os_partial = nullptr;
@@ -4026,4 +3972,42 @@ extern "C" int rhip_conv_backward_weight_rows_supported(int32_t dtype, int32_t c
       n_out < 0)
     return 0;
   return dw_rows_supported(dtype, cin, cout, K, n_in, n_out) ? 1 : 0;
+}
+
+extern "C" int rhip_conv_backward_weight_thin(
+    const void *x, int64_t n_in, int32_t cin, const void *grad_y, int64_t n_out, int32_t cout,
+    int32_t K, const int32_t *nbr, const int32_t *out_order, void *grad_w, int32_t dtype,
+    void *workspace, size_t workspace_bytes, hipStream_t stream) {
+  return guarded([&] {
+    check_dtype(dtype);
+    RHIP_CHECK_ARG(K >= 1 && cin >= 1 && cout >= 1, "sizes must be positive");
+    RHIP_CHECK_ARG(n_in >= 0 && n_out >= 0, "bad sizes");
+    if (!dw_thin(dtype, cin, cout, K, n_in, n_out))
+      throw Error(RHIP_ERR_UNSUPPORTED,
+                  "rhip_conv_backward_weight_thin: channel counts that are not both multiples of "
+                  "16, offsets times input channels of at most " + std::to_string(kThinMaxCols) +
+                  " (use rhip_conv_backward_weight)");
+    RHIP_CHECK_ARG(grad_w != nullptr, "grad_w is null");
+    RHIP_CHECK_ARG(n_out == 0 || (grad_y && nbr), "grad_y and nbr are required");
+    RHIP_CHECK_ARG(n_in == 0 || n_out == 0 || x, "x is null");
+    RHIP_CHECK_ARG(workspace != nullptr, "workspace is null");
+    Carve cv(workspace, workspace_bytes);
+    const ConvWs w = carve_conv(cv, K, cin, cout, dtype, n_in, n_out, DwPlan{});
+    if (dtype == RHIP_F32)
+      conv_dw_thin<float>(static_cast<const float *>(x), n_in, cin,
+                          static_cast<const float *>(grad_y), cout, nbr, n_out, K, out_order,
+                          w.partial, static_cast<float *>(grad_w), stream);
+    else
+      conv_dw_thin<__bf16>(static_cast<const __bf16 *>(x), n_in, cin,
+                           static_cast<const __bf16 *>(grad_y), cout, nbr, n_out, K, out_order,
+                           w.partial, static_cast<__bf16 *>(grad_w), stream);
+  });
+}
+
+extern "C" int rhip_conv_backward_weight_thin_supported(int32_t dtype, int32_t cin, int32_t cout,
+                                                        int32_t K, int64_t n_in, int64_t n_out) {
+  if ((dtype != RHIP_F32 && dtype != RHIP_BF16) || K < 1 || cin < 1 || cout < 1 || n_in < 0 ||
+      n_out < 0)
+    return 0;
+  return dw_thin(dtype, cin, cout, K, n_in, n_out) ? 1 : 0;
 }

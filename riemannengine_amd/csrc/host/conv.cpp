@@ -42,20 +42,23 @@ at::Tensor conv_workspace(int32_t K, int64_t cin, int64_t cout, int32_t dt, int6
 using torch::autograd::AutogradContext;
 using torch::autograd::tensor_list;
 
+// Sources of the weight gradient: the pair lists (in_rows, out_rows), or the
+// neighbour table through the tiled or the thin kernels.
+enum DwSource : int64_t { kDwPairs, kDwRows, kDwThin };
+
 // Inputs after (features, kernel, bias) are the kernel map's index tensors;
 // they are integer tensors, so autograd gives them no gradient. bias is fp32
 // [cout], or empty for none (autograd needs a defined tensor for every
 // input); the forward adds it to the fp32 sums before rounding. The input
 // gradient runs on (dx_table, dx_order) with weight slice wperm[k] for table
 // row k (wperm empty: k): the transposed table, or for a symmetric map nbr
-// itself with the stencil partners. pairs_dw: the weight gradient takes the
-// pair lists (in_rows, out_rows), else the neighbour table.
+// itself with the stencil partners. dw: where the weight gradient comes from.
 struct HipConvolutionFunction : public torch::autograd::Function<HipConvolutionFunction> {
   static at::Tensor forward(AutogradContext *ctx, at::Tensor features, at::Tensor kernel,
                             at::Tensor bias, at::Tensor nbr, at::Tensor out_order,
                             at::Tensor dx_table, at::Tensor dx_order, at::Tensor wperm,
                             at::Tensor offsets, at::Tensor in_rows, at::Tensor out_rows,
-                            int64_t n_out, int64_t n_pairs, bool pairs_dw) {
+                            int64_t n_out, int64_t n_pairs, int64_t dw) {
     TORCH_CHECK(features.is_cuda() && kernel.is_cuda(),
                 "features and kernel must be device tensors");
     TORCH_CHECK(features.scalar_type() == kernel.scalar_type(),
@@ -86,7 +89,7 @@ struct HipConvolutionFunction : public torch::autograd::Function<HipConvolutionF
     ctx->save_for_backward({x, w, dx_table, dx_order, offsets, in_rows, out_rows, nbr, out_order,
                             wperm});
     ctx->saved_data["n_pairs"] = n_pairs;
-    ctx->saved_data["pairs_dw"] = pairs_dw;
+    ctx->saved_data["dw"] = dw;
     ctx->saved_data["n_out"] = n_out;
     ctx->saved_data["has_bias"] = has_bias;
     return y;
@@ -97,7 +100,7 @@ struct HipConvolutionFunction : public torch::autograd::Function<HipConvolutionF
     auto x = saved[0], w = saved[1], dx_table = saved[2], dx_order = saved[3];
     auto offsets = saved[4], in_rows = saved[5], out_rows = saved[6];
     auto nbr = saved[7], out_order = saved[8], wperm = saved[9];
-    const bool pairs_dw = ctx->saved_data["pairs_dw"].toBool();
+    const int64_t dw = ctx->saved_data["dw"].toInt();
     const int64_t n_pairs = ctx->saved_data["n_pairs"].toInt();
     const int64_t n_out = ctx->saved_data["n_out"].toInt();
     const auto dev = x.device();
@@ -129,8 +132,8 @@ struct HipConvolutionFunction : public torch::autograd::Function<HipConvolutionF
     if (need_dw) {
       gw = torch::empty_like(w);
       int rc;
-      if (!pairs_dw) {
-        rc = rhip_conv_backward_weight_rows(
+      if (dw != kDwPairs) {
+        rc = (dw == kDwRows ? rhip_conv_backward_weight_rows : rhip_conv_backward_weight_thin)(
             x.data_ptr(), n_in, static_cast<int32_t>(cin), gy.data_ptr(), n_out,
             static_cast<int32_t>(cout), K, nbr.data_ptr<int32_t>(),
             out_order.numel() > 0 ? out_order.data_ptr<int32_t>() : nullptr, gw.data_ptr(), dt,
@@ -143,7 +146,7 @@ struct HipConvolutionFunction : public torch::autograd::Function<HipConvolutionF
                                        in_rows.data_ptr<int32_t>(), out_rows.data_ptr<int32_t>(),
                                        gw.data_ptr(), dt, ws.data_ptr(), ws.numel(), st);
       }
-      check_rhip(rc, "rhip_conv_backward_weight(_rows)");
+      check_rhip(rc, "rhip_conv_backward_weight(_rows, _thin)");
     }
     return {gx, gw, gb, {}, {}, {}, {}, {}, {}, {}, {}, {}, {}, {}};
   }
@@ -161,7 +164,7 @@ at::Tensor hip_sparse_convolution(const at::Tensor &features, const at::Tensor &
       bias.defined() ? bias
                      : torch::empty({0}, features.options().dtype(torch::kFloat));
   // dW from the neighbour table where the library has a kernel for the
-  // shape, else from the pair lists (built now, once per map, when a weight
+  // shape (tiled, or thin for odd channel counts), else from the pair lists (built now, once per map, when a weight
   // gradient may follow). bf16 maps of at most 8 offsets take the pair lists
   // when they hold fewer than 2 pairs per output row (a transposed stride-2
   // map), or pair each input row at most once (a stride-2 map) with channel
@@ -174,13 +177,17 @@ at::Tensor hip_sparse_convolution(const at::Tensor &features, const at::Tensor &
   const bool sparse_small =
       dt == RHIP_BF16 && map.K <= 8 &&
       (map.size() < 2 * map.n_out || (map.size() <= map.n_in && kin % 64 == 0 && kout % 64 == 0));
-  const bool pairs_dw =
-      sparse_small || rhip_conv_backward_weight_rows_supported(
-                          dt, static_cast<int32_t>(kernel.size(1)),
-                          static_cast<int32_t>(kernel.size(2)), map.K, map.n_in, map.n_out) == 0;
+  const int32_t cin = static_cast<int32_t>(kin), cout = static_cast<int32_t>(kout);
+  const int64_t dw =
+      !sparse_small &&
+              rhip_conv_backward_weight_rows_supported(dt, cin, cout, map.K, map.n_in, map.n_out)
+          ? kDwRows
+      : rhip_conv_backward_weight_thin_supported(dt, cin, cout, map.K, map.n_in, map.n_out)
+          ? kDwThin
+          : kDwPairs;
   const auto iempty = torch::empty({0}, map.nbr.options());
   at::Tensor in_rows = iempty, out_rows = iempty;
-  if (pairs_dw && kernel.requires_grad() && torch::autograd::GradMode::is_enabled()) {
+  if (dw == kDwPairs && kernel.requires_grad() && torch::autograd::GradMode::is_enabled()) {
     map.ensure_pairs();
     in_rows = map.in_rows;
     out_rows = map.out_rows;
@@ -188,10 +195,10 @@ at::Tensor hip_sparse_convolution(const at::Tensor &features, const at::Tensor &
   if (!map.symmetric)
     return HipConvolutionFunction::apply(features, kernel, b, map.nbr, map.out_order, map.nbr_t,
                                          map.in_order, iempty, map.offsets, in_rows, out_rows,
-                                         map.n_out, map.size(), pairs_dw);
+                                         map.n_out, map.size(), dw);
   return HipConvolutionFunction::apply(features, kernel, b, map.nbr, map.out_order, map.nbr,
                                        map.out_order, map.partner, map.offsets, in_rows, out_rows,
-                                       map.n_out, map.size(), pairs_dw);
+                                       map.n_out, map.size(), dw);
 }
 
 // ------------------------------------------------------------ layers
