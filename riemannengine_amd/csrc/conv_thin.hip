@@ -67,66 +67,137 @@ __device__ __forceinline__ bool piece_bad(const typename PieceOf<PB>::type &v) {
     return word_bad<T>(v);
 }
 
-// Columns [r0, r0 + rlen) of the im2col rows of positions pos0 .. pos0 + 63
-// to LDS rows of LDA elements: pieces of PB bytes, ppr per feature row of C
-// channels; piece q of a position is piece q % ppr of offset q / ppr (div:
-// ceil(2^20 / ppr)). Missing neighbours, positions past the end and columns
-// past the last offset give zeros without a memory access. idx(k, position):
-// the feature row or -1. Pieces under 16 bytes go position-fastest (the
-// table reads are then coalesced; 16-byte pieces go piece-fastest, so that a
-// wave reads whole rows. Returns whether a value read was not finite (CHECK).
-template <typename T, int PB, int LDA, bool CHECK, typename Idx>
-__device__ __forceinline__ bool gather_tile(T *s, __amdgpu_buffer_rsrc_t rx, int64_t pos0,
-                                            int64_t n_rows, int r0, int rlen, int K, int C,
-                                            int ppr, uint32_t div, Idx &&idx) {
+// How a layer's im2col columns split into LDS chunks of at most kRC: up to kc
+// whole offsets each, or for C > kRC one offset's channels in `parts` parts
+// of cw (a multiple of 32, the last one shorter).
+struct Thin {
+  int K, C;
+  int ppr;       // pieces per feature row
+  uint32_t div;  // ceil(2^20 / ppr): piece -> offset
+  uint32_t cdiv; // ceil(2^20 / C): column -> offset
+  int kc, parts, cw, chunks;
+  int64_t blocks; // position tiles
+};
+struct Chunk {
+  int k0, kn, c0, cw; // offsets k0 .. k0 + kn - 1, channels c0 .. c0 + cw - 1
+  __device__ int cols() const { return kn * cw; }
+};
+__device__ __forceinline__ Chunk chunk_of(const Thin &th, int ch) {
+  if (th.parts == 1)
+    return {ch * th.kc, min(th.kc, th.K - ch * th.kc), 0, th.C};
+  const int c0 = (ch % th.parts) * th.cw;
+  return {ch / th.parts, 1, c0, min(th.cw, th.C - c0)};
+}
+// the offset of column r of a chunk
+__device__ __forceinline__ int offset_of(const Thin &th, const Chunk &c, int r) {
+  return c.k0 + (c.kn == 1 ? 0 : static_cast<int>((static_cast<uint32_t>(r) * th.cdiv) >> 20));
+}
+
+// A chunk's im2col columns of positions pos0 .. pos0 + 63 to LDS rows of LDA
+// elements. Missing
+// neighbours, and with TAIL positions past the end, give zeros without a
+// memory access (a row index past the buffer's last). idx(k, position): the
+// feature row or -1. Pieces under 16 bytes: lane = position and wave w the
+// offsets w, w + 4, ..., so that the table reads are coalesced and an
+// offset's row address serves all its pieces; 16-byte pieces go piece-fastest,
+// so that a wave reads whole rows. Returns whether a value read was not
+// finite (CHECK).
+template <typename T, int PB, int LDA, bool CHECK, bool TAIL, typename Idx>
+__device__ __forceinline__ bool gather_tile(T *s, __amdgpu_buffer_rsrc_t rx, uint32_t n_x,
+                                            int64_t pos0, int64_t n_rows, const Thin &th,
+                                            const Chunk &ck, Idx &&idx) {
   constexpr int VE = PB / sizeof(T);
-  constexpr int U = 8; // pieces in flight per thread
-  const int q0 = r0 / VE, qn = rlen / VE;
-  const uint32_t row_bytes = static_cast<uint32_t>(C * sizeof(T));
+  constexpr int U = 8; // loads in flight per thread
+  const uint32_t row_bytes = static_cast<uint32_t>(th.C * sizeof(T));
+  const uint32_t c0_bytes = static_cast<uint32_t>(ck.c0 * sizeof(T));
+  const int k0 = ck.k0, kn = ck.kn;
+  const int tid = threadIdx.x;
   bool bad = false;
-  // thread's j-th piece: position p, piece q0 + i of the chunk
-  auto run = [&](int count, auto &&at) {
-    for (int j0 = 0; j0 < count; j0 += U) {
-      int32_t id[U];
-      int p[U], i[U];
+  if constexpr (PB < 16) {
+    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int p = tid & (kSeg - 1);
+    const int64_t pos = min(pos0 + p, n_rows - 1);
+    const int32_t in = TAIL && pos0 + p >= n_rows ? -1 : 0;
+    if (kn < kWaves) { // few offsets: the waves share out their pieces
+      const int ppc = ck.cw / VE, items = kn * ppc;
+      for (int j0 = wv; j0 < items; j0 += kWaves * U) {
+        uint32_t off[U];
+        T *dst[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) { // past the last piece: the last one again
+          const int j = min(j0 + kWaves * u, items - 1);
+          const int k = (j >= ppc ? 1 : 0) + (j >= 2 * ppc ? 1 : 0), q = j - k * ppc;
+          off[u] = min(static_cast<uint32_t>(idx(k0 + k, pos) | in), n_x) * row_bytes + c0_bytes +
+                   static_cast<uint32_t>(q * PB);
+          dst[u] = s + p * LDA + k * th.C + q * VE;
+        }
+        typename PieceOf<PB>::type v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          v[u] = load_piece<PB>(rx, off[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          store_piece<PB>(dst[u], v[u]);
+          if constexpr (CHECK)
+            bad = bad || piece_bad<PB, T>(v[u]);
+        }
+      }
+      return bad;
+    }
+    for (int j0 = wv; j0 < kn; j0 += kWaves * U) {
+      // past the last offset: the last one again (the same values once more)
       uint32_t off[U];
 #pragma unroll
+      for (int u = 0; u < U; ++u)
+        off[u] = min(static_cast<uint32_t>(idx(k0 + min(j0 + kWaves * u, kn - 1), pos) | in),
+                     n_x) * row_bytes + c0_bytes;
+      T *dst = s + p * LDA;
+      for (int q = 0; q < ck.cw / VE; ++q) {
+        typename PieceOf<PB>::type v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          v[u] = load_piece<PB>(rx, off[u] + static_cast<uint32_t>(q * PB));
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          store_piece<PB>(dst + min(j0 + kWaves * u, kn - 1) * th.C + q * VE, v[u]);
+          if constexpr (CHECK)
+            bad = bad || piece_bad<PB, T>(v[u]);
+        }
+      }
+    }
+  } else {
+    const int qn = kn * (ck.cw / VE); // pieces per position
+    const int sh = 32 - __builtin_clz(max(qn - 1, 1)); // rounded up to a power of two
+    const int count = max((kSeg << sh) / kThreads, 1);
+    for (int j0 = 0; j0 < count; j0 += U) {
+      uint32_t off[U];
+      T *dst[U];
+      bool live[U];
+#pragma unroll
       for (int u = 0; u < U; ++u) {
-        at(j0 + u, p[u], i[u]);
-        const int q = q0 + min(i[u], qn - 1);
-        const int k = static_cast<int>((static_cast<uint32_t>(q) * div) >> 20);
-        const bool in = j0 + u < count && i[u] < qn && k < K && pos0 + p[u] < n_rows;
-        id[u] = idx(min(k, K - 1), min(pos0 + p[u], n_rows - 1)) | (in ? 0 : -1);
-        off[u] = static_cast<uint32_t>((q - k * ppr) * PB);
+        const int e = (j0 + u) * kThreads + tid;
+        const int p = min(e >> sh, kSeg - 1), i = min(e & ((1 << sh) - 1), qn - 1);
+        live[u] = j0 + u < count && (e >> sh) < kSeg && (e & ((1 << sh) - 1)) < qn;
+        const int k = kn == 1 ? 0 : static_cast<int>((static_cast<uint32_t>(i) * th.div) >> 20);
+        const int q = i - k * th.ppr;
+        const int32_t id = idx(k0 + k, min(pos0 + p, n_rows - 1)) |
+                           (live[u] && pos0 + p < n_rows ? 0 : -1);
+        off[u] = min(static_cast<uint32_t>(id), n_x) * row_bytes +
+                 static_cast<uint32_t>(q * PB) + c0_bytes;
+        dst[u] = s + p * LDA + k * th.C + q * VE;
       }
       typename PieceOf<PB>::type v[U];
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        v[u] = load_piece<PB>(rx, pick_off(static_cast<uint32_t>(id[u]) * row_bytes + off[u],
-                                           ~(id[u] >> 31)));
+        v[u] = load_piece<PB>(rx, off[u]);
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        if (j0 + u < count && i[u] < qn) {
-          store_piece<PB>(s + p[u] * LDA + i[u] * VE, v[u]);
+        if (live[u]) {
+          store_piece<PB>(dst[u], v[u]);
           if constexpr (CHECK)
             bad = bad || piece_bad<PB, T>(v[u]);
         }
     }
-  };
-  const int tid = threadIdx.x;
-  if constexpr (PB < 16) {
-    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
-    run((qn - wv + kWaves - 1) / kWaves, [&](int j, int &p, int &i) {
-      p = tid & (kSeg - 1);
-      i = wv + kWaves * j;
-    });
-  } else {
-    const int sh = 32 - __builtin_clz(max(qn - 1, 1)); // pieces rounded up to a power of two
-    run(max((kSeg << sh) / kThreads, 1), [&](int j, int &p, int &i) {
-      const int e = j * kThreads + tid;
-      p = min(e >> sh, kSeg - 1);
-      i = (e >> sh) < kSeg ? e & ((1 << sh) - 1) : qn;
-    });
   }
   return bad;
 }
@@ -137,14 +208,16 @@ __device__ __forceinline__ bool gather_tile(T *s, __amdgpu_buffer_rsrc_t rx, int
 // of A and W go through LDS, W only once where one chunk holds it all.
 // Bound by the latency of a tile's loads (table, then features). Measured on
 // MI355X, kernel alone: a first layer of 194k rows, 3^3, 3->32 bf16, 236 us
-// on the one-lane-per-output kernel, 45 here; a 1^3 layer of 96k rows, 64->20
-// fp32, forward and dX 193 us each, 24 here.
+// on the one-lane-per-output kernel, 31 here (45 with the offset, table index
+// and row address worked out anew for every piece); a 1^3 layer of 96k rows,
+// 64->20 fp32, forward and dX 193 us each, 22 here. 1024 workgroups at most,
+// so that the staged weights serve three tiles or more on a large map.
 template <typename T, int NT, int PB>
 __global__ __launch_bounds__(kThreads) void conv_thin_kernel(
-    const T *__restrict__ x, int64_t n_x, int C, const T *__restrict__ w, int64_t wk, int64_t wc,
-    int64_t wn, const int32_t *__restrict__ wperm, int ncols, const float *__restrict__ bias,
-    const int32_t *__restrict__ nbr, int64_t n_rows, int K, const int32_t *__restrict__ order,
-    T *__restrict__ y, int ppr, uint32_t div, int rc, int chunks) {
+    const T *__restrict__ x, int64_t n_x, const Thin th, const T *__restrict__ w, int64_t wk,
+    int64_t wc, int64_t wn, const int32_t *__restrict__ wperm, int ncols,
+    const float *__restrict__ bias, const int32_t *__restrict__ nbr, int64_t n_rows,
+    const int32_t *__restrict__ order, T *__restrict__ y) {
   using M = Mfma<T>;
   using Frag = typename M::Frag;
   constexpr int CH = M::kCh, EPL = CH / 4;
@@ -157,47 +230,73 @@ __global__ __launch_bounds__(kThreads) void conv_thin_kernel(
   const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int i16 = lane & 15, g = lane >> 4;
   const int col0 = blockIdx.y * NT;
-  const int R = K * C;
-  const __amdgpu_buffer_rsrc_t rx = buf_rsrc(x, n_x * C * static_cast<int64_t>(sizeof(T)));
+  const __amdgpu_buffer_rsrc_t rx = buf_rsrc(x, n_x * th.C * static_cast<int64_t>(sizeof(T)));
   auto idx = [&](int k, int64_t p) { return nbr[k * n_rows + p]; };
   if (tid == 0)
     sbad = 0;
-  const int64_t tiles = (n_rows + kSeg - 1) / kSeg;
-  bool staged = false;
-  for (int64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
+  // the chunk's weights transposed to [n][r], zeros past its columns (up to a
+  // whole MFMA step) and past ncols; the tile's columns past the chunk's zero
+  // too. Consecutive threads go along the contiguous axis of w.
+  auto stage = [&](const Chunk &ck, int ch) {
+    const int cols = ck.cols(), rc = (cols + CH - 1) / CH * CH;
+    constexpr int WU = 8;
+    const int count = wn == 1 ? rc * NT : NT * kRC; // elements, NT or kRC per row
+    for (int e0 = tid; e0 < count; e0 += WU * kThreads) {
+      T v[WU];
+      int at[WU];
+      int k[WU], r[WU], n[WU];
+#pragma unroll
+      for (int i = 0; i < WU; ++i) {
+        const int e = e0 + i * kThreads;
+        n[i] = wn == 1 ? e % NT : e / kRC;
+        r[i] = wn == 1 ? e / NT : e % kRC;
+        const int rr = min(r[i], cols - 1);
+        k[i] = offset_of(th, ck, rr);
+        at[i] = (ck.c0 + rr - (k[i] - ck.k0) * th.C) * static_cast<int>(wc) +
+                min(col0 + n[i], ncols - 1) * static_cast<int>(wn);
+      }
+      if (wperm) {
+#pragma unroll
+        for (int i = 0; i < WU; ++i)
+          k[i] = wperm[k[i]];
+      }
+#pragma unroll
+      for (int i = 0; i < WU; ++i) // at clamped places, all in flight
+        v[i] = w[k[i] * wk + at[i]];
+#pragma unroll
+      for (int i = 0; i < WU; ++i) {
+        const bool in = r[i] < cols && col0 + n[i] < ncols;
+        const float f = to_f32(v[i]);
+        if (in && !(f - f == 0.f))
+          sbad = ch + 1;
+        if (r[i] < rc && n[i] < NT)
+          sB[n[i] * LD + r[i]] = in ? v[i] : from_f32<T>(0.f);
+      }
+    }
+    for (int p = wv; p < kSeg; p += kWaves)
+      if (cols + lane < rc)
+        sA[p * LD + cols + lane] = from_f32<T>(0.f);
+  };
+  for (int64_t t = blockIdx.x; t < th.blocks; t += gridDim.x) {
     const int64_t pos0 = t * kSeg;
     v4f acc[NB];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
       acc[nb] = v4f{0.f, 0.f, 0.f, 0.f};
-    for (int ch = 0; ch < chunks; ++ch) {
-      const int r0 = ch * rc;
+    for (int ch = 0; ch < th.chunks; ++ch) {
+      const Chunk ck = chunk_of(th, ch);
       __syncthreads(); // every wave is done with the previous chunk
-      if (!staged) {
-        // transposed to [n][r], zeros past R and ncols; consecutive threads
-        // along the contiguous axis of w
-        for (int e = tid; e < NT * rc; e += kThreads) {
-          const int n = wn == 1 ? e % NT : e / rc;
-          const int r = wn == 1 ? e / NT : e % rc;
-          T v = from_f32<T>(0.f);
-          if (r0 + r < R && col0 + n < ncols) {
-            const int k = (r0 + r) / C, c = r0 + r - k * C;
-            v = w[(wperm ? wperm[k] : k) * wk + c * wc + (col0 + n) * wn];
-            const float f = to_f32(v);
-            if (!(f - f == 0.f))
-              sbad = ch + 1;
-          }
-          sB[n * LD + r] = v;
-        }
-        staged = chunks == 1;
-      }
-      gather_tile<T, PB, LD, false>(sA, rx, pos0, n_rows, r0, rc, K, C, ppr, div, idx);
+      if (th.chunks > 1 || t == blockIdx.x)
+        stage(ck, ch);
+      // rows past the end repeat the last one; they are not stored
+      gather_tile<T, PB, LD, false, false>(sA, rx, static_cast<uint32_t>(n_x), pos0, n_rows, th,
+                                           ck, idx);
       __syncthreads();
       if (sbad == ch + 1) { // over the pairs that exist only
         for (int e = 0; e < 4; ++e) {
           const int64_t pos = pos0 + 16 * wv + 4 * g + e;
-          for (int r = 0; r < rc && r0 + r < R && pos < n_rows; ++r) {
-            if (nbr[((r0 + r) / C) * n_rows + pos] < 0)
+          for (int r = 0; r < ck.cols() && pos < n_rows; ++r) {
+            if (nbr[offset_of(th, ck, r) * n_rows + pos] < 0)
               continue;
             const float a = to_f32(sA[(16 * wv + 4 * g + e) * LD + r]);
 #pragma unroll
@@ -207,7 +306,8 @@ __global__ __launch_bounds__(kThreads) void conv_thin_kernel(
         }
         continue;
       }
-      for (int s = 0; s < rc; s += CH) {
+#pragma unroll 2
+      for (int s = 0; s < ck.cols(); s += CH) {
         const Frag a = *reinterpret_cast<const Frag *>(&sA[(16 * wv + i16) * LD + s + g * EPL]);
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
@@ -240,12 +340,12 @@ __global__ __launch_bounds__(kThreads) void conv_thin_kernel(
 // row-major LDS tiles through ds_read_b64_tr_b16. Measured on MI355X with the
 // reduction, the layers above: 74.5 ms and 32.3 ms on the pair lists with one
 // lane per element of dW (each lane a serial walk over its offset's pairs),
-// 52 us and 38 us here.
+// 41 us and 34 us here.
 template <typename T, int NT, int PB, int PBY>
 __global__ __launch_bounds__(kThreads) void conv_dw_thin_kernel(
-    const T *__restrict__ x, int64_t n_x, int C, const T *__restrict__ gy, int cout,
-    const int32_t *__restrict__ nbr, int64_t n_rows, int K, const int32_t *__restrict__ order,
-    int ppr, uint32_t div, int rc, int ppy, uint32_t divy, float *__restrict__ partial) {
+    const T *__restrict__ x, int64_t n_x, const Thin th, const T *__restrict__ gy, const Thin ty,
+    const int32_t *__restrict__ nbr, int64_t n_rows, const int32_t *__restrict__ order,
+    float *__restrict__ partial) {
   constexpr int NB = NT / 16;
   constexpr int WPB = kWaves / NB;           // waves per column block
   constexpr int TPW = (kRB + WPB - 1) / WPB; // row blocks per wave
@@ -259,10 +359,11 @@ __global__ __launch_bounds__(kThreads) void conv_dw_thin_kernel(
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int i16 = lane & 15, g = lane >> 4;
-  const int R = K * C;
-  const int r0 = blockIdx.y * rc, n0 = blockIdx.z * NT;
-  const int nrb = (min(rc, R - r0) + 15) / 16;
-  const __amdgpu_buffer_rsrc_t rx = buf_rsrc(x, n_x * C * static_cast<int64_t>(sizeof(T)));
+  const int cout = ty.C, n0 = blockIdx.z * NT;
+  const Chunk ck = chunk_of(th, blockIdx.y);
+  const Chunk cy = {0, 1, n0, min(NT, cout - n0)};
+  const int cols = ck.cols(), nrb = (cols + 15) / 16;
+  const __amdgpu_buffer_rsrc_t rx = buf_rsrc(x, n_x * th.C * static_cast<int64_t>(sizeof(T)));
   const __amdgpu_buffer_rsrc_t ry = buf_rsrc(gy, n_rows * cout * static_cast<int64_t>(sizeof(T)));
   auto idx = [&](int k, int64_t p) { return nbr[k * n_rows + p]; };
   auto row = [&](int, int64_t p) { return order ? order[p] : static_cast<int32_t>(p); };
@@ -273,22 +374,21 @@ __global__ __launch_bounds__(kThreads) void conv_dw_thin_kernel(
     acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
   if (tid == 0)
     sbad = 0;
-  const int64_t segs = (n_rows + kSeg - 1) / kSeg;
-  for (int64_t s = blockIdx.x; s < segs; s += gridDim.x) {
+  for (int64_t s = blockIdx.x; s < th.blocks; s += gridDim.x) {
     __syncthreads(); // every wave is done with the previous segment
-    const bool bad = gather_tile<T, PBY, LDY, true>(sY, ry, s * kSeg, n_rows, n0, NT, 1, cout,
-                                                    ppy, divy, row);
-    if (bad)
+    if (gather_tile<T, PBY, LDY, true, true>(sY, ry, static_cast<uint32_t>(n_rows), s * kSeg,
+                                             n_rows, ty, cy, row))
       sbad = s + 1;
-    gather_tile<T, PB, LDA, false>(sA, rx, s * kSeg, n_rows, r0, rc, K, C, ppr, div, idx);
+    gather_tile<T, PB, LDA, false, true>(sA, rx, static_cast<uint32_t>(n_x), s * kSeg, n_rows, th,
+                                         ck, idx);
     __syncthreads();
     if (sbad == s + 1) { // over the pairs that exist only
       for (int j = 0; j < TPW; ++j)
         for (int e = 0; e < 4; ++e) {
           const int r = 16 * (wv / NB + WPB * j) + 4 * g + e;
-          for (int p = 0; p < kSeg && r < rc && r0 + r < R; ++p) {
+          for (int p = 0; p < kSeg && r < cols; ++p) {
             const int64_t pos = s * kSeg + p;
-            if (pos < n_rows && nbr[((r0 + r) / C) * n_rows + pos] >= 0)
+            if (pos < n_rows && nbr[offset_of(th, ck, r) * n_rows + pos] >= 0)
               acc[j][e] += to_f32(sA[p * LDA + r]) * to_f32(sY[p * LDY + 16 * nb + i16]);
           }
         }
@@ -328,15 +428,16 @@ __global__ __launch_bounds__(kThreads) void conv_dw_thin_kernel(
       }
     }
   }
-  float *slot = partial + static_cast<int64_t>(blockIdx.x) * R * cout;
+  float *slot = partial + (static_cast<int64_t>(blockIdx.x) * th.K * th.C + ck.k0 * th.C + ck.c0) *
+                              cout;
   const int n = n0 + 16 * nb + i16;
 #pragma unroll
   for (int j = 0; j < TPW; ++j)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int r = 16 * (wv / NB + WPB * j) + 4 * g + e;
-      if (r < rc && r0 + r < R && n < cout)
-        slot[static_cast<int64_t>(r0 + r) * cout + n] = acc[j][e];
+      if (r < cols && n < cout)
+        slot[static_cast<int64_t>(r) * cout + n] = acc[j][e];
     }
 }
 
@@ -372,13 +473,20 @@ int piece_bytes(const void *p, int64_t row_bytes) {
   return a % 16 == 0 ? 16 : (a % 4 == 0 ? 4 : 2);
 }
 
-uint32_t piece_div(int ppr) { return ((1u << 20) + ppr - 1) / ppr; }
-
-// columns per LDS chunk: the im2col width in equal parts of at most kRC, in
-// multiples of 32 (whole MFMA steps and whole pieces)
-int chunk_cols(int R) {
-  const int n = static_cast<int>(ceil_div(R, kRC));
-  return static_cast<int>(ceil_div(ceil_div(R, n), 32) * 32);
+// The chunks of K offsets of C channels, in equal shares.
+Thin thin_of(int K, int C, int pieces, int64_t n_rows) {
+  auto inv = [](int d) { return static_cast<uint32_t>(((1 << 20) + d - 1) / d); };
+  Thin t{K, C, pieces, inv(pieces), inv(C), 1, 1, C, 1, ceil_div(n_rows, kSeg)};
+  if (C <= kRC) {
+    t.chunks = static_cast<int>(ceil_div(K, kRC / C));
+    t.kc = static_cast<int>(ceil_div(K, t.chunks));
+    t.chunks = static_cast<int>(ceil_div(K, t.kc));
+  } else {
+    t.cw = static_cast<int>(ceil_div(ceil_div(C, ceil_div(C, kRC)), 32) * 32);
+    t.parts = static_cast<int>(ceil_div(C, t.cw));
+    t.chunks = K * t.parts;
+  }
+  return t;
 }
 
 } // namespace
@@ -392,16 +500,13 @@ void conv_thin(const T *x, int64_t n_x, int C, const T *w, int64_t wk, int64_t w
                const int32_t *wperm, int ncols, const float *bias, const int32_t *nbr,
                int64_t n_rows, int K, const int32_t *order, T *y, hipStream_t s) {
   const int pb = piece_bytes(x, static_cast<int64_t>(C) * sizeof(T));
-  const int ppr = C * static_cast<int>(sizeof(T)) / pb;
-  const int rc = chunk_cols(K * C), chunks = static_cast<int>(ceil_div(K * C, rc));
-  const int64_t tiles = ceil_div(n_rows, kSeg);
+  const Thin th = thin_of(K, C, C * static_cast<int>(sizeof(T)) / pb, n_rows);
   auto go = [&](auto ntc, auto pbc) {
     constexpr int NT = decltype(ntc)::value;
-    const dim3 grid(static_cast<unsigned>(std::min<int64_t>(tiles, 2048)),
+    const dim3 grid(static_cast<unsigned>(std::min<int64_t>(th.blocks, 1024)),
                     static_cast<unsigned>(ceil_div(ncols, NT)));
     hipLaunchKernelGGL((conv_thin_kernel<T, NT, decltype(pbc)::value>), grid, dim3(kThreads), 0,
-                       s, x, n_x, C, w, wk, wc, wn, wperm, ncols, bias, nbr, n_rows, K, order, y,
-                       ppr, piece_div(ppr), rc, chunks);
+                       s, x, n_x, th, w, wk, wc, wn, wperm, ncols, bias, nbr, n_rows, order, y);
   };
   using N16 = std::integral_constant<int, 16>;
   using N32 = std::integral_constant<int, 32>;
@@ -423,7 +528,7 @@ void conv_thin(const T *x, int64_t n_x, int C, const T *w, int64_t wk, int64_t w
 // Ranges of the thin dW kernel: about 1024 workgroups (four per CU), each
 // range at least two segments, at most 512 partial slots.
 int conv_dw_thin_ranges(int K, int C, int cout, int64_t n_rows) {
-  const int64_t units = ceil_div(K * C, chunk_cols(K * C)) * ceil_div(cout, cout <= 32 ? 32 : 64);
+  const int64_t units = thin_of(K, C, 1, 1).chunks * ceil_div(cout, cout <= 32 ? 32 : 64);
   const int64_t segs = ceil_div(std::max<int64_t>(n_rows, 1), kSeg);
   return static_cast<int>(std::max<int64_t>(
       1, std::min<int64_t>({512, 1024 / units, ceil_div(segs, 2)})));
@@ -437,18 +542,18 @@ void conv_dw_thin(const T *x, int64_t n_x, int C, const T *gy, int cout, const i
   int pby = piece_bytes(gy, static_cast<int64_t>(cout) * sizeof(T));
   if (pby == 4 && !kF32<T>)
     pby = 2;
-  const int ppr = C * static_cast<int>(sizeof(T)) / pb, ppy = cout * static_cast<int>(sizeof(T)) / pby;
-  const int rc = chunk_cols(K * C), chunks = static_cast<int>(ceil_div(K * C, rc));
+  const Thin th = thin_of(K, C, C * static_cast<int>(sizeof(T)) / pb, n_rows);
+  const Thin ty = thin_of(1, cout, cout * static_cast<int>(sizeof(T)) / pby, n_rows);
   const int ranges = conv_dw_thin_ranges(K, C, cout, n_rows);
   const int64_t n = static_cast<int64_t>(K) * C * cout;
   if (n_rows > 0) {
     auto go = [&](auto ntc, auto pbc, auto pbyc) {
       constexpr int NT = decltype(ntc)::value;
-      const dim3 grid(static_cast<unsigned>(ranges), static_cast<unsigned>(chunks),
+      const dim3 grid(static_cast<unsigned>(ranges), static_cast<unsigned>(th.chunks),
                       static_cast<unsigned>(ceil_div(cout, NT)));
       hipLaunchKernelGGL((conv_dw_thin_kernel<T, NT, decltype(pbc)::value, decltype(pbyc)::value>),
-                         grid, dim3(kThreads), 0, s, x, n_x, C, gy, cout, nbr, n_rows, K, order,
-                         ppr, piece_div(ppr), rc, ppy, piece_div(ppy), partial);
+                         grid, dim3(kThreads), 0, s, x, n_x, th, gy, ty, nbr, n_rows, order,
+                         partial);
     };
     auto pick_n = [&](auto pbc, auto pbyc) {
       cout <= 16   ? go(std::integral_constant<int, 16>{}, pbc, pbyc)
