@@ -2592,15 +2592,27 @@ __global__ __launch_bounds__(kThreads) void colsum_partial_kernel(const T *__res
   }
 }
 
+// out[c] = sum over the chunks of partial[chunk][c]: a workgroup owns 16
+// columns, thread t the chunks t / 16 (mod 16) of column t % 16, whose sums
+// are added in order. One thread per column walked all 256 chunks in series
+// (a 20-column layer on MI355X: 45 us, here 5).
 __global__ __launch_bounds__(kThreads) void colsum_final_kernel(const float *__restrict__ partial,
                                                                 int chunks, int C,
                                                                 float *__restrict__ out) {
-  const int c = blockIdx.x * kThreads + threadIdx.x;
-  if (c >= C)
-    return;
+  __shared__ float red[kThreads];
+  const int t = threadIdx.x, c = blockIdx.x * 16 + t % 16;
   float v = 0.f;
-  for (int b = 0; b < chunks; ++b)
-    v += partial[static_cast<int64_t>(b) * C + c];
+  if (c < C) {
+#pragma unroll 8
+    for (int b = t / 16; b < chunks; b += kThreads / 16)
+      v += partial[static_cast<int64_t>(b) * C + c];
+  }
+  red[t] = v;
+  __syncthreads();
+  if (t >= 16 || c >= C)
+    return;
+  for (int q = 1; q < kThreads / 16; ++q)
+    v += red[q * 16 + t];
   out[c] = v;
 }
 
@@ -3827,7 +3839,7 @@ extern "C" int rhip_conv_bias_grad(const void *grad_y, int64_t n_out, int32_t co
       hipLaunchKernelGGL((colsum_partial_kernel<__bf16>), dim3(chunks), dim3(kThreads), 0, stream,
                          static_cast<const __bf16 *>(grad_y), n_out, cout, rpc, partial);
     RHIP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(colsum_final_kernel, dim3(static_cast<unsigned>(ceil_div(cout, kThreads))),
+    hipLaunchKernelGGL(colsum_final_kernel, dim3(static_cast<unsigned>(ceil_div(cout, 16))),
                        dim3(kThreads), 0, stream, partial, chunks, cout, grad_bias);
     RHIP_LAUNCH_CHECK();
   });
