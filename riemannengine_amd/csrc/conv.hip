@@ -37,29 +37,12 @@
 #include <type_traits>
 
 #include "conv_thin.hpp"
+#include "conv_x3.hpp"
 
 namespace rhip {
 
 constexpr int kMaskWords = 4; // the MFMA paths handle K <= 128 offsets
 constexpr int kWideRG = 2;    // row groups per wave of conv_os_lds_kernel's bf16 128-column tiles
-
-// Gathered rows in quad order. The L1 serves a vector load four lanes at a
-// time and looks up one cache line per distinct line among them; in the MFMA
-// operand layout (lane (i16, g): row i16, bytes 16g..16g+15 of a 64-byte
-// slice) the four lanes of a quad hold four rows, so every lane costs an
-// access. Loading lane 4m + c with row m's bytes 16c..16c+15 instead makes
-// each quad one 64-byte access (a quarter of the accesses); quad_to_mfma
-// then moves lane 4m + c's 16 bytes to lane 16c + m with four ds_bpermute.
-__device__ __forceinline__ int quad_src(int lane) { return (4 * (lane & 15) + (lane >> 4)) * 4; }
-
-__device__ __forceinline__ v4u quad_to_mfma(const v4u &v, int src) {
-  v4u o;
-#pragma unroll
-  for (int d = 0; d < 4; ++d)
-    o[d] = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(src, static_cast<int32_t>(v[d])));
-  return o;
-}
-
 
 // ------------------------------------------------ output-stationary GEMM
 //
@@ -3582,6 +3565,7 @@ static void run_dw_rows(const __bf16 *x, int64_t n_in, int cin, const __bf16 *gy
 // rhip_conv_forward_workspace_bytes serves the forward and input gradient.
 struct ConvWs {
   void *wt = nullptr;
+  size_t wt_bytes = 0;
   float *os_partial = nullptr;
   float *bias_partial = nullptr;
   float *partial = nullptr;
@@ -3595,11 +3579,18 @@ static ConvWs carve_conv_front(Carve &cv, int32_t K, int32_t cin, int32_t cout, 
   const size_t nw = static_cast<size_t>(K) *
                     std::max(static_cast<size_t>(cout) * red_width(dtype, cin),
                              static_cast<size_t>(cin) * red_width(dtype, cout));
-  w.wt = cv.take<char>(nw * (dtype == RHIP_F32 ? 4 : 2));
+  // (fp32: their three bf16 parts where conv_x3 takes the layer)
+  w.wt_bytes = nw * (dtype == RHIP_F32 ? 4 : 2);
   const bool f32 = dtype == RHIP_F32;
+  if (f32 && (conv_x3_takes(cin, cout, K, n_in) || conv_x3_takes(cout, cin, K, n_out)))
+    w.wt_bytes = std::max(w.wt_bytes, conv_x3_weight_bytes(K, cin, cout));
+  w.wt = cv.take<char>(w.wt_bytes);
   auto osp = [&](int64_t n, int cred, int ncols) {
-    return f32 ? os_partial_floats<float>(n, cred, ncols, K)
-               : os_partial_floats<__bf16>(n, cred, ncols, K);
+    if (!f32)
+      return os_partial_floats<__bf16>(n, cred, ncols, K);
+    const int sp = conv_x3_splits(n, cred, ncols, K);
+    return std::max(os_partial_floats<float>(n, cred, ncols, K),
+                    sp > 1 ? static_cast<size_t>(sp) * n * ncols : size_t(0));
   };
   w.os_partial = cv.take<float>(std::max<size_t>({1, osp(n_out, cin, cout), osp(n_in, cout, cin)}));
   w.bias_partial = cv.take<float>(static_cast<size_t>(kBiasChunks) * cout);
@@ -3619,12 +3610,14 @@ static ConvWs carve_conv(Carve &cv, int32_t K, int32_t cin, int32_t cout, int32_
   return w;
 }
 
-// The forward with the transposed weights at wt (K * cin * cout elements) and
-// the split partial sums at os_partial (null: no split).
+// The forward with the transposed weights at wt (wt_bytes: K * cin * cout
+// elements at least) and the split partial sums at os_partial (null: no
+// split).
 static void conv_forward_into(const void *x, int64_t n_in, int32_t cin, const void *weight,
                               int32_t K, int32_t cout, const float *bias, const int32_t *nbr,
                               const int32_t *out_order, int64_t n_out, void *y, int32_t dtype,
-                              void *wt, float *os_partial, hipStream_t stream) {
+                              void *wt, size_t wt_bytes, float *os_partial,
+                              hipStream_t stream) {
   auto thin = [&](auto *xt) {
     using T = std::remove_const_t<std::remove_pointer_t<decltype(xt)>>;
     if (!os_thin<T>(n_in, cin, cout, K))
@@ -3640,7 +3633,12 @@ static void conv_forward_into(const void *x, int64_t n_in, int32_t cin, const vo
   // the MFMA path reads W[k] column-wise: stage the [K, cout, credw] copy
   const int credw = red_width(dtype, cin);
   const int64_t nw = static_cast<int64_t>(K) * cout * credw;
-  if (dtype == RHIP_F32) {
+  if (dtype == RHIP_F32 && conv_x3_takes(cin, cout, K, n_in) && aligned16(x) &&
+      wt_bytes >= conv_x3_weight_bytes(K, cin, cout)) {
+    conv_x3(static_cast<const float *>(x), n_in, cin, static_cast<const float *>(weight), cout, 1,
+            nullptr, cout, bias, nbr, n_out, K, out_order, static_cast<float *>(y), wt, os_partial,
+            stream);
+  } else if (dtype == RHIP_F32) {
     float *w = static_cast<float *>(wt);
     hipLaunchKernelGGL((transpose_w_kernel<float>), dim3(ceil_div(nw, kThreads)),
                        dim3(kThreads), 0, stream, static_cast<const float *>(weight), K, cin,
@@ -3784,7 +3782,7 @@ extern "C" int rhip_conv_forward(const void *x, int64_t n_in, int32_t cin,
     Carve cv(workspace, workspace_bytes);
     const ConvWs w = carve_conv_front(cv, K, cin, cout, dtype, n_in, n_out);
     conv_forward_into(x, n_in, cin, weight, K, cout, bias, nbr, out_order, n_out, y, dtype, w.wt,
-                      w.os_partial, stream);
+                      w.wt_bytes, w.os_partial, stream);
   });
 }
 
@@ -3812,7 +3810,7 @@ extern "C" int rhip_conv_forward_noalloc(const void *x, int64_t n_in, int32_t ci
     // no split of the offset axis: it would need partial sums beyond the scratch
     with_device_scratch(stream, [&](void *scratch_ptr) {
       conv_forward_into(x, n_in, cin, weight, K, cout, bias, nbr, out_order, n_out, y, dtype,
-                        scratch_ptr, nullptr, stream);
+                        scratch_ptr, kConvScratchBytes, nullptr, stream);
     });
   });
 }
@@ -3886,6 +3884,12 @@ extern "C" int rhip_conv_backward_input(const void *grad_y, int64_t n_out,
       const ConvWs w = carve_conv_front(cv, K, cin, cout, dtype, n_in, n_out);
       os_partial = w.os_partial;
       wperm_buf = w.wt;
+      if (dtype == RHIP_F32 && conv_x3_takes(cout, cin, K, n_out) && aligned16(grad_y)) {
+        conv_x3(static_cast<const float *>(grad_y), n_out, cout,
+                static_cast<const float *>(weight), 1, cout, weight_perm, cin, nullptr, nbr_t,
+                n_in, K, in_order, static_cast<float *>(grad_x), w.wt, os_partial, stream);
+        return;
+      }
       if (red_width(dtype, cout) != cout) { // [K][cin][cout] rows padded to credw
         credw = red_width(dtype, cout);
         const int64_t ne = static_cast<int64_t>(K) * cin * credw;

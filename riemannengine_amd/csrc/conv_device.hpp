@@ -106,6 +106,23 @@ __device__ __forceinline__ uint32_t pick_off(uint32_t off, int32_t keep) {
   return (off & static_cast<uint32_t>(keep)) | (kBufOob & ~static_cast<uint32_t>(keep));
 }
 
+// Gathered rows in quad order. The L1 serves a vector load four lanes at a
+// time and looks up one cache line per distinct line among them; in the MFMA
+// operand layout (lane (i16, g): row i16, bytes 16g..16g+15 of a 64-byte
+// slice) the four lanes of a quad hold four rows, so every lane costs an
+// access. Loading lane 4m + c with row m's bytes 16c..16c+15 instead makes
+// each quad one 64-byte access (a quarter of the accesses); quad_to_mfma
+// then moves lane 4m + c's 16 bytes to lane 16c + m with four ds_bpermute.
+__device__ __forceinline__ int quad_src(int lane) { return (4 * (lane & 15) + (lane >> 4)) * 4; }
+
+__device__ __forceinline__ v4u quad_to_mfma(const v4u &v, int src) {
+  v4u o;
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+    o[d] = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(src, static_cast<int32_t>(v[d])));
+  return o;
+}
+
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 } // namespace rhip
