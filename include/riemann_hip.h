@@ -403,23 +403,24 @@ int rhip_conv_backward_weight_rows_supported(int32_t dtype, int32_t cin, int32_t
 /*
  * The same weight gradient for channel counts that are not both multiples of
  * 16 (a first layer's few input channels, a classifier's outputs), from the
- * dense neighbour table, as one dense product over im2col rows; fp32
- * accumulation, deterministic. At most 1024 offsets times input channels and
- * 1024 output channels, x and grad_y under 2 GiB each; other shapes return
- * RHIP_ERR_UNSUPPORTED, for which rhip_conv_backward_weight is the fallback.
- * Workspace as for rhip_conv_workspace_bytes.
+ * dense neighbour table: short reductions as one dense product over im2col
+ * rows, others on padded copies; fp32 accumulation, deterministic. At most 128
+ * offsets, or 1024 offsets times input channels, x and grad_y under 2 GiB
+ * each; other shapes return RHIP_ERR_UNSUPPORTED, for which
+ * rhip_conv_backward_weight is the fallback. Workspace as for
+ * rhip_conv_workspace_bytes.
  * Replaces the dW half of MmBackward (engine/nn/conv.cpp:62), like
  * rhip_conv_backward_weight.
  */
-int rhip_conv_backward_weight_thin(const void *x, int64_t n_in, int32_t cin,
+int rhip_conv_backward_weight_ragged(const void *x, int64_t n_in, int32_t cin,
                                    const void *grad_y, int64_t n_out,
                                    int32_t cout, int32_t K, const int32_t *nbr,
                                    const int32_t *out_order, void *grad_w,
                                    int32_t dtype, void *workspace,
                                    size_t workspace_bytes, hipStream_t stream);
 
-/* 1 if rhip_conv_backward_weight_thin takes this shape, else 0 (no status). */
-int rhip_conv_backward_weight_thin_supported(int32_t dtype, int32_t cin, int32_t cout,
+/* 1 if rhip_conv_backward_weight_ragged takes this shape, else 0 (no status). */
+int rhip_conv_backward_weight_ragged_supported(int32_t dtype, int32_t cin, int32_t cout,
                                              int32_t K, int64_t n_in, int64_t n_out);
 
 /* --------------------------------------------------------------- pooling */

@@ -34,7 +34,7 @@ EXPORTS = (
     "rhip_stride_coords",
     "rhip_expand_coords", "rhip_kmap_workspace_bytes", "rhip_kmap_count", "rhip_kmap_fill",
     "rhip_kmap_pairs_workspace_bytes", "rhip_kmap_pairs", "rhip_stencil_partners",
-    "rhip_conv_backward_weight_thin", "rhip_conv_backward_weight_thin_supported",
+    "rhip_conv_backward_weight_ragged", "rhip_conv_backward_weight_ragged_supported",
     "rhip_conv_backward_weight_rows_supported",
     "rhip_conv_workspace_bytes", "rhip_conv_forward_workspace_bytes", "rhip_conv_forward",
     "rhip_conv_forward_noalloc", "rhip_conv_bias_grad",
@@ -110,9 +110,9 @@ def _declare(lib):
                                                      _i32, _vp, _sz, _vp]),
         "rhip_conv_backward_weight_rows": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i64, _i32, _i32,
                                                           _vp, _vp, _vp, _i32, _vp, _sz, _vp]),
-        "rhip_conv_backward_weight_thin": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i64, _i32, _i32,
+        "rhip_conv_backward_weight_ragged": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i64, _i32, _i32,
                                                           _vp, _vp, _vp, _i32, _vp, _sz, _vp]),
-        "rhip_conv_backward_weight_thin_supported": (ctypes.c_int, [_i32, _i32, _i32, _i32,
+        "rhip_conv_backward_weight_ragged_supported": (ctypes.c_int, [_i32, _i32, _i32, _i32,
                                                                     _i64, _i64]),
         "rhip_stride_map_workspace_bytes": (ctypes.c_int, [_i64, _i64, _P(_sz)]),
         "rhip_stride_map_count": (ctypes.c_int, [_P(RhipTable), _vp, _i64, _P(_i32), _vp, _sz,
@@ -604,8 +604,8 @@ RHIP_ERR_UNSUPPORTED = 3
 def conv_weight_grad(x: torch.Tensor, grad_y: torch.Tensor, kmap: KernelMap,
                      K: int) -> torch.Tensor:
     """dW as the convolution layer computes it: from the neighbour table where
-    the library has a kernel for the shape (the tiled ones, else the thin
-    one), else from the pair list. bf16
+    the library has a kernel for the shape (the tiled ones, else those
+    for ragged channel counts), else from the pair list. bf16
     maps of at most 8 offsets also take the pair list, which is faster there,
     when they hold fewer than 2 pairs per output row (a transposed stride-2
     map: one neighbour per row) or pair each input row at most once (a
@@ -626,7 +626,7 @@ def conv_weight_grad(x: torch.Tensor, grad_y: torch.Tensor, kmap: KernelMap,
                                                   _ptr(kmap.out_order), _ptr(gw), dt, _ptr(ws),
                                                   ws.numel(), _stream(x.device))
     if st == RHIP_ERR_UNSUPPORTED:
-        st = lib().rhip_conv_backward_weight_thin(_ptr(x), kmap.n_in, cin, _ptr(grad_y),
+        st = lib().rhip_conv_backward_weight_ragged(_ptr(x), kmap.n_in, cin, _ptr(grad_y),
                                                   kmap.n_out, cout, K, _ptr(kmap.nbr),
                                                   _ptr(kmap.out_order), _ptr(gw), dt, _ptr(ws),
                                                   ws.numel(), _stream(x.device))

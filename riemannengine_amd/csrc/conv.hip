@@ -36,6 +36,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "conv_pad.hpp"
 #include "conv_thin.hpp"
 #include "conv_x3.hpp"
 
@@ -2716,12 +2717,32 @@ static bool os_fast(const T *x, int cred, const T *wt, int credw, int ncols, int
   return os_shape<T>(cred, credw, ncols, K) && aligned16(x) && aligned16(wt);
 }
 
-// The thin kernels' part: shapes the tiled kernels do not take, up to
-// kThinMaxCols im2col columns (a 3^3 layer of 37 channels).
-template <typename T>
-static bool os_thin(int64_t n_x, int cred, int ncols, int K) {
-  const int32_t dt = kIsF32<T> ? RHIP_F32 : RHIP_BF16;
-  return !os_shape<T>(cred, red_width(dt, cred), ncols, K) && conv_thin_takes(K, cred, n_x, sizeof(T));
+static bool os_shape_of(int32_t dtype, int cred, int ncols, int K) {
+  return dtype == RHIP_F32 ? os_shape<float>(cred, cred, ncols, K)
+                           : os_shape<__bf16>(cred, red_width(dtype, cred), ncols, K);
+}
+
+// Layers with channel counts that a tiled kernel does not take in some
+// direction: these directions run on the thin kernels, or with padded copies
+// on the tiled ones (conv_pad).
+static bool ragged(int32_t dtype, int cin, int cout, int K) {
+  return !(os_shape_of(dtype, cin, cout, K) && os_shape_of(dtype, cout, cin, K));
+}
+static bool pads(int32_t dtype, int cin, int cout, int K) {
+  return K <= 32 * kMaskWords && ragged(dtype, cin, cout, K);
+}
+
+// Whether the thin kernels run a reduction of C channels over K offsets that
+// the tiled ones do not take; where it can be padded, up to kThinCols im2col
+// columns, kThinChannels channels (a padded row is mostly zeros there) or
+// kThinCols1 columns of one offset (nothing is missing). Measured on MI355X,
+// 200k rows, forward, thin / padded: 5^3 3->32 bf16 123 / 160 us, fp32 155 /
+// 308; 5^3 6->64 280 / 202 and 575 / 507; 3^3 6->64 85 / 63 and 168 / 129;
+// 24->24 192 / 53 and 250 / 88; dW in the same order.
+constexpr int kThinCols = 128, kThinCols1 = 256, kThinChannels = 4;
+static bool thin_runs(int K, int C, int64_t n_x, int elem_bytes, bool can_pad) {
+  return conv_thin_takes(K, C, n_x, elem_bytes) &&
+         (!can_pad || C <= kThinChannels || K * C <= kThinCols || (K == 1 && C <= kThinCols1));
 }
 
 // Splits of the offset axis for the MFMA kernel: a map with few rows and
@@ -3136,14 +3157,6 @@ static int dw_width(int c) { return c % 64 == 0 ? 4 : (c % 32 == 0 ? 2 : 1); }
 // counts (most workgroups idle), 15.5 at 3 waves per SIMD, 15.9-18.7 with
 // rows 2 to 4 steps ahead, and 36.3 for conv_dw_kernel.
 constexpr int kDwPairsD = 1, kDwPairsWaves = 2;
-// dW's: channel counts that neither the table's nor the pair lists' tiled
-// kernels take.
-static bool dw_thin(int32_t dtype, int cin, int cout, int K, int64_t n_in, int64_t n_out) {
-  const int s = dtype == RHIP_F32 ? 4 : 2;
-  return !(cin % 16 == 0 && cout % 16 == 0) && cout <= kThinMaxCols &&
-         conv_thin_takes(K, cin, n_in, s) && n_out * cout * s <= kBufMaxBytes;
-}
-
 static DwPlan dw_plan(int32_t dtype, int cin, int cout, int K, int64_t n_pairs, int64_t n_in,
                       int64_t n_out, int wgs = 0) {
   DwPlan p;
@@ -3492,6 +3505,37 @@ static void run_dw_pos(const float *x, int64_t n_in, int cin, const float *gy, i
   RHIP_LAUNCH_CHECK();
 }
 
+// dW of channel counts that are not both multiples of 16 (which neither the
+// table's nor the pair lists' kernels take): thin, or padded on the table's
+// position kernels; 0 none.
+enum class Ragged { kNone, kThin, kPad };
+static Ragged dw_ragged(int32_t dtype, int cin, int cout, int K, int64_t n_in, int64_t n_out) {
+  const int64_t s = dtype == RHIP_F32 ? 4 : 2;
+  if (cin % 16 == 0 && cout % 16 == 0)
+    return Ragged::kNone;
+  const bool pad = K <= 32 * kMaskWords && n_in * pad_width(cin) * s <= kBufMaxBytes &&
+                   n_out * pad_width(cout) * s <= kBufMaxBytes && K * n_out * 4 <= kBufMaxBytes;
+  if (cout <= kThinMaxCols && n_out * cout * s <= kBufMaxBytes &&
+      thin_runs(K, cin, n_in, static_cast<int>(s), pad))
+    return Ragged::kThin;
+  return pad ? Ragged::kPad : Ragged::kNone;
+}
+static size_t dw_ragged_floats(int32_t dtype, int cin, int cout, int K, int64_t n_in,
+                               int64_t n_out) {
+  switch (dw_ragged(dtype, cin, cout, K, n_in, n_out)) {
+  case Ragged::kThin:
+    return static_cast<size_t>(conv_dw_thin_ranges(K, cin, cout, n_out)) * K * cin * cout;
+  case Ragged::kPad: {
+    const int cp = pad_width(cin), np = pad_width(cout);
+    const int slots = dtype == RHIP_F32 ? dw_pos_f32_ranges(K, cp, np, n_out)
+                                        : dw_pos_bf16_ranges(K, cp, np, n_out);
+    return static_cast<size_t>(slots) * K * cp * np;
+  }
+  default:
+    return 0;
+  }
+}
+
 // Row blocks of conv_dw_rows_kernel for n_out output rows.
 static int dw_rows_blocks(int64_t n_out) {
   return static_cast<int>(std::min<int64_t>(kDwRowsBlocks, ceil_div(n_out, kDwRowsSP)));
@@ -3568,6 +3612,12 @@ struct ConvWs {
   size_t wt_bytes = 0;
   float *os_partial = nullptr;
   float *bias_partial = nullptr;
+  // padded layers: the padded widths, both sides' rows, the weights (or dW)
+  // and the bias, and the flag of a value that is not finite
+  int cp = 0, np = 0;
+  void *px = nullptr, *py = nullptr, *pw = nullptr;
+  float *pbias = nullptr;
+  int *bad = nullptr;
   float *partial = nullptr;
   float *acc = nullptr;
 };
@@ -3575,15 +3625,20 @@ struct ConvWs {
 static ConvWs carve_conv_front(Carve &cv, int32_t K, int32_t cin, int32_t cout, int32_t dtype,
                                int64_t n_in, int64_t n_out) {
   ConvWs w;
-  // transposed forward weights, or the padded copy of dX's
-  const size_t nw = static_cast<size_t>(K) *
-                    std::max(static_cast<size_t>(cout) * red_width(dtype, cin),
-                             static_cast<size_t>(cin) * red_width(dtype, cout));
-  // (fp32: their three bf16 parts where conv_x3 takes the layer)
-  w.wt_bytes = nw * (dtype == RHIP_F32 ? 4 : 2);
   const bool f32 = dtype == RHIP_F32;
-  if (f32 && (conv_x3_takes(cin, cout, K, n_in) || conv_x3_takes(cout, cin, K, n_out)))
-    w.wt_bytes = std::max(w.wt_bytes, conv_x3_weight_bytes(K, cin, cout));
+  const size_t es = f32 ? 4 : 2;
+  // channel counts the tiled kernels see
+  const bool pad = pads(dtype, cin, cout, K);
+  w.cp = pad ? pad_width(cin) : cin;
+  w.np = pad ? pad_width(cout) : cout;
+  // transposed forward weights, or the padded copy of dX's (fp32: their three
+  // bf16 parts where conv_x3 takes the layer)
+  const size_t nw = static_cast<size_t>(K) *
+                    std::max(static_cast<size_t>(w.np) * red_width(dtype, w.cp),
+                             static_cast<size_t>(w.cp) * red_width(dtype, w.np));
+  w.wt_bytes = nw * es;
+  if (f32 && (conv_x3_takes(w.cp, w.np, K, n_in) || conv_x3_takes(w.np, w.cp, K, n_out)))
+    w.wt_bytes = std::max(w.wt_bytes, conv_x3_weight_bytes(K, w.cp, w.np));
   w.wt = cv.take<char>(w.wt_bytes);
   auto osp = [&](int64_t n, int cred, int ncols) {
     if (!f32)
@@ -3592,80 +3647,154 @@ static ConvWs carve_conv_front(Carve &cv, int32_t K, int32_t cin, int32_t cout, 
     return std::max(os_partial_floats<float>(n, cred, ncols, K),
                     sp > 1 ? static_cast<size_t>(sp) * n * ncols : size_t(0));
   };
-  w.os_partial = cv.take<float>(std::max<size_t>({1, osp(n_out, cin, cout), osp(n_in, cout, cin)}));
+  w.os_partial =
+      cv.take<float>(std::max<size_t>({1, osp(n_out, w.cp, w.np), osp(n_in, w.np, w.cp)}));
   w.bias_partial = cv.take<float>(static_cast<size_t>(kBiasChunks) * cout);
+  if (pad) {
+    w.px = cv.take<char>(n_in * w.cp * es);
+    w.py = cv.take<char>(n_out * w.np * es);
+    w.pw = cv.take<char>(static_cast<size_t>(K) * w.cp * w.np * es);
+    w.pbias = cv.take<float>(w.np);
+    w.bad = cv.take<int>(1);
+  }
   return w;
 }
 
 static ConvWs carve_conv(Carve &cv, int32_t K, int32_t cin, int32_t cout, int32_t dtype,
                          int64_t n_in, int64_t n_out, const DwPlan &p) {
   ConvWs w = carve_conv_front(cv, K, cin, cout, dtype, n_in, n_out);
-  const size_t thin = dw_thin(dtype, cin, cout, K, n_in, n_out)
-                          ? static_cast<size_t>(conv_dw_thin_ranges(K, cin, cout, n_out)) * K *
-                                cin * cout
-                          : 0;
-  w.partial = cv.take<float>(std::max<size_t>(
-      {1, p.partial_floats() * K, dw_table_floats(dtype, cin, cout, K, n_in, n_out), thin}));
+  w.partial = cv.take<float>(
+      std::max<size_t>({1, p.partial_floats() * K, dw_table_floats(dtype, cin, cout, K, n_in, n_out),
+                        dw_ragged_floats(dtype, cin, cout, K, n_in, n_out)}));
   w.acc = cv.take<float>(static_cast<size_t>(K) * cin * cout);
   return w;
 }
 
-// The forward with the transposed weights at wt (wt_bytes: K * cin * cout
-// elements at least) and the split partial sums at os_partial (null: no
-// split).
-static void conv_forward_into(const void *x, int64_t n_in, int32_t cin, const void *weight,
-                              int32_t K, int32_t cout, const float *bias, const int32_t *nbr,
-                              const int32_t *out_order, int64_t n_out, void *y, int32_t dtype,
-                              void *wt, size_t wt_bytes, float *os_partial,
+// The forward in workspace w: the transposed weights at w.wt (w.wt_bytes: K *
+// cin * cout elements at least), the split partial sums at w.os_partial (null:
+// no split) and the padded copies (w.px null: none).
+template <typename T>
+static void conv_forward_into(const T *x, int64_t n_in, int32_t cin, const T *weight, int32_t K,
+                              int32_t cout, const float *bias, const int32_t *nbr,
+                              const int32_t *out_order, int64_t n_out, T *y, const ConvWs &w,
                               hipStream_t stream) {
-  auto thin = [&](auto *xt) {
-    using T = std::remove_const_t<std::remove_pointer_t<decltype(xt)>>;
-    if (!os_thin<T>(n_in, cin, cout, K))
-      return false;
-    conv_thin<T>(xt, n_in, cin, static_cast<const T *>(weight), static_cast<int64_t>(cin) * cout,
-                 cout, 1, nullptr, cout, bias, nbr, n_out, K, out_order, static_cast<T *>(y),
-                 stream);
-    return true;
-  };
-  if (dtype == RHIP_F32 ? thin(static_cast<const float *>(x))
-                        : thin(static_cast<const __bf16 *>(x)))
-    return;
+  constexpr int32_t dtype = kIsF32<T> ? RHIP_F32 : RHIP_BF16;
+  const int64_t per = static_cast<int64_t>(cin) * cout;
+  if (!os_shape_of(dtype, cin, cout, K)) {
+    if (thin_runs(K, cin, n_in, sizeof(T), w.px != nullptr)) {
+      conv_thin<T>(x, n_in, cin, weight, per, cout, 1, nullptr, cout, bias, nbr, n_out, K,
+                   out_order, y, stream);
+      return;
+    }
+    if (w.px != nullptr) { // on padded copies
+      T *px = static_cast<T *>(w.px), *pw = static_cast<T *>(w.pw);
+      const bool copy = w.cp != cin || !aligned16(x);
+      pad_features<T>(x, copy ? n_in : 0, cin, w.cp, px, w.bad, nullptr, stream);
+      pad_weights<T>(weight, K, cin, cout, w.cp, w.np, pw, bias, w.pbias, w.bad, stream);
+      T *out = w.np != cout ? static_cast<T *>(w.py) : y;
+      ConvWs inner = w;
+      inner.px = nullptr;
+      conv_forward_into<T>(copy ? px : x, n_in, w.cp, pw, K, w.np, bias ? w.pbias : nullptr, nbr,
+                           out_order, n_out, out, inner, stream);
+      finish_rows<T>(out, w.np, y,
+                     PadSum<T>{x, weight, cin, cout, cout, 1, nullptr, bias, nbr, out_order, n_out,
+                               K},
+                     w.bad, stream);
+      return;
+    }
+  }
+  if constexpr (kIsF32<T>) {
+    if (conv_x3_takes(cin, cout, K, n_in) && aligned16(x) && aligned16(y) &&
+        w.wt_bytes >= conv_x3_weight_bytes(K, cin, cout)) {
+      conv_x3(x, n_in, cin, weight, cout, 1, nullptr, cout, bias, nbr, n_out, K, out_order, y,
+              w.wt, w.os_partial, stream);
+      return;
+    }
+  }
   // the MFMA path reads W[k] column-wise: stage the [K, cout, credw] copy
   const int credw = red_width(dtype, cin);
   const int64_t nw = static_cast<int64_t>(K) * cout * credw;
-  if (dtype == RHIP_F32 && conv_x3_takes(cin, cout, K, n_in) && aligned16(x) &&
-      wt_bytes >= conv_x3_weight_bytes(K, cin, cout)) {
-    conv_x3(static_cast<const float *>(x), n_in, cin, static_cast<const float *>(weight), cout, 1,
-            nullptr, cout, bias, nbr, n_out, K, out_order, static_cast<float *>(y), wt, os_partial,
-            stream);
-  } else if (dtype == RHIP_F32) {
-    float *w = static_cast<float *>(wt);
-    hipLaunchKernelGGL((transpose_w_kernel<float>), dim3(ceil_div(nw, kThreads)),
-                       dim3(kThreads), 0, stream, static_cast<const float *>(weight), K, cin,
-                       cout, credw, w);
-    RHIP_LAUNCH_CHECK();
-    run_os<float>(static_cast<const float *>(x), n_in, cin, w, credw, cout, bias, nbr, n_out, K,
-                  out_order, static_cast<float *>(y), os_partial, stream);
-  } else {
+  if constexpr (!kIsF32<T>) {
     // the LDS-indexed kernel reads W itself where it takes the shape
     // (unpadded reductions, unsplit 128-column tiles): no transposed copy
     if (n_out > 0 && credw == cin) {
-      const int splits = os_partial ? os_splits<__bf16>(n_out, cin, cout, K) : 1;
-      if (run_os_lds(static_cast<const __bf16 *>(x), n_in, cin,
-                     static_cast<const __bf16 *>(weight), nullptr, cin, cout, bias, nbr, n_out, K,
-                     out_order, static_cast<__bf16 *>(y), splits, os_partial, stream, true)) {
+      const int splits = w.os_partial ? os_splits<T>(n_out, cin, cout, K) : 1;
+      if (run_os_lds(x, n_in, cin, weight, nullptr, cin, cout, bias, nbr, n_out, K, out_order, y,
+                     splits, w.os_partial, stream, true)) {
         RHIP_LAUNCH_CHECK();
         return;
       }
     }
-    __bf16 *w = static_cast<__bf16 *>(wt);
-    hipLaunchKernelGGL((transpose_w_kernel<__bf16>), dim3(ceil_div(nw, kThreads)),
-                       dim3(kThreads), 0, stream, static_cast<const __bf16 *>(weight), K, cin,
-                       cout, credw, w);
-    RHIP_LAUNCH_CHECK();
-    run_os<__bf16>(static_cast<const __bf16 *>(x), n_in, cin, w, credw, cout, bias, nbr, n_out,
-                   K, out_order, static_cast<__bf16 *>(y), os_partial, stream);
   }
+  T *wt = static_cast<T *>(w.wt);
+  hipLaunchKernelGGL((transpose_w_kernel<T>), dim3(ceil_div(nw, kThreads)), dim3(kThreads), 0,
+                     stream, weight, K, cin, cout, credw, wt);
+  RHIP_LAUNCH_CHECK();
+  run_os<T>(x, n_in, cin, wt, credw, cout, bias, nbr, n_out, K, out_order, y, w.os_partial,
+            stream);
+}
+
+// The input gradient in workspace w (null: none, and then no split of the
+// offset axis, no padding, no fp32 parts and no weight permutation outside
+// the LDS-indexed kernel).
+template <typename T>
+static void conv_backward_input_into(const T *grad_y, int64_t n_out, int32_t cout,
+                                     const T *weight, int32_t K, int32_t cin,
+                                     const int32_t *nbr_t, const int32_t *weight_perm,
+                                     const int32_t *in_order, int64_t n_in, T *grad_x,
+                                     const ConvWs *w, hipStream_t stream) {
+  constexpr int32_t dtype = kIsF32<T> ? RHIP_F32 : RHIP_BF16;
+  const int64_t per = static_cast<int64_t>(cin) * cout;
+  if (w != nullptr && !os_shape_of(dtype, cout, cin, K)) {
+    if (thin_runs(K, cout, n_out, sizeof(T), w->px != nullptr)) {
+      conv_thin<T>(grad_y, n_out, cout, weight, per, 1, cout, weight_perm, cin, nullptr, nbr_t,
+                   n_in, K, in_order, grad_x, stream);
+      return;
+    }
+    if (w->px != nullptr) { // on padded copies
+      T *py = static_cast<T *>(w->py), *pw = static_cast<T *>(w->pw);
+      const bool copy = w->np != cout || !aligned16(grad_y);
+      pad_features<T>(grad_y, copy ? n_out : 0, cout, w->np, py, w->bad, nullptr, stream);
+      pad_weights<T>(weight, K, cin, cout, w->cp, w->np, pw, nullptr, nullptr, w->bad, stream);
+      T *out = w->cp != cin ? static_cast<T *>(w->px) : grad_x;
+      ConvWs inner = *w;
+      inner.px = nullptr;
+      conv_backward_input_into<T>(copy ? py : grad_y, n_out, w->np, pw, K, w->cp, nbr_t,
+                                  weight_perm, in_order, n_in, out, &inner, stream);
+      finish_rows<T>(out, w->cp, grad_x,
+                     PadSum<T>{grad_y, weight, cout, cin, 1, cout, weight_perm, nullptr, nbr_t,
+                               in_order, n_in, K},
+                     w->bad, stream);
+      return;
+    }
+  }
+  const T *wk = weight;
+  const int32_t *wperm = weight_perm;
+  int credw = cout;
+  if (w != nullptr) {
+    if constexpr (kIsF32<T>) {
+      if (conv_x3_takes(cout, cin, K, n_out) && aligned16(grad_y) && aligned16(grad_x) &&
+          w->wt_bytes >= conv_x3_weight_bytes(K, cin, cout)) {
+        conv_x3(grad_y, n_out, cout, weight, 1, cout, weight_perm, cin, nullptr, nbr_t, n_in, K,
+                in_order, grad_x, w->wt, w->os_partial, stream);
+        return;
+      }
+    }
+    if (red_width(dtype, cout) != cout) { // [K][cin][cout] rows padded to credw
+      credw = red_width(dtype, cout);
+      const int64_t ne = static_cast<int64_t>(K) * cin * credw;
+      hipLaunchKernelGGL((pad_rows_kernel<T>), dim3(ceil_div(ne, kThreads)), dim3(kThreads), 0,
+                         stream, weight, static_cast<int64_t>(K) * cin, cout, credw, wperm,
+                         static_cast<int64_t>(cin), static_cast<T *>(w->wt));
+      RHIP_LAUNCH_CHECK();
+      wk = static_cast<const T *>(w->wt);
+      wperm = nullptr; // applied by the padding copy
+    }
+  }
+  // dX rows gather dY rows; W[k] [cin][cout] is already [n = cin][c = cout].
+  run_os<T>(grad_y, n_out, cout, wk, credw, cin, nullptr, nbr_t, n_in, K, in_order, grad_x,
+            w ? w->os_partial : nullptr, stream, true, wperm,
+            w ? static_cast<T *>(w->wt) : nullptr);
 }
 
 // Device scratch of rhip_conv_forward_noalloc: the transposed weights go
@@ -3781,8 +3910,14 @@ extern "C" int rhip_conv_forward(const void *x, int64_t n_in, int32_t cin,
     // plan does not change the forward's pieces
     Carve cv(workspace, workspace_bytes);
     const ConvWs w = carve_conv_front(cv, K, cin, cout, dtype, n_in, n_out);
-    conv_forward_into(x, n_in, cin, weight, K, cout, bias, nbr, out_order, n_out, y, dtype, w.wt,
-                      w.wt_bytes, w.os_partial, stream);
+    if (dtype == RHIP_F32)
+      conv_forward_into<float>(static_cast<const float *>(x), n_in, cin,
+                               static_cast<const float *>(weight), K, cout, bias, nbr, out_order,
+                               n_out, static_cast<float *>(y), w, stream);
+    else
+      conv_forward_into<__bf16>(static_cast<const __bf16 *>(x), n_in, cin,
+                                static_cast<const __bf16 *>(weight), K, cout, bias, nbr, out_order,
+                                n_out, static_cast<__bf16 *>(y), w, stream);
   });
 }
 
@@ -3809,8 +3944,17 @@ extern "C" int rhip_conv_forward_noalloc(const void *x, int64_t n_in, int32_t ci
     RHIP_CHECK_ARG(n_in == 0 || x != nullptr, "x is null");
     // no split of the offset axis: it would need partial sums beyond the scratch
     with_device_scratch(stream, [&](void *scratch_ptr) {
-      conv_forward_into(x, n_in, cin, weight, K, cout, bias, nbr, out_order, n_out, y, dtype,
-                        scratch_ptr, kConvScratchBytes, nullptr, stream);
+      ConvWs w;
+      w.wt = scratch_ptr;
+      w.wt_bytes = kConvScratchBytes;
+      if (dtype == RHIP_F32)
+        conv_forward_into<float>(static_cast<const float *>(x), n_in, cin,
+                                 static_cast<const float *>(weight), K, cout, bias, nbr, out_order,
+                                 n_out, static_cast<float *>(y), w, stream);
+      else
+        conv_forward_into<__bf16>(static_cast<const __bf16 *>(x), n_in, cin,
+                                  static_cast<const __bf16 *>(weight), K, cout, bias, nbr,
+                                  out_order, n_out, static_cast<__bf16 *>(y), w, stream);
     });
   });
 }
@@ -3860,59 +4004,22 @@ extern "C" int rhip_conv_backward_input(const void *grad_y, int64_t n_out,
       return;
     RHIP_CHECK_ARG(grad_x && weight && nbr_t, "grad_x, weight and nbr_t are required");
     RHIP_CHECK_ARG(n_out == 0 || grad_y != nullptr, "grad_y is null");
-    auto thin = [&](auto *gy) {
-      using T = std::remove_const_t<std::remove_pointer_t<decltype(gy)>>;
-      if (workspace == nullptr || !os_thin<T>(n_out, cout, cin, K))
-        return false;
-      conv_thin<T>(gy, n_out, cout, static_cast<const T *>(weight),
-                   static_cast<int64_t>(cin) * cout, 1, cout, weight_perm, cin, nullptr, nbr_t,
-                   n_in, K, in_order, static_cast<T *>(grad_x), stream);
-      return true;
-    };
-    if (dtype == RHIP_F32 ? thin(static_cast<const float *>(grad_y))
-                          : thin(static_cast<const __bf16 *>(grad_y)))
-      return;
-    // without a workspace the offset axis is not split, and a reduction the
-    // MFMA kernels would pad goes to the one-lane-per-output kernel
-    float *os_partial = nullptr;
-    const void *wk = weight;
-    const int32_t *wperm = weight_perm;
-    void *wperm_buf = nullptr;
-    int credw = cout;
+    ConvWs w;
     if (workspace != nullptr) {
       Carve cv(workspace, workspace_bytes);
-      const ConvWs w = carve_conv_front(cv, K, cin, cout, dtype, n_in, n_out);
-      os_partial = w.os_partial;
-      wperm_buf = w.wt;
-      if (dtype == RHIP_F32 && conv_x3_takes(cout, cin, K, n_out) && aligned16(grad_y)) {
-        conv_x3(static_cast<const float *>(grad_y), n_out, cout,
-                static_cast<const float *>(weight), 1, cout, weight_perm, cin, nullptr, nbr_t,
-                n_in, K, in_order, static_cast<float *>(grad_x), w.wt, os_partial, stream);
-        return;
-      }
-      if (red_width(dtype, cout) != cout) { // [K][cin][cout] rows padded to credw
-        credw = red_width(dtype, cout);
-        const int64_t ne = static_cast<int64_t>(K) * cin * credw;
-        hipLaunchKernelGGL((pad_rows_kernel<__bf16>), dim3(ceil_div(ne, kThreads)),
-                           dim3(kThreads), 0, stream, static_cast<const __bf16 *>(weight),
-                           static_cast<int64_t>(K) * cin, cout, credw, wperm,
-                           static_cast<int64_t>(cin), static_cast<__bf16 *>(w.wt));
-        RHIP_LAUNCH_CHECK();
-        wk = w.wt;
-        wperm = nullptr; // applied by the padding copy
-      }
+      w = carve_conv_front(cv, K, cin, cout, dtype, n_in, n_out);
     }
-    // dX rows gather dY rows; W[k] [cin][cout] is already [n = cin][c = cout].
+    const ConvWs *pw = workspace != nullptr ? &w : nullptr;
     if (dtype == RHIP_F32)
-      run_os<float>(static_cast<const float *>(grad_y), n_out, cout,
-                    static_cast<const float *>(wk), credw, cin, nullptr, nbr_t, n_in, K,
-                    in_order, static_cast<float *>(grad_x), os_partial, stream, true, wperm,
-                    static_cast<float *>(wperm_buf));
+      conv_backward_input_into<float>(static_cast<const float *>(grad_y), n_out, cout,
+                                      static_cast<const float *>(weight), K, cin, nbr_t,
+                                      weight_perm, in_order, n_in, static_cast<float *>(grad_x),
+                                      pw, stream);
     else
-      run_os<__bf16>(static_cast<const __bf16 *>(grad_y), n_out, cout,
-                     static_cast<const __bf16 *>(wk), credw, cin, nullptr, nbr_t, n_in, K,
-                     in_order, static_cast<__bf16 *>(grad_x), os_partial, stream, true, wperm,
-                     static_cast<__bf16 *>(wperm_buf));
+      conv_backward_input_into<__bf16>(static_cast<const __bf16 *>(grad_y), n_out, cout,
+                                       static_cast<const __bf16 *>(weight), K, cin, nbr_t,
+                                       weight_perm, in_order, n_in,
+                                       static_cast<__bf16 *>(grad_x), pw, stream);
   });
 }
 
@@ -3990,7 +4097,22 @@ extern "C" int rhip_conv_backward_weight_rows_supported(int32_t dtype, int32_t c
   return dw_rows_supported(dtype, cin, cout, K, n_in, n_out) ? 1 : 0;
 }
 
-extern "C" int rhip_conv_backward_weight_thin(
+// dW of the padded layer on the position kernels, cropped.
+template <typename T>
+static void conv_dw_padded(const T *x, int64_t n_in, int cin, const T *gy, int64_t n_out, int cout,
+                           int K, const int32_t *nbr, const int32_t *out_order, T *dw,
+                           const ConvWs &w, hipStream_t s) {
+  T *px = static_cast<T *>(w.px), *py = static_cast<T *>(w.py), *pdw = static_cast<T *>(w.pw);
+  pad_features<T>(x, n_in, cin, w.cp, px, w.bad, nullptr, s);
+  pad_features<T>(gy, n_out, cout, w.np, py, nullptr, w.bad, s);
+  if constexpr (kIsF32<T>)
+    run_dw_pos(px, n_in, w.cp, py, n_out, w.np, K, nbr, out_order, w.partial, pdw, s);
+  else
+    run_dw_pos_bf16(px, n_in, w.cp, py, n_out, w.np, K, nbr, out_order, w.partial, pdw, s);
+  finish_weights<T>(pdw, w.cp, w.np, x, cin, gy, cout, nbr, out_order, n_out, K, dw, w.bad, s);
+}
+
+extern "C" int rhip_conv_backward_weight_ragged(
     const void *x, int64_t n_in, int32_t cin, const void *grad_y, int64_t n_out, int32_t cout,
     int32_t K, const int32_t *nbr, const int32_t *out_order, void *grad_w, int32_t dtype,
     void *workspace, size_t workspace_bytes, hipStream_t stream) {
@@ -3998,32 +4120,34 @@ extern "C" int rhip_conv_backward_weight_thin(
     check_dtype(dtype);
     RHIP_CHECK_ARG(K >= 1 && cin >= 1 && cout >= 1, "sizes must be positive");
     RHIP_CHECK_ARG(n_in >= 0 && n_out >= 0, "bad sizes");
-    if (!dw_thin(dtype, cin, cout, K, n_in, n_out))
+    const Ragged how = dw_ragged(dtype, cin, cout, K, n_in, n_out);
+    if (how == Ragged::kNone)
       throw Error(RHIP_ERR_UNSUPPORTED,
-                  "rhip_conv_backward_weight_thin: channel counts that are not both multiples of "
-                  "16, offsets times input channels of at most " + std::to_string(kThinMaxCols) +
-                  " (use rhip_conv_backward_weight)");
+                  "rhip_conv_backward_weight_ragged: channel counts that are not both multiples "
+                  "of 16, at most 128 offsets (use rhip_conv_backward_weight)");
     RHIP_CHECK_ARG(grad_w != nullptr, "grad_w is null");
     RHIP_CHECK_ARG(n_out == 0 || (grad_y && nbr), "grad_y and nbr are required");
     RHIP_CHECK_ARG(n_in == 0 || n_out == 0 || x, "x is null");
     RHIP_CHECK_ARG(workspace != nullptr, "workspace is null");
     Carve cv(workspace, workspace_bytes);
     const ConvWs w = carve_conv(cv, K, cin, cout, dtype, n_in, n_out, DwPlan{});
-    if (dtype == RHIP_F32)
-      conv_dw_thin<float>(static_cast<const float *>(x), n_in, cin,
-                          static_cast<const float *>(grad_y), cout, nbr, n_out, K, out_order,
-                          w.partial, static_cast<float *>(grad_w), stream);
-    else
-      conv_dw_thin<__bf16>(static_cast<const __bf16 *>(x), n_in, cin,
-                           static_cast<const __bf16 *>(grad_y), cout, nbr, n_out, K, out_order,
-                           w.partial, static_cast<__bf16 *>(grad_w), stream);
+    auto run = [&](auto *dw) {
+      using T = std::remove_pointer_t<decltype(dw)>;
+      const T *xt = static_cast<const T *>(x), *gt = static_cast<const T *>(grad_y);
+      if (how == Ragged::kThin)
+        conv_dw_thin<T>(xt, n_in, cin, gt, cout, nbr, n_out, K, out_order, w.partial, dw, stream);
+      else
+        conv_dw_padded<T>(xt, n_in, cin, gt, n_out, cout, K, nbr, out_order, dw, w, stream);
+    };
+    dtype == RHIP_F32 ? run(static_cast<float *>(grad_w)) : run(static_cast<__bf16 *>(grad_w));
   });
 }
 
-extern "C" int rhip_conv_backward_weight_thin_supported(int32_t dtype, int32_t cin, int32_t cout,
-                                                        int32_t K, int64_t n_in, int64_t n_out) {
+extern "C" int rhip_conv_backward_weight_ragged_supported(int32_t dtype, int32_t cin,
+                                                          int32_t cout, int32_t K, int64_t n_in,
+                                                          int64_t n_out) {
   if ((dtype != RHIP_F32 && dtype != RHIP_BF16) || K < 1 || cin < 1 || cout < 1 || n_in < 0 ||
       n_out < 0)
     return 0;
-  return dw_thin(dtype, cin, cout, K, n_in, n_out) ? 1 : 0;
+  return dw_ragged(dtype, cin, cout, K, n_in, n_out) != Ragged::kNone ? 1 : 0;
 }

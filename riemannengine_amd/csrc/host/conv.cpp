@@ -43,8 +43,8 @@ using torch::autograd::AutogradContext;
 using torch::autograd::tensor_list;
 
 // Sources of the weight gradient: the pair lists (in_rows, out_rows), or the
-// neighbour table through the tiled or the thin kernels.
-enum DwSource : int64_t { kDwPairs, kDwRows, kDwThin };
+// neighbour table through the tiled kernels or those for ragged channel counts.
+enum DwSource : int64_t { kDwPairs, kDwRows, kDwRagged };
 
 // Inputs after (features, kernel, bias) are the kernel map's index tensors;
 // they are integer tensors, so autograd gives them no gradient. bias is fp32
@@ -133,7 +133,7 @@ struct HipConvolutionFunction : public torch::autograd::Function<HipConvolutionF
       gw = torch::empty_like(w);
       int rc;
       if (dw != kDwPairs) {
-        rc = (dw == kDwRows ? rhip_conv_backward_weight_rows : rhip_conv_backward_weight_thin)(
+        rc = (dw == kDwRows ? rhip_conv_backward_weight_rows : rhip_conv_backward_weight_ragged)(
             x.data_ptr(), n_in, static_cast<int32_t>(cin), gy.data_ptr(), n_out,
             static_cast<int32_t>(cout), K, nbr.data_ptr<int32_t>(),
             out_order.numel() > 0 ? out_order.data_ptr<int32_t>() : nullptr, gw.data_ptr(), dt,
@@ -146,7 +146,7 @@ struct HipConvolutionFunction : public torch::autograd::Function<HipConvolutionF
                                        in_rows.data_ptr<int32_t>(), out_rows.data_ptr<int32_t>(),
                                        gw.data_ptr(), dt, ws.data_ptr(), ws.numel(), st);
       }
-      check_rhip(rc, "rhip_conv_backward_weight(_rows, _thin)");
+      check_rhip(rc, "rhip_conv_backward_weight(_rows, _ragged)");
     }
     return {gx, gw, gb, {}, {}, {}, {}, {}, {}, {}, {}, {}, {}, {}};
   }
@@ -164,7 +164,7 @@ at::Tensor hip_sparse_convolution(const at::Tensor &features, const at::Tensor &
       bias.defined() ? bias
                      : torch::empty({0}, features.options().dtype(torch::kFloat));
   // dW from the neighbour table where the library has a kernel for the
-  // shape (tiled, or thin for odd channel counts), else from the pair lists (built now, once per map, when a weight
+  // shape (tiled, or ragged channel counts), else from the pair lists (built now, once per map, when a weight
   // gradient may follow). bf16 maps of at most 8 offsets take the pair lists
   // when they hold fewer than 2 pairs per output row (a transposed stride-2
   // map), or pair each input row at most once (a stride-2 map) with channel
@@ -182,8 +182,8 @@ at::Tensor hip_sparse_convolution(const at::Tensor &features, const at::Tensor &
       !sparse_small &&
               rhip_conv_backward_weight_rows_supported(dt, cin, cout, map.K, map.n_in, map.n_out)
           ? kDwRows
-      : rhip_conv_backward_weight_thin_supported(dt, cin, cout, map.K, map.n_in, map.n_out)
-          ? kDwThin
+      : rhip_conv_backward_weight_ragged_supported(dt, cin, cout, map.K, map.n_in, map.n_out)
+          ? kDwRagged
           : kDwPairs;
   const auto iempty = torch::empty({0}, map.nbr.options());
   at::Tensor in_rows = iempty, out_rows = iempty;

@@ -1,9 +1,9 @@
-"""Layers on the thin kernels (im2col rows on MFMA: channel counts that are
-not multiples of 16) against the oracle: forward with bias, input gradient
-and weight gradient at the edges of their tiles (64 positions, 96 im2col
-columns, 16 / 32 / 64 output columns; rows of 2-, 4- and 16-byte pieces) and
-with weights or gradients that are not finite. Tolerance: norm-wise rel 1e-4
-for fp32 and 2e-2 for bf16 (helpers.TOL)."""
+"""Layers whose channel counts are not multiples of 16 against the oracle:
+forward with bias, input gradient and weight gradient at the edges of the
+thin kernels' tiles (64 positions, 96 im2col columns, 16 / 32 / 64 output
+columns; rows of 2-, 4- and 16-byte pieces) and of the padded widths (32, 64,
+128, 192, 256), and with weights or gradients that are not finite. Tolerance:
+norm-wise rel 1e-4 for fp32 and 2e-2 for bf16 (helpers.TOL)."""
 import numpy as np
 import pytest
 import torch
@@ -13,11 +13,12 @@ from riemannengine_amd import abi
 from helpers import DEV, TOL, assert_rel, gpu_tables_and_map, random_coords, to_dev
 
 
-def test_thin_weight_gradient_query_without_a_gpu():
-    q = abi.lib().rhip_conv_backward_weight_thin_supported
+def test_ragged_weight_gradient_query_without_a_gpu():
+    q = abi.lib().rhip_conv_backward_weight_ragged_supported
     assert q(abi.F32, 3, 32, 27, 1000, 1000) == 1 and q(abi.BF16, 64, 20, 1, 1000, 1000) == 1
     assert q(abi.BF16, 64, 48, 27, 1000, 1000) == 0  # the tiled kernels' shapes
-    assert q(abi.F32, 40, 8, 27, 1000, 1000) == 0    # more than 1024 im2col columns
+    assert q(abi.F32, 40, 8, 27, 1000, 1000) == 1    # padded
+    assert q(abi.F32, 40, 8, 129, 1000, 1000) == 0   # neither thin nor at most 128 offsets
     assert q(7, 3, 32, 27, 1000, 1000) == 0 and q(abi.F32, 3, 32, 27, -1, 1000) == 0
 
 
@@ -35,15 +36,15 @@ def _reference(km, x, w, gy):
     return (y, *oracle.conv_backward(x, gy, w, kofs, ir, orr))
 
 
-def _thin_dw(x, gy, km):
-    """rhip_conv_backward_weight_thin itself (no fallback)."""
+def _ragged_dw(x, gy, km):
+    """rhip_conv_backward_weight_ragged itself (no fallback)."""
     dt = abi._dtype_code(x.dtype)
     gw = torch.empty((km.K, x.shape[1], gy.shape[1]), dtype=x.dtype, device=DEV)
     ws = abi._conv_ws(km.K, x.shape[1], gy.shape[1], dt, DEV, km)
-    abi._check(abi.lib().rhip_conv_backward_weight_thin(
+    abi._check(abi.lib().rhip_conv_backward_weight_ragged(
         abi._ptr(x), km.n_in, x.shape[1], abi._ptr(gy), km.n_out, gy.shape[1], km.K,
         abi._ptr(km.nbr), abi._ptr(km.out_order), abi._ptr(gw), dt, abi._ptr(ws), ws.numel(),
-        abi._stream(DEV)), "rhip_conv_backward_weight_thin")
+        abi._stream(DEV)), "rhip_conv_backward_weight_ragged")
     return gw
 
 
@@ -52,52 +53,56 @@ def _thin_dw(x, gy, km):
 @pytest.mark.parametrize("n,ks,cin,cout", [
     (1, 3, 3, 32), (63, 3, 1, 16), (64, 3, 2, 33), (65, 3, 3, 64), (700, 3, 3, 32),
     (700, 3, 4, 80), (129, 3, 6, 13), (300, 5, 1, 20), (300, 5, 6, 40), (257, 1, 64, 20),
-    (1000, 1, 256, 10), (500, 1, 13, 21), (200, 2, 12, 100), (130, 3, 24, 24), (90, 3, 37, 5)])
-def test_thin_layers_match_oracle(n, ks, cin, cout, dtype):
+    (1000, 1, 256, 10), (500, 1, 13, 21), (200, 2, 12, 100), (130, 3, 24, 24), (90, 3, 37, 5),
+    (400, 3, 64, 20), (400, 3, 20, 64), (257, 3, 33, 65), (129, 2, 40, 129), (300, 3, 200, 72),
+    (200, 5, 24, 40), (150, 3, 300, 8), (3000, 3, 40, 40)])
+def test_ragged_layers_match_oracle(n, ks, cin, cout, dtype):
     km = _map(n, ks, seed=n + ks)
     rng = np.random.default_rng(cin * 31 + cout)
     x, gy = rng.standard_normal((n, cin)), rng.standard_normal((n, cout))
     w = rng.standard_normal((km.K, cin, cout)) / np.sqrt(cin * km.K)
     b = rng.standard_normal(cout).astype(np.float32)
     xt, wt, gyt = (to_dev(a.astype(np.float32), dtype) for a in (x, w, gy))
-    print(f"thin n={n} ks={ks} {cin}->{cout} {dtype}", flush=True)
+    print(f"ragged n={n} ks={ks} {cin}->{cout} {dtype}", flush=True)
     y = abi.conv_forward(xt, wt, km, bias=to_dev(b))
     gx = abi.conv_backward_input(gyt, wt, km)
     ry, rgx, rgw = _reference(km, *(t.float().cpu().numpy() for t in (xt, wt, gyt)))
     assert_rel(y.float().cpu().numpy(), ry + b, TOL[dtype], "Y")
     assert_rel(gx.float().cpu().numpy(), rgx, TOL[dtype], "dX")
-    if not (cin % 16 == 0 and cout % 16 == 0) and km.K * cin <= 1024:
-        gw = _thin_dw(xt, gyt, km)
+    if not (cin % 16 == 0 and cout % 16 == 0):
+        gw = _ragged_dw(xt, gyt, km)
         assert_rel(gw.float().cpu().numpy(), rgw, TOL[dtype], "dW")
-        assert torch.equal(gw, _thin_dw(xt, gyt, km))
+        assert torch.equal(gw, _ragged_dw(xt, gyt, km))
         assert torch.equal(gw, abi.conv_weight_grad(xt, gyt, km, km.K))
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("offset", [1, 3])
-def test_thin_layers_on_views_off_the_piece_alignment(dtype, offset):
+@pytest.mark.parametrize("c", [4, 24])
+def test_ragged_layers_on_views_off_the_piece_alignment(dtype, offset, c):
     """Feature rows that start off 4 or 16 bytes (a contiguous view into a
-    longer buffer) go in smaller pieces."""
+    longer buffer) go in smaller pieces or are copied."""
     km = _map(200, 3, seed=9)
     rng = np.random.default_rng(5)
-    flat = to_dev(rng.standard_normal(200 * 12 + offset).astype(np.float32), dtype)
-    x = flat[offset:].view(200, 12)
-    w = to_dev(rng.standard_normal((27, 12, 12)).astype(np.float32) / 18, dtype)
-    y, gw = abi.conv_forward(x, w, km), _thin_dw(x, x, km)
+    flat = to_dev(rng.standard_normal(200 * c + offset).astype(np.float32), dtype)
+    x = flat[offset:].view(200, c)
+    w = to_dev(rng.standard_normal((27, c, c)).astype(np.float32) / 18, dtype)
+    y, gw = abi.conv_forward(x, w, km), _ragged_dw(x, x, km)
     xc = x.clone()
     assert torch.equal(y, abi.conv_forward(xc, w, km))
-    assert torch.equal(gw, _thin_dw(xc, xc, km))
+    assert torch.equal(gw, _ragged_dw(xc, xc, km))
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("bad", [np.inf, np.nan])
-def test_thin_layers_keep_non_finite_values_to_their_pairs(dtype, bad):
+@pytest.mark.parametrize("cin,cout", [(3, 20), (24, 20), (64, 40)])
+def test_ragged_layers_keep_non_finite_values_to_their_pairs(cin, cout, dtype, bad):
     """A weight or gradient that is not finite reaches the outputs its pairs
     reach and no others, as in the pair sums (a missing neighbour is no 0 *
     inf), and a feature row's only the rows that gather it."""
-    n, cin, cout = 400, 3, 20
+    n = 400
     km = _map(n, 3, seed=4, span=5)
     rng = np.random.default_rng(8)
     x, gy = (rng.standard_normal((n, c)).astype(np.float32) for c in (cin, cout))
@@ -107,7 +112,7 @@ def test_thin_layers_keep_non_finite_values_to_their_pairs(dtype, bad):
     for xs, ws, gs in ((x, wb, gb), (xb, w, gy)):
         xt, wt, gt = (to_dev(a, dtype) for a in (xs, ws, gs))
         got = (abi.conv_forward(xt, wt, km), abi.conv_backward_input(gt, wt, km),
-               _thin_dw(xt, gt, km))
+               _ragged_dw(xt, gt, km))
         with np.errstate(invalid="ignore"):
             ref = _reference(km, xs, ws, gs)
         for name, a, r in zip(("Y", "dX", "dW"), got, ref):
