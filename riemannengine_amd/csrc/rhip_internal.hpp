@@ -256,17 +256,18 @@ struct StrideArg {
 // round-robin (id b runs on XCD b % 8); this mapping hands each XCD runs of
 // consecutive tiles, so tiles that share neighbour rows share an L2, while
 // the runs stay interleaved over the whole map to keep the XCDs balanced:
-// at least eight runs per XCD, of at most 2^kXcdRunLog tiles. (With 16-tile
+// at least two runs per XCD, of at most 2^kXcdRunLog tiles. (With 16-tile
 // runs throughout, a map of 17 tiles ran on two XCDs and left six idle: the
 // 256-channel fp32 forward on 2,057 rows 285 us, dealt evenly 126; bf16 89
-// and 44.) The grid is padded to a multiple of 8 runs (padding ids map past
+// and 44; with four or eight runs per XCD, bf16 96->96 on 101k rows 142 / 141
+// us against 139-142, 64->64 on 48k rows 35.4 / 34.9 against 34.1.) The grid is padded to a multiple of 8 runs (padding ids map past
 // the last tile). The run follows from the padded grid, which the padding
 // lifts to the next run's threshold only where it is a multiple of that run
 // too.
 constexpr int kXcds = 8;
 constexpr int kXcdRunLog = 4;
 __host__ __device__ __forceinline__ int xcd_run_log(uint32_t tiles) {
-  const uint32_t runs = tiles / (8 * kXcds);
+  const uint32_t runs = tiles / (2 * kXcds);
   return runs < 1 ? 0 : (runs >> kXcdRunLog ? kXcdRunLog : 31 - __builtin_clz(runs));
 }
 __device__ __forceinline__ int64_t xcd_tile(uint32_t b) {
