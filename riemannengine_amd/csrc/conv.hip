@@ -2315,7 +2315,10 @@ conv_dw_pos_bf16_kernel(const __bf16 *__restrict__ x, int64_t n_in, int cin,
 // whole workgroup. Indices, out-of-range buffer loads, segments dealt to
 // ranges and the partial slots [range][k][cin][cout] are as in
 // conv_dw_pos_bf16_kernel.
-template <int NB, int KPW, int WAVES>
+// MASK: channel counts that are not multiples of 64, their last chunk and
+// tile part empty (loads past the row's channels read nothing, outputs there
+// are not written).
+template <int NB, int KPW, int WAVES, bool MASK = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(WAVES))) void
 conv_dw_shx_bf16_kernel(const __bf16 *__restrict__ x, int64_t n_in, int cin,
                         const __bf16 *__restrict__ gy, int cout, const int32_t *__restrict__ nbr,
@@ -2404,19 +2407,23 @@ conv_dw_shx_bf16_kernel(const __bf16 *__restrict__ x, int64_t n_in, int cin,
   // 16-byte piece l%8 of its X rows (64 channels) and of its dY row (16*NB
   // channels: lanes past 16*NB load nothing)
   const int prow8 = 8 * wv + (lane >> 3);
+  const uint32_t xoob = MASK && c0 + 8 * (lane & 7) >= cin ? kBufOob : 0u;
+  const int32_t ykeep =
+      opaque(lane < 16 * NB && (!MASK || co0 + 8 * (lane % (2 * NB)) < cout) ? -1 : 0);
   auto load_dat = [&](const Seg &S, int s, Dat &D) {
     const int src = (32 * s + prow8) * 4;
 #pragma unroll
     for (int j = 0; j < KPW; ++j) {
-      const uint32_t o = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(src, S.id[j])) + 16 * (lane & 7);
+      uint32_t o = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(src, S.id[j])) + 16 * (lane & 7);
+      if constexpr (MASK)
+        o |= xoob;
       D.xv[j] = __builtin_amdgcn_raw_buffer_load_b128(rx, o, 0, 0);
     }
     const int q = 8 * wv + lane / (2 * NB);
     const uint32_t o =
         static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute((32 * s + (q & 31)) * 4, S.orow)) +
         16 * (lane % (2 * NB));
-    D.yv = __builtin_amdgcn_raw_buffer_load_b128(ry, pick(o, opaque(lane < 16 * NB ? -1 : 0)), 0,
-                                                 0);
+    D.yv = __builtin_amdgcn_raw_buffer_load_b128(ry, pick(o, ykeep), 0, 0);
   };
   auto step_live = [](const uint64_t (&live)[KPW], int j, int s) {
     return ((live[j] >> (32 * s)) & 0xffffffffull) != 0;
@@ -2496,7 +2503,7 @@ conv_dw_shx_bf16_kernel(const __bf16 *__restrict__ x, int64_t n_in, int cin,
   // lane holds D[4g+e][i16] of block nb: dW[k][ci0 + 4g + e][co0 + 16nb + i16]
 #pragma unroll
   for (int j = 0; j < KPW; ++j) {
-    if (kk[j] >= K)
+    if (kk[j] >= K || (MASK && ci0 >= cin))
       continue;
     float *dst = partial + ((static_cast<int64_t>(rg) * K + kk[j]) * cin + ci0 + 4 * g) * cout +
                  co0 + i16;
@@ -2504,7 +2511,8 @@ conv_dw_shx_bf16_kernel(const __bf16 *__restrict__ x, int64_t n_in, int cin,
     for (int e = 0; e < 4; ++e)
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb)
-        dst[static_cast<int64_t>(e) * cout + 16 * nb] = acc[j][nb][e];
+        if (!MASK || co0 + 16 * nb < cout)
+          dst[static_cast<int64_t>(e) * cout + 16 * nb] = acc[j][nb][e];
   }
 }
 
@@ -2663,6 +2671,8 @@ static void launch_os(const T *x, int cred, const T *wt, int credw, int ncols,
 template <typename T> static int os_nt(int ncols) {
   if (!kIsF32<T> && ncols % 128 == 0)
     return 128;
+  if (!kIsF32<T> && ncols % 96 == 0)
+    return 96;
   return ncols % 64 == 0 ? 64 : (ncols % 32 == 0 ? 32 : 16);
 }
 
@@ -2756,7 +2766,8 @@ template <typename T> static int os_splits(int64_t n_rows, int cred, int ncols, 
   if (n_rows <= 0 || ncols % 16 != 0)
     return 1;
   const int nt = os_nt<T>(ncols);
-  const int rows = kWaves * 16 * (!kIsF32<T> && nt >= 128 ? kWideRG : 1);
+  const bool wide = !kIsF32<T> && (nt >= 128 || (nt == 96 && cred >= 64));
+  const int rows = kWaves * 16 * (wide ? kWideRG : 1);
   const int64_t blocks = ceil_div(n_rows, rows) * (ncols / nt);
   const int64_t stages = static_cast<int64_t>(K) * std::max(1, cred / 64);
   const int64_t want = (640 + blocks / 2) / blocks; // nearest
@@ -2869,6 +2880,18 @@ static bool os_lds_shape(const T *x, int64_t n_x, int cred, const T *wt, const i
     constexpr int G = NT <= 32 ? 4 / CSUB : 1;
     return launch_os_lds<T, NT, 1, CSUB, G, NT == 64 ? 6 : 8, KQ>(
         x, n_x, cred, wt, wperm, ncols, bias, nbr, n_rows, K, order, y, splits, partial, s);
+  } else if constexpr (NT == 96 || (NT < 96 && CSUB == 3)) {
+    // widths of 96 and 192: whole 96-channel stages and 96-column tiles where
+    // 32-channel stages and 32-column tiles gathered every row again per tile.
+    // Forward on MI355X, before / one / two row groups per wave: 96->96 on 101k
+    // rows 146 / 77 / 79 us, on 10k rows 60 / 30 / 30; 192->192 on 48k rows 174
+    // / 167 / 154; 128->96 80 / 66 / 60; 96->64 63 / 37 / 43; 32->96 on 101k
+    // rows 39 / 33 / 39
+    if (wtr)
+      return false;
+    constexpr int RG = NT == 96 && CSUB >= 2 ? kWideRG : 1;
+    return launch_os_lds<T, NT, RG, CSUB, 1, 4, KQ>(x, n_x, cred, wt, wperm, ncols, bias, nbr,
+                                                    n_rows, K, order, y, splits, partial, s);
   } else if constexpr (NT < 128) {
     // untransposed weights only in 128-column tiles: the narrower shapes run
     // at 6-8 waves per SIMD, where the transposed reads' registers spill
@@ -2906,6 +2929,10 @@ static bool os_lds_csub(const T *x, int64_t n_x, int cred, const T *wt, const in
     if (cred % (4 * CH) == 0)
       return os_lds_shape<T, NT, 4, KQ>(x, n_x, cred, wt, wperm, ncols, bias, nbr, n_rows, K,
                                         order, y, splits, partial, s, wtr);
+  } else {
+    if (cred == 3 * CH || cred == 6 * CH)
+      return os_lds_shape<T, NT, 3, KQ>(x, n_x, cred, wt, wperm, ncols, bias, nbr, n_rows, K,
+                                        order, y, splits, partial, s, wtr);
   }
   if (cred % (2 * CH) == 0)
     return os_lds_shape<T, NT, 2, KQ>(x, n_x, cred, wt, wperm, ncols, bias, nbr, n_rows, K, order,
@@ -2924,6 +2951,9 @@ static bool run_os_lds_nt(const T *x, int64_t n_x, int cred, const T *wt, const 
     if (nt == 128)
       return os_lds_csub<T, 128, KQ>(x, n_x, cred, wt, wperm, ncols, bias, nbr, n_rows, K, order,
                                      y, splits, partial, s, wtr);
+    if (nt == 96)
+      return os_lds_csub<T, 96, KQ>(x, n_x, cred, wt, wperm, ncols, bias, nbr, n_rows, K, order,
+                                    y, splits, partial, s, wtr);
   }
   if (nt == 64)
     return os_lds_csub<T, 64, KQ>(x, n_x, cred, wt, wperm, ncols, bias, nbr, n_rows, K, order, y,
@@ -3372,17 +3402,29 @@ static int dw_pos_ranges(int K, int cin, int cout, int vb, int waves, int64_t n_
 // at most 8 offsets and channel counts that are not multiples of 64 keep
 // conv_dw_pos_bf16_kernel.
 constexpr int kDwShxKPW = 7;
-static bool dw_shx_bf16(int K, int cin, int cout) {
-  return K > kDwPosMaxKSmall && cin % 64 == 0 && cout % 64 == 0;
+// Output channels that are not a multiple of 64 (96 above all) take it too,
+// the last tile part empty: conv_dw_pos_bf16_kernel has them in 32-channel
+// tiles, which read the X rows once each. Measured per call: 128->96 on 48k
+// rows 110 -> 74 us. Where the last input chunk is part empty as well, only on
+// large maps: 96->96 on 101k rows 149 -> 129, but on 10k 41 -> 54; with whole
+// output tiles never (96->128 on 48k 64 -> 72).
+constexpr int64_t kDwShxPartRows = 65536;
+static bool dw_shx_bf16(int K, int cin, int cout, int64_t n_out) {
+  if (K <= kDwPosMaxKSmall || cin % 16 != 0 || cout % 32 != 0)
+    return false;
+  if (cout % 64 == 0)
+    return cin % 64 == 0;
+  return cout > 64 && (cin % 64 == 0 || (cin > 64 && n_out >= kDwShxPartRows));
 }
 
 // Ranges of conv_dw_pos_bf16_kernel (or conv_dw_shx_bf16_kernel) and
 // conv_dw_pos_kernel for a shape (the workspace query and the launches share
 // them).
 static int dw_pos_bf16_ranges(int K, int cin, int cout, int64_t n_out) {
-  if (dw_shx_bf16(K, cin, cout))
-    return dw_ranges_for((cin / 64) * (cout / 64) * static_cast<int>(ceil_div(K, kDwShxKPW)), 2,
-                         n_out, 16);
+  if (dw_shx_bf16(K, cin, cout, n_out))
+    return dw_ranges_for(static_cast<int>(ceil_div(cin, 64) * ceil_div(cout, 64) *
+                                          ceil_div(K, kDwShxKPW)),
+                         2, n_out, 16);
   const int waves = K <= kDwPosMaxKSmall ? 4 : 2;
   return dw_pos_ranges(K, cin, cout, cout % 64 == 0 ? 4 : 2, waves, n_out, 16);
 }
@@ -3426,12 +3468,17 @@ static void run_dw_pos_bf16(const __bf16 *x, int64_t n_in, int cin, const __bf16
   const int ranges = dw_pos_bf16_ranges(K, cin, cout, n_out);
   const int groups = static_cast<int>(ceil_div(K, kWaves * dw_pos_kpw(K)));
   const int ct = cin / 16, ot = cout / (16 * vb);
-  if (n_in > 0 && n_out > 0 && dw_shx_bf16(K, cin, cout)) {
-    const int cc = cin / 64, sgroups = static_cast<int>(ceil_div(K, kDwShxKPW));
-    hipLaunchKernelGGL((conv_dw_shx_bf16_kernel<4, kDwShxKPW, 2>),
-                       dim3(static_cast<unsigned>(ranges * cc * ot * sgroups)), dim3(kThreads), 0,
-                       s, x, n_in, cin, gy, cout, nbr, out_order, n_out, K, ranges, cc, ot,
-                       partial);
+  if (n_in > 0 && n_out > 0 && dw_shx_bf16(K, cin, cout, n_out)) {
+    const int cc = static_cast<int>(ceil_div(cin, 64)), co = static_cast<int>(ceil_div(cout, 64));
+    const int sgroups = static_cast<int>(ceil_div(K, kDwShxKPW));
+    const dim3 grid(static_cast<unsigned>(ranges * cc * co * sgroups));
+    if (cin % 64 == 0 && cout % 64 == 0)
+      hipLaunchKernelGGL((conv_dw_shx_bf16_kernel<4, kDwShxKPW, 2>), grid, dim3(kThreads), 0, s, x,
+                         n_in, cin, gy, cout, nbr, out_order, n_out, K, ranges, cc, co, partial);
+    else
+      hipLaunchKernelGGL((conv_dw_shx_bf16_kernel<4, kDwShxKPW, 2, true>), grid, dim3(kThreads), 0,
+                         s, x, n_in, cin, gy, cout, nbr, out_order, n_out, K, ranges, cc, co,
+                         partial);
     RHIP_LAUNCH_CHECK();
   } else if (n_in > 0 && n_out > 0) {
     const dim3 grid(static_cast<unsigned>(ranges * ct * ot * groups));
