@@ -28,7 +28,8 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 
 HIP_SOURCES = ["abi.hip", "sort.hip", "hash.hip", "kmap.hip", "conv.hip", "conv_thin.hip",
-               "conv_x3.hip", "conv_pad.hip", "pool.hip", "norm.hip"]
+               "conv_x3.hip", "conv_pad.hip", "conv_small.hip",
+               "pool.hip", "norm.hip"]
 # gfx950 only. Packed-FP32 instructions are disabled: the compiler would
 # otherwise form v_pk_* FP32 ops from plain float code.
 HIP_FLAGS = [

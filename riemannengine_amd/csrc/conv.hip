@@ -37,6 +37,7 @@
 #include <type_traits>
 
 #include "conv_pad.hpp"
+#include "conv_small.hpp"
 #include "conv_thin.hpp"
 #include "conv_x3.hpp"
 
@@ -3750,6 +3751,20 @@ static void conv_forward_into(const T *x, int64_t n_in, int32_t cin, const T *we
       return;
     }
   }
+  if (conv_small_takes<T>(n_out, n_in, cin, cout, K) && aligned16(x)) {
+    const T *wn = weight;
+    if constexpr (!kIsF32<T>) { // the bf16 operands hold eight channels of a column
+      T *wt = static_cast<T *>(w.wt);
+      const int64_t nw = static_cast<int64_t>(K) * cin * cout;
+      hipLaunchKernelGGL((transpose_w_kernel<T>), dim3(ceil_div(nw, kThreads)), dim3(kThreads), 0,
+                         stream, weight, K, cin, cout, cin, wt);
+      RHIP_LAUNCH_CHECK();
+      wn = wt;
+    }
+    conv_small<T>(x, n_in, cin, wn, kIsF32<T>, nullptr, cout, bias, nbr, n_out, K, out_order, y,
+                  stream);
+    return;
+  }
   if constexpr (kIsF32<T>) {
     if (conv_x3_takes(cin, cout, K, n_in) && aligned16(x) && aligned16(y) &&
         w.wt_bytes >= conv_x3_weight_bytes(K, cin, cout)) {
@@ -3818,6 +3833,11 @@ static void conv_backward_input_into(const T *grad_y, int64_t n_out, int32_t cou
   const T *wk = weight;
   const int32_t *wperm = weight_perm;
   int credw = cout;
+  if (conv_small_takes<T>(n_in, n_out, cout, cin, K) && aligned16(grad_y) && aligned16(weight)) {
+    conv_small<T>(grad_y, n_out, cout, weight, false, weight_perm, cin, nullptr, nbr_t, n_in, K,
+                  in_order, grad_x, stream);
+    return;
+  }
   if (w != nullptr) {
     if constexpr (kIsF32<T>) {
       if (conv_x3_takes(cout, cin, K, n_out) && aligned16(grad_y) && aligned16(grad_x) &&

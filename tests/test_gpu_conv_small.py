@@ -1,0 +1,39 @@
+"""Maps with few rows: forward with bias and input gradient of the kernel
+whose waves share out a 16-row tile's stages, against the oracle at its edges
+(16 rows, 16 / 32 / 64 columns, one chunk or several, fewer stages than waves,
+1 to 32 offsets, both weight layouts). Tolerance: norm-wise rel 1e-4 for fp32
+and 2e-2 for bf16 (helpers.TOL)."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from riemannengine_amd import abi
+from helpers import TOL, assert_rel, gpu_tables_and_map, random_coords, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,off,cin,cout", [
+    (1, (3, 3), 32, 16), (15, (3, 3), 16, 32), (16, (3, 1), 64, 64), (17, (3, 3), 32, 48),
+    (33, (3, 3), 96, 32), (200, (3, 2), 32, 64), (500, (3, 3), 64, 64), (900, (2, 5), 32, 32),
+    (130, (5, 2), 32, 80), (700, (3, 3), 256, 16), (2100, (3, 3), 32, 32)])
+def test_small_map_layers_match_oracle(n, off, cin, cout, dtype):
+    D, ks = off
+    rng = np.random.default_rng(n + cin)
+    span = 30 if D == 2 else (3 if D == 5 else 6)
+    c, _, _ = oracle.insert_and_map(random_coords(rng, 6 * n + 8, D, span))
+    km = gpu_tables_and_map(c[:n], c[:n], oracle.region_offsets(D, ks), same=True)[2]
+    x, gy = (to_dev(rng.standard_normal((n, k)).astype(np.float32), dtype) for k in (cin, cout))
+    w = to_dev((rng.standard_normal((km.K, cin, cout)) / 20).astype(np.float32), dtype)
+    b = rng.standard_normal(cout).astype(np.float32)
+    print(f"small n={n} K={km.K} {cin}->{cout} {dtype}", flush=True)
+    y, gx = abi.conv_forward(x, w, km, bias=to_dev(b)), abi.conv_backward_input(gy, w, km)
+    kofs, ir, orr = km.offsets_host, km.in_rows.cpu().numpy(), km.out_rows.cpu().numpy()
+    xs, gs, ws = (t.float().cpu().numpy() for t in (x, gy, w))
+    assert_rel(y.float().cpu().numpy(), oracle.conv_forward(xs, ws, kofs, ir, orr, n) + b,
+               TOL[dtype], "Y")
+    assert_rel(gx.float().cpu().numpy(), oracle.conv_backward(xs, gs, ws, kofs, ir, orr)[0],
+               TOL[dtype], "dX")
+    assert torch.equal(y, abi.conv_forward(x, w, km, bias=to_dev(b)))
