@@ -31,7 +31,9 @@
 //   sort     stable radix sort of the rows by key;
 //   query    one lane per processing position p resolves its row's K
 //            neighbours and writes nbr[k][p] (coalesced over p), out_order[p]
-//            and per wave and offset the count of hits (ballots);
+//            and per wave and offset the count of hits (ballots); without
+//            bricks and for up to 32 offsets the masks pass keeps the
+//            neighbours it found and this pass permutes them;
 //   scan     per-offset exclusive scans of the wave counts, then the CSR
 //            offsets of the pairs.
 // Phase 2 (rhip_kmap_fill):
@@ -373,18 +375,28 @@ __device__ __forceinline__ void probe81_bricks(const TableView &t, const int32_t
   }
 }
 
+// Entries per row of the neighbours the mask pass keeps (16-byte pieces).
+__host__ __device__ __forceinline__ int kept_stride(int K) { return (K + 3) / 4 * 4; }
+constexpr int kKeptK = 32; // kept for at most this many offsets
+
 // Mask pass: one lane per output row j in spatial order (row spatial[j]):
 // keys[j] = the sort key of the row's neighbour mask, vals[j] = its output
 // row spatial[j].
 // KC > 0: K == KC at compile time (the probe rounds unroll and the stencil
 // loads hoist out of them). NBHD: the symmetric 3^3 map through
 // probe27_bricks (KC == 27, D == 3) or 3^4 map through probe81_bricks
-// (KC == 81, D == 4).
-template <int D, int KC = 0, bool NBHD = false>
+// (KC == 81, D == 4). KEEP: also the neighbours found, rows[o][k] of
+// kept_stride(K) entries, for kmap_permute_kernel: a probe of a table
+// without bricks is a random slot read, and the query repeated all of them
+// (a LiDAR sweep's 3^3 map of 76k rows on MI355X: mask and query 50 + 50 us,
+// with the rows kept 56 + 10; the whole voxelisation and map 855 -> 755). With
+// bricks a probe is one load near the last one's, and the passes stay as they
+// were (not compared there).
+template <int D, int KC = 0, bool NBHD = false, bool KEEP = false>
 __global__ __launch_bounds__(kMapBlock) void kmap_mask_kernel(
     TableView t, const int32_t *__restrict__ out_coords, const int32_t *__restrict__ spatial,
     int64_t n_out, const int32_t *__restrict__ offsets, int K, uint32_t *__restrict__ keys,
-    int32_t *__restrict__ vals) {
+    int32_t *__restrict__ vals, int32_t *__restrict__ rows = nullptr) {
   if constexpr (KC > 0)
     K = KC;
   const int64_t j = blockIdx.x * (int64_t)kMapBlock + threadIdx.x;
@@ -425,7 +437,15 @@ __global__ __launch_bounds__(kMapBlock) void kmap_mask_kernel(
 #pragma unroll
   for (int k0 = 0; k0 < (KC > 0 ? KC : K); k0 += 8) {
     int32_t r[8];
-    probe8<D, false>(t, c, d0, row_ok, offsets, k0, K, r);
+    probe8<D, KEEP>(t, c, d0, row_ok, offsets, k0, K, r);
+    if constexpr (KEEP) {
+      const int ks = kept_stride(K);
+#pragma unroll
+      for (int u = 0; u < 8; u += 4)
+        if (k0 + u < ks)
+          *reinterpret_cast<int4 *>(rows + o * ks + k0 + u) =
+              make_int4(r[u], r[u + 1], r[u + 2], r[u + 3]);
+    }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int k = k0 + u;
@@ -515,6 +535,40 @@ __global__ __launch_bounds__(kMapBlock) void kmap_query_kernel(
         if (in)
           nbr[k * n_out + p] = r[u];
         const uint64_t hits = __ballot(r[u] >= 0);
+        if (lane_id() == 0)
+          wave_counts[k * nw + w] = __popcll(hits);
+      }
+    }
+  }
+}
+
+// The query pass from kept neighbours: position p's row of `rows` to nbr's
+// column p, with the outputs of kmap_query_kernel.
+__global__ __launch_bounds__(kMapBlock) void kmap_permute_kernel(
+    const int32_t *__restrict__ rows, const int32_t *__restrict__ jpos, int64_t n_out, int K,
+    int64_t nw, int32_t *__restrict__ nbr, int32_t *__restrict__ out_order,
+    int32_t *__restrict__ wave_counts, uint32_t *__restrict__ ticket) {
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+    *ticket = 0;
+  const int64_t p = blockIdx.x * (int64_t)kMapBlock + threadIdx.x;
+  const int64_t w = p / kWave;
+  if (w >= nw) // whole waves past the last row
+    return;
+  const bool in = p < n_out;
+  const int32_t o = in ? jpos[p] : 0;
+  if (in)
+    out_order[p] = o;
+  const int ks = kept_stride(K);
+  for (int k0 = 0; k0 < K; k0 += 4) {
+    const int4 v4 = *reinterpret_cast<const int4 *>(rows + static_cast<int64_t>(o) * ks + k0);
+    const int32_t v[4] = {v4.x, v4.y, v4.z, v4.w};
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int k = k0 + u;
+      if (k < K) { // uniform
+        if (in)
+          nbr[k * n_out + p] = v[u];
+        const uint64_t hits = __ballot(in && v[u] >= 0);
         if (lane_id() == 0)
           wave_counts[k * nw + w] = __popcll(hits);
       }
@@ -736,6 +790,7 @@ struct KmapWs {
   int32_t *vals_a, *vals_b;
   void *sort_tmp;
   size_t sort_bytes;
+  int32_t *rows; // the mask pass's neighbours (tables without bricks)
   // phase 2
   unsigned long long *mask_t;
   uint32_t *tkeys_a, *tkeys_b;
@@ -761,6 +816,7 @@ static KmapWs carve_kmap(Carve &cv, int64_t n_in, int64_t n_out, int32_t K, int3
   w.vals_b = cv.take<int32_t>(mo);
   w.sort_bytes = sort_pairs_u32_bytes(mo);
   w.sort_tmp = cv.take<char>(w.sort_bytes);
+  w.rows = cv.take<int32_t>(K <= kKeptK ? static_cast<size_t>(mo) * kept_stride(K) : 1);
   const size_t end1 = cv.used;
   cv.used = base;
   w.mask_t = cv.take<unsigned long long>(2 * mi);
@@ -973,6 +1029,23 @@ extern "C" int rhip_kmap_count(const rhip_table *in_table, const int32_t *out_co
             RHIP_LAUNCH_CHECK();
             return;
           }
+        }
+        if (masks && K <= kKeptK && tv.bricks == nullptr) {
+          if (k27)
+            hipLaunchKernelGGL((kmap_mask_kernel<DD, 27, false, true>), dim3(nb), dim3(kMapBlock),
+                               0, stream, tv, out_coords, out_spatial_order, n_out, w.offsets, K,
+                               w.keys_a, w.vals_a, w.rows);
+          else
+            hipLaunchKernelGGL((kmap_mask_kernel<DD, 0, false, true>), dim3(nb), dim3(kMapBlock),
+                               0, stream, tv, out_coords, out_spatial_order, n_out, w.offsets, K,
+                               w.keys_a, w.vals_a, w.rows);
+          RHIP_LAUNCH_CHECK();
+          sort_pairs_u32(w.sort_tmp, w.sort_bytes, w.keys_a, w.keys_b, w.vals_a, w.vals_b,
+                         n_out, mask_key_bits(K), stream);
+          hipLaunchKernelGGL(kmap_permute_kernel, dim3(nb), dim3(kMapBlock), 0, stream, w.rows,
+                             w.vals_b, n_out, K, nw, nbr, out_order, w.wave_counts, w.ticket);
+          RHIP_LAUNCH_CHECK();
+          return;
         }
         if (masks) {
           if (k27)
