@@ -14,21 +14,26 @@
 //    rows straight into MFMA operands. conv_os_lds_kernel (stencils of up to
 //    96 offsets) keeps its row groups' neighbour indices in LDS and walks the
 //    workgroup's offsets as a bit mask; conv_os_kernel is the general form
-//    (larger stencils, fp32 offset splits, padded 16-channel bf16 layers);
-//    conv_fr_kernel keeps every offset's weights for its columns resident in
+//    (larger stencils, narrow fp32 offset splits, padded 16-channel bf16
+//    layers); conv_fr_kernel keeps every offset's weights for its columns resident in
 //    LDS (bf16 maps the first does not take whose weights fit). Without an
 //    offset split each output row is written once: no atomics, no zero
-//    fill; with one, fp32 partial sums are added in split order.
+//    fill; with one, fp32 partial sums are added in split order. Beside them:
+//    conv_x3 runs fp32 layers of 64 channels and more on the bf16 matrix cores
+//    (each operand in three parts), conv_small maps with few rows, conv_thin
+//    layers with few im2col columns, and layers whose channel counts no tiled
+//    kernel takes run here on padded copies (conv_pad).
 //  * Gathered rows are loaded in quad order (four consecutive lanes read 64
 //    contiguous bytes of one row, one L1 access) and moved to the MFMA layout
 //    with ds_bpermute.
-//  * dW has three kernels, all writing per-workgroup partial tiles that a
-//    second kernel adds in a fixed order (deterministic, no atomics):
-//    conv_dw_kernel over the per-offset pair lists (split-pair reduction),
-//    conv_dw_rows_kernel over the neighbour table for narrow bf16 layers, and
-//    the position-stationary conv_dw_pos_kernel / conv_dw_pos_bf16_kernel,
-//    which keep the tiles of up to 28 offsets in registers while they stream
-//    the output positions.
+//  * The dW kernels all write per-workgroup partial tiles that a second
+//    kernel adds in a fixed order (deterministic, no atomics): conv_dw_kernel
+//    and conv_dw_pairs_bf16_kernel over the per-offset pair lists (split-pair
+//    reduction), conv_dw_rows_kernel over the neighbour table for narrow bf16
+//    layers, the position-stationary conv_dw_pos_kernel / conv_dw_pos64_kernel
+//    / conv_dw_pos_bf16_kernel / conv_dw_shx_bf16_kernel, which keep the tiles
+//    of up to 28 offsets in registers while they stream the output positions,
+//    and conv_dw_thin for layers with few im2col columns.
 //  * The reduction order inside an MFMA is a permutation of the reduced axis
 //    chosen so that each lane reads 16 contiguous bytes; A and B use the same
 //    permutation, so the sum is unchanged.
@@ -2967,8 +2972,8 @@ static bool run_os_lds_nt(const T *x, int64_t n_x, int cred, const T *wt, const 
 }
 
 // The fast forward/dX kernel where it applies: at most 96 offsets, no split,
-// unpadded reductions of one, two or four chunks and inputs that 32-bit
-// buffer offsets reach. Returns whether it launched.
+// unpadded reductions of one, two or four chunks (bf16 also three and six)
+// and inputs that 32-bit buffer offsets reach. Returns whether it launched.
 template <typename T>
 static bool run_os_lds(const T *x, int64_t n_x, int cred, const T *wt, const int32_t *wperm,
                        int credw, int ncols, const float *bias, const int32_t *nbr,

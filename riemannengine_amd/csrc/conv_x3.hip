@@ -13,7 +13,9 @@
 // MFMAs': 64->64 9.6e-8 / 7.9e-8 against 3.8e-7 / 2.7e-7, 256->256 3.7e-7 /
 // 3.0e-7 against 1.1e-6 / 7.5e-7.
 //
-// Where parts cannot represent a value (infinities, NaN, magnitudes that
+// Below 2^-110 the later parts reach bf16's smallest values and hold fewer
+// bits: such an operand is off by up to 2^-134 itself. Where parts cannot
+// represent a value (infinities, NaN, magnitudes that
 // round to infinity in bf16) some part is not finite, and so is every output
 // it reaches. A wave that finds such an output adds its rows up again in
 // plain fp32, over the pairs that exist (the split form: in its reduction).

@@ -164,8 +164,9 @@ at::Tensor hip_sparse_convolution(const at::Tensor &features, const at::Tensor &
       bias.defined() ? bias
                      : torch::empty({0}, features.options().dtype(torch::kFloat));
   // dW from the neighbour table where the library has a kernel for the
-  // shape (tiled, or ragged channel counts), else from the pair lists (built now, once per map, when a weight
-  // gradient may follow). bf16 maps of at most 8 offsets take the pair lists
+  // shape (tiled, or ragged channel counts), else from the pair lists (built
+  // now, once per map, when a weight gradient may follow). bf16 maps of at
+  // most 8 offsets take the pair lists
   // when they hold fewer than 2 pairs per output row (a transposed stride-2
   // map), or pair each input row at most once (a stride-2 map) with channel
   // counts that are multiples of 64 (the per-wave pair kernel). Measured per
