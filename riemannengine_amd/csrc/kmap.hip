@@ -24,7 +24,8 @@
 //            issued together; a symmetric 3^3 map in 3-D reads the (at most
 //            8) bricks of a row's neighbourhood once and derives all 27
 //            probes from them (probe27_bricks);
-//   masks    one lane per output row (in the output map's locality order)
+//   masks    one lane per output row (in the output map's locality order;
+//            without bricks and for up to 32 offsets four offsets a lane)
 //            folds the existence of its K neighbours into a sort key (the
 //            mask for K <= 16, else the neighbour count above a 15-bit hash
 //            of the mask);
@@ -87,7 +88,7 @@ __device__ __forceinline__ uint32_t mask_key(uint64_t m0, uint64_t m1, int K) {
 // Bits of mask_key for K offsets.
 static int mask_key_bits(int K) { return K <= kKeyBits ? K : (K <= 31 ? 16 : 22); }
 
-// Resolves probes k0 .. k0+7 of an output row with coordinates c (batch
+// Resolves probes k0 .. k0+U-1 of an output row with coordinates c (batch
 // offset d0 = c[0] - lo[0], row_ok = the batch is in range): r[u] = the
 // input row at c + offsets[k0 + u] (batch kept, wrap-around int32 arithmetic
 // as the coordinate type has), or -1. With kRows false only r[u] >= 0
@@ -95,22 +96,22 @@ static int mask_key_bits(int K) { return K <= kKeyBits ? K : (K <= 31 ? 16 : 22)
 //   brick index: the neighbour's brick entry, then the rank of its cell among
 //     the brick's occupied cells gives its locality-order position;
 //   packed keys: each neighbour's key is packed column by column (a column
-//     leaving [lo, hi] is a miss, as in pack_row), the home slots of all 8
+//     leaving [lo, hi] is a miss, as in pack_row), the home slots of all U
 //     probes are loaded before any chain is followed;
 //   row-reference tables: table_find.
-template <int D, bool kRows>
-__device__ __forceinline__ void probe8(const TableView &t, const int32_t *c, uint32_t d0,
-                                       bool row_ok, const int32_t *__restrict__ offsets, int k0,
-                                       int K, int32_t (&r)[8]) {
+template <int D, bool kRows, int U = 8>
+__device__ __forceinline__ void probe_run(const TableView &t, const int32_t *c, uint32_t d0,
+                                          bool row_ok, const int32_t *__restrict__ offsets,
+                                          int k0, int K, int32_t (&r)[U]) {
   if constexpr (D <= 6) {
     if (t.bricks != nullptr) {
       constexpr int L = 6 / D;
-      uint64_t g[8];
-      uint32_t cell[8];
-      bool ok[8];
-      Brick br[8];
+      uint64_t g[U];
+      uint32_t cell[U];
+      bool ok[U];
+      Brick br[U];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
+      for (int u = 0; u < U; ++u) {
         const int k = k0 + u;
         ok[u] = row_ok && k < K;
         g[u] = d0;
@@ -130,29 +131,29 @@ __device__ __forceinline__ void probe8(const TableView &t, const int32_t *c, uin
         }
       }
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
+      for (int u = 0; u < U; ++u)
         if (ok[u])
           br[u] = t.bricks[g[u]];
-      int32_t jj[8];
+      int32_t jj[U];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
+      for (int u = 0; u < U; ++u) {
         jj[u] = -1;
         if (ok[u] && ((br[u].mask >> cell[u]) & 1ull))
           jj[u] = br[u].base + __popcll(br[u].mask & ((1ull << cell[u]) - 1ull));
       }
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
+      for (int u = 0; u < U; ++u)
         r[u] = kRows ? (jj[u] >= 0 ? t.order[jj[u]] : -1) : jj[u];
       return;
     }
   }
   if (t.mode == RHIP_KEY_PACKED64) {
     const uint64_t base = static_cast<uint64_t>(d0) << t.shift[0];
-    uint64_t key[8], h[8];
-    bool ok[8];
-    Slot sl[8];
+    uint64_t key[U], h[U];
+    bool ok[U];
+    Slot sl[U];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int k = k0 + u;
       ok[u] = row_ok && k < K;
       key[u] = base;
@@ -168,11 +169,11 @@ __device__ __forceinline__ void probe8(const TableView &t, const int32_t *c, uin
       h[u] = mix64(key[u]) & t.mask;
     }
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
+    for (int u = 0; u < U; ++u)
       if (ok[u])
         sl[u] = t.slots[h[u]];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < U; ++u) {
       r[u] = -1;
       if (ok[u]) {
         while (sl[u].word != key[u] && sl[u].word != kEmptyWord) {
@@ -186,7 +187,7 @@ __device__ __forceinline__ void probe8(const TableView &t, const int32_t *c, uin
     return;
   }
 #pragma unroll
-  for (int u = 0; u < 8; ++u) {
+  for (int u = 0; u < U; ++u) {
     const int k = k0 + u;
     r[u] = -1;
     if (k < K) {
@@ -209,7 +210,7 @@ __device__ __forceinline__ void probe8(const TableView &t, const int32_t *c, uin
 // exact. Its 27 neighbours lie in at most 8 bricks: along each column the
 // row's brick and, where the cell sits on the brick's low (high) face, the
 // brick below (above). The row loads those bricks once, corner cc holding
-// the brick shifted along column i when bit i - 1 of cc is set (probe8 loads
+// the brick shifted along column i when bit i - 1 of cc is set (probe_run loads
 // one brick per offset: 27 loads, most of them the row's own brick again),
 // and reads every neighbour's occupancy bit and rank from the brick its
 // offset reaches. kRows: r[k] = the neighbour's row (through the locality
@@ -296,7 +297,7 @@ __device__ __forceinline__ void probe27_bricks(const TableView &t, const int32_t
 // the low face, 1: the high one), so its 81 neighbours lie in 16 bricks: the
 // row's own and, along each column, the one below (cell 0) or above (cell
 // 1). The row loads those 16 once, corner cc holding the brick shifted along
-// column i when bit i - 1 of cc is set (probe8 loads one brick per offset:
+// column i when bit i - 1 of cc is set (probe_run loads one brick per offset:
 // 81 loads), and each offset reads its neighbour's occupancy bit and rank
 // from the brick it reaches, selected by a 16-way tree. f(k, v) receives
 // each offset's result: the neighbour's row (through the locality order) or
@@ -378,6 +379,7 @@ __device__ __forceinline__ void probe81_bricks(const TableView &t, const int32_t
 // Entries per row of the neighbours the mask pass keeps (16-byte pieces).
 __host__ __device__ __forceinline__ int kept_stride(int K) { return (K + 3) / 4 * 4; }
 constexpr int kKeptK = 32; // kept for at most this many offsets
+constexpr int kKeptU = 4;  // probed by one lane
 
 // Mask pass: one lane per output row j in spatial order (row spatial[j]):
 // keys[j] = the sort key of the row's neighbour mask, vals[j] = its output
@@ -385,18 +387,12 @@ constexpr int kKeptK = 32; // kept for at most this many offsets
 // KC > 0: K == KC at compile time (the probe rounds unroll and the stencil
 // loads hoist out of them). NBHD: the symmetric 3^3 map through
 // probe27_bricks (KC == 27, D == 3) or 3^4 map through probe81_bricks
-// (KC == 81, D == 4). KEEP: also the neighbours found, rows[o][k] of
-// kept_stride(K) entries, for kmap_permute_kernel: a probe of a table
-// without bricks is a random slot read, and the query repeated all of them
-// (a LiDAR sweep's 3^3 map of 76k rows on MI355X: mask and query 50 + 50 us,
-// with the rows kept 56 + 10; the whole voxelisation and map 855 -> 755). With
-// bricks a probe is one load near the last one's, and the passes stay as they
-// were (not compared there).
-template <int D, int KC = 0, bool NBHD = false, bool KEEP = false>
+// (KC == 81, D == 4).
+template <int D, int KC = 0, bool NBHD = false>
 __global__ __launch_bounds__(kMapBlock) void kmap_mask_kernel(
     TableView t, const int32_t *__restrict__ out_coords, const int32_t *__restrict__ spatial,
     int64_t n_out, const int32_t *__restrict__ offsets, int K, uint32_t *__restrict__ keys,
-    int32_t *__restrict__ vals, int32_t *__restrict__ rows = nullptr) {
+    int32_t *__restrict__ vals) {
   if constexpr (KC > 0)
     K = KC;
   const int64_t j = blockIdx.x * (int64_t)kMapBlock + threadIdx.x;
@@ -437,15 +433,7 @@ __global__ __launch_bounds__(kMapBlock) void kmap_mask_kernel(
 #pragma unroll
   for (int k0 = 0; k0 < (KC > 0 ? KC : K); k0 += 8) {
     int32_t r[8];
-    probe8<D, KEEP>(t, c, d0, row_ok, offsets, k0, K, r);
-    if constexpr (KEEP) {
-      const int ks = kept_stride(K);
-#pragma unroll
-      for (int u = 0; u < 8; u += 4)
-        if (k0 + u < ks)
-          *reinterpret_cast<int4 *>(rows + o * ks + k0 + u) =
-              make_int4(r[u], r[u + 1], r[u + 2], r[u + 3]);
-    }
+    probe_run<D, false>(t, c, d0, row_ok, offsets, k0, K, r);
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int k = k0 + u;
@@ -527,7 +515,7 @@ __global__ __launch_bounds__(kMapBlock) void kmap_query_kernel(
 #pragma unroll
   for (int k0 = 0; k0 < (KC > 0 ? KC : K); k0 += 8) {
     int32_t r[8];
-    probe8<D, true>(t, c, d0, row_ok, offsets, k0, K, r);
+    probe_run<D, true>(t, c, d0, row_ok, offsets, k0, K, r);
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int k = k0 + u;
@@ -539,6 +527,54 @@ __global__ __launch_bounds__(kMapBlock) void kmap_query_kernel(
           wave_counts[k * nw + w] = __popcll(hits);
       }
     }
+  }
+}
+
+// The mask pass that also keeps the neighbours it finds, rows[o][k] of
+// kept_stride(K) entries, for kmap_permute_kernel: a probe of a table without
+// bricks is a random slot read, and the query repeated all of them. The pass
+// is bound by the probes' latency, so 2^lp adjacent lanes share a row, kKeptU
+// offsets each (K <= kKeptU << lp). A LiDAR sweep's 76k rows on MI355X, 27
+// offsets / a 2^3 map: probing twice 50 + 50 us for 27; kept by one lane per
+// row 56 + 10 / 18 + 10, by lanes of eight offsets 29 / 16, of four 28 / 14.
+// Following the eight chains of a lane in step instead of in turn, or two
+// slots of a chain per step, was slower (24 and 25 us against 22, mean of the
+// two maps). With bricks a probe is one load near the last one's and keeping the
+// rows lost (409k rows: 25 + 33 us probing twice, 40 + 39 kept).
+template <int D>
+__global__ __launch_bounds__(kMapBlock) void kmap_keep_kernel(
+    TableView t, const int32_t *__restrict__ out_coords, const int32_t *__restrict__ spatial,
+    int64_t n_out, const int32_t *__restrict__ offsets, int K, int lp,
+    uint32_t *__restrict__ keys, int32_t *__restrict__ vals, int32_t *__restrict__ rows) {
+  const int64_t i = blockIdx.x * (int64_t)kMapBlock + threadIdx.x;
+  const int64_t j = i >> lp;
+  if (j >= n_out) // all lanes of the row
+    return;
+  const int k0 = kKeptU * static_cast<int>(i & ((1 << lp) - 1));
+  const int64_t o = spatial ? spatial[j] : j;
+  int32_t c[D + 1];
+#pragma unroll
+  for (int d = 0; d <= D; ++d)
+    c[d] = out_coords[o * (D + 1) + d];
+  const uint32_t d0 = static_cast<uint32_t>(c[0]) - static_cast<uint32_t>(t.lo[0]);
+  int32_t r[kKeptU];
+  probe_run<D, true, kKeptU>(t, c, d0, d0 <= t.span[0], offsets, k0, K, r);
+  const int ks = kept_stride(K);
+  uint32_t m = 0;
+#pragma unroll
+  for (int u = 0; u < kKeptU; ++u)
+    m |= (r[u] >= 0 ? 1u : 0u) << u;
+#pragma unroll
+  for (int u = 0; u < kKeptU; u += 4)
+    if (k0 + u < ks)
+      *reinterpret_cast<int4 *>(rows + o * ks + k0 + u) =
+          make_int4(r[u], r[u + 1], r[u + 2], r[u + 3]);
+  m <<= k0;
+  for (int b = 1; b < (1 << lp); b <<= 1)
+    m |= __shfl_xor(m, b);
+  if (k0 == 0) {
+    keys[j] = mask_key(m, 0, K);
+    vals[j] = static_cast<int32_t>(o);
   }
 }
 
@@ -1031,14 +1067,13 @@ extern "C" int rhip_kmap_count(const rhip_table *in_table, const int32_t *out_co
           }
         }
         if (masks && K <= kKeptK && tv.bricks == nullptr) {
-          if (k27)
-            hipLaunchKernelGGL((kmap_mask_kernel<DD, 27, false, true>), dim3(nb), dim3(kMapBlock),
-                               0, stream, tv, out_coords, out_spatial_order, n_out, w.offsets, K,
-                               w.keys_a, w.vals_a, w.rows);
-          else
-            hipLaunchKernelGGL((kmap_mask_kernel<DD, 0, false, true>), dim3(nb), dim3(kMapBlock),
-                               0, stream, tv, out_coords, out_spatial_order, n_out, w.offsets, K,
-                               w.keys_a, w.vals_a, w.rows);
+          int lp = 0;
+          while (kKeptU << lp < K)
+            ++lp;
+          hipLaunchKernelGGL((kmap_keep_kernel<DD>),
+                             dim3(static_cast<unsigned>(ceil_div(n_out << lp, kMapBlock))),
+                             dim3(kMapBlock), 0, stream, tv, out_coords, out_spatial_order, n_out,
+                             w.offsets, K, lp, w.keys_a, w.vals_a, w.rows);
           RHIP_LAUNCH_CHECK();
           sort_pairs_u32(w.sort_tmp, w.sort_bytes, w.keys_a, w.keys_b, w.vals_a, w.vals_b,
                          n_out, mask_key_bits(K), stream);
