@@ -286,6 +286,29 @@ int rhip_conv_forward_workspace_bytes(int32_t K, int32_t cin, int32_t cout,
                                       int32_t dtype, int64_t n_in, int64_t n_out,
                                       size_t *bytes);
 
+/* The kernels of rhip_conv_forward and rhip_conv_backward_input. */
+typedef enum rhip_conv_kernel {
+  RHIP_CONV_ROWS = 0,     /* one lane per output */
+  RHIP_CONV_THIN = 1,     /* im2col rows in LDS (few reduced channels) */
+  RHIP_CONV_PADDED = 2,   /* one of those below, on padded copies */
+  RHIP_CONV_SMALL = 3,    /* 16-row tiles, the waves share out the stages */
+  RHIP_CONV_PARTS = 4,    /* fp32 operands as three bf16 parts */
+  RHIP_CONV_LDS = 5,      /* neighbour indices in LDS */
+  RHIP_CONV_RESIDENT = 6, /* all offsets' weights in LDS */
+  RHIP_CONV_TILED = 7     /* the general tiled kernel */
+} rhip_conv_kernel;
+
+/*
+ * Which kernel a call with a workspace and 16-byte aligned operands runs, and
+ * into how many parts it splits the (offset, channel) stages (1: no split;
+ * parts keep fp32 partial sums of n_rows x ncols in the workspace). A forward
+ * reduces cred = cin channels of n_x = n_in rows to ncols = cout columns of
+ * n_rows = n_out rows; an input gradient cout channels of n_out rows to cin
+ * columns of n_in rows. Host only, for tests and tools.
+ */
+int rhip_conv_plan(int32_t dtype, int32_t K, int32_t cred, int32_t ncols,
+                   int64_t n_x, int64_t n_rows, int32_t *kernel, int32_t *splits);
+
 /*
  * Y[out_order[j]] = sum_k X[nbr[k*n_out+j]] @ W[k] (+ bias), fp32 accumulate.
  * x [n_in, cin], weight [K, cin, cout], y [n_out, cout], all in `dtype`;

@@ -36,7 +36,8 @@ EXPORTS = (
     "rhip_kmap_pairs_workspace_bytes", "rhip_kmap_pairs", "rhip_stencil_partners",
     "rhip_conv_backward_weight_ragged", "rhip_conv_backward_weight_ragged_supported",
     "rhip_conv_backward_weight_rows_supported",
-    "rhip_conv_workspace_bytes", "rhip_conv_forward_workspace_bytes", "rhip_conv_forward",
+    "rhip_conv_workspace_bytes", "rhip_conv_forward_workspace_bytes", "rhip_conv_plan",
+    "rhip_conv_forward",
     "rhip_conv_forward_noalloc", "rhip_conv_bias_grad",
     "rhip_conv_backward_input", "rhip_conv_backward_weight", "rhip_conv_backward_weight_rows",
     "rhip_stride_map_workspace_bytes", "rhip_stride_map_count", "rhip_group_map_count",
@@ -90,6 +91,8 @@ def _declare(lib):
                                           _vp, _vp, _vp, _vp, _vp, _vp]),
         "rhip_conv_workspace_bytes": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i64, _i64, _i64,
                                                      _P(_sz)]),
+        "rhip_conv_plan": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i64, _i64, _P(_i32),
+                                          _P(_i32)]),
         "rhip_conv_forward": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i32, _i32, _vp, _vp,
                                              _vp, _i64, _vp, _i32, _vp, _sz, _vp]),
         "rhip_conv_forward_workspace_bytes": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i64, _i64,
@@ -482,6 +485,19 @@ def _conv_fwd_ws(K, cin, cout, dtype, dev, kmap: "KernelMap") -> torch.Tensor:
     """Workspace of the forward, input-gradient and bias-gradient calls."""
     return torch.empty(_sizeq(lib().rhip_conv_forward_workspace_bytes, K, cin, cout, dtype,
                               kmap.n_in, kmap.n_out), dtype=torch.uint8, device=dev)
+
+
+CONV_KERNELS = ("rows", "thin", "padded", "small", "parts", "lds", "resident", "tiled")
+
+
+def conv_plan(dtype: torch.dtype, K: int, cred: int, ncols: int, n_x: int, n_rows: int):
+    """(kernel name, splits) of a forward or input gradient with a workspace
+    and aligned operands, from rhip_conv_plan: cred channels of n_x rows to
+    ncols columns of n_rows rows."""
+    kernel, splits = _i32(0), _i32(0)
+    _check(lib().rhip_conv_plan(_dtype_code(dtype), K, cred, ncols, n_x, n_rows,
+                                ctypes.byref(kernel), ctypes.byref(splits)), "rhip_conv_plan")
+    return CONV_KERNELS[kernel.value], splits.value
 
 
 def conv_bias_grad(grad_y: torch.Tensor) -> torch.Tensor:

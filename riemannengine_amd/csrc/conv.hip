@@ -2718,6 +2718,15 @@ static void pick_csub(const T *x, int cred, const T *wt, int credw, int ncols,
                            partial, s);
 }
 
+// Offsets, and reduction widths, that the LDS-indexed kernel is built for
+// (os_lds_csub and launch_os_lds: one, two or four chunks, bf16 also three
+// and six).
+constexpr int kLdsMaxK = 96;
+template <typename T> constexpr bool os_lds_width(int cred) {
+  return cred == 32 || cred == 64 || cred == 128 || cred == 256 ||
+         (kIsF32<T> ? cred == 16 : cred == 96 || cred == 192);
+}
+
 // Whether the tiled MFMA kernels take a reduction of cred channels (credw
 // with its padding) to ncols columns over K offsets.
 template <typename T> static bool os_shape(int cred, int credw, int ncols, int K) {
@@ -2766,27 +2775,45 @@ static bool thin_runs(int K, int C, int64_t n_x, int elem_bytes, bool can_pad) {
 // for 9k rows at 256 channels), so the (offset, channel chunk) stages are
 // shared among up to 8 workgroups per tile, aiming at ~640 workgroups
 // (measured on the config-5 stages), each keeping at least 4 stages on
-// average. 1 = no split. The tiles counted are the fast kernel's (bf16
-// 128-column tiles hold kWideRG row groups per wave).
-template <typename T> static int os_splits(int64_t n_rows, int cred, int ncols, int K) {
+// average. 1 = no split. The tiles counted are those the reduction runs in:
+// bf16 128-column tiles hold kWideRG row groups per wave, and 96-column tiles
+// exist in the LDS-indexed kernel alone (32-column tiles elsewhere). credw:
+// the width red_width pads cred to, which is what the stages are counted in.
+template <typename T>
+static int os_splits(int64_t n_rows, int cred, int credw, int ncols, int K) {
   if (n_rows <= 0 || ncols % 16 != 0)
     return 1;
-  const int nt = os_nt<T>(ncols);
+  int nt = os_nt<T>(ncols);
+  if (nt == 96 && !(cred == credw && K <= kLdsMaxK && os_lds_width<T>(cred)))
+    nt = 32;
   const bool wide = !kIsF32<T> && (nt >= 128 || (nt == 96 && cred >= 64));
   const int rows = kWaves * 16 * (wide ? kWideRG : 1);
   const int64_t blocks = ceil_div(n_rows, rows) * (ncols / nt);
-  const int64_t stages = static_cast<int64_t>(K) * std::max(1, cred / 64);
+  const int64_t stages = static_cast<int64_t>(K) * std::max(1, credw / 64);
   const int64_t want = (640 + blocks / 2) / blocks; // nearest
   return static_cast<int>(
       std::max<int64_t>(1, std::min<int64_t>({8, want, std::max<int64_t>(1, stages / 4)})));
 }
 
-// Floats of split partial sums run_os needs (0 without a split).
+// Floats of split partial sums run_os needs (0 without a split) for a
+// reduction of cred channels that it pads by itself.
 template <typename T>
 static size_t os_partial_floats(int64_t n_rows, int cred, int ncols, int K) {
-  const int sp = os_splits<T>(n_rows, cred, ncols, K);
+  const int credw = red_width(kIsF32<T> ? RHIP_F32 : RHIP_BF16, cred);
+  const int sp = os_splits<T>(n_rows, cred, credw, ncols, K);
   return sp > 1 ? static_cast<size_t>(sp) * n_rows * ncols : 0;
 }
+
+// Partial sums of a split offset axis: `floats` of them at p (null: none).
+struct PartialBuf {
+  float *p = nullptr;
+  size_t floats = 0;
+  // the splits that a launch of n_rows x ncols outputs may use of `want`
+  int fit(int want, int64_t n_rows, int ncols) const {
+    const size_t per = static_cast<size_t>(n_rows) * ncols;
+    return p != nullptr && want > 1 && floats / per >= static_cast<size_t>(want) ? want : 1;
+  }
+};
 
 // One conv_os_lds_kernel launch; the split form is built for bf16 only (fp32
 // splits stay on conv_os_kernel).
@@ -2979,7 +3006,7 @@ static bool run_os_lds(const T *x, int64_t n_x, int cred, const T *wt, const int
                        int credw, int ncols, const float *bias, const int32_t *nbr,
                        int64_t n_rows, int K, const int32_t *order, T *y, int splits,
                        float *partial, hipStream_t s, bool wtr = false) {
-  if (K > 96 || cred != credw || n_x < 1 || !os_fast(x, cred, wt, credw, ncols, K) ||
+  if (K > kLdsMaxK || cred != credw || n_x < 1 || !os_fast(x, cred, wt, credw, ncols, K) ||
       n_x * cred * static_cast<int64_t>(sizeof(T)) > kBufMaxBytes)
     return false;
   if (K > 32)
@@ -3091,6 +3118,34 @@ static bool run_fr(const __bf16 *x, int64_t n_x, int cred, const __bf16 *wt, int
   return true;
 }
 
+// What a forward or input gradient with 16-byte aligned operands runs, and
+// the splits of its offset axis where the workspace holds their partial
+// sums. One rule for the launches, the workspace and rhip_conv_plan. can_pad:
+// whether padded copies are at hand (a workspace, and at most 128 offsets).
+struct ConvPlan {
+  int how = RHIP_CONV_ROWS, splits = 1;
+};
+template <typename T>
+static ConvPlan conv_plan(int64_t n_x, int cred, int64_t n_rows, int ncols, int K, bool can_pad) {
+  const int credw = red_width(kIsF32<T> ? RHIP_F32 : RHIP_BF16, cred);
+  if (!os_shape<T>(cred, credw, ncols, K)) {
+    if (thin_runs(K, cred, n_x, sizeof(T), can_pad))
+      return {RHIP_CONV_THIN};
+    return {can_pad ? RHIP_CONV_PADDED : RHIP_CONV_ROWS};
+  }
+  if (conv_small_takes<T>(n_rows, n_x, cred, ncols, K))
+    return {RHIP_CONV_SMALL};
+  if (kIsF32<T> && conv_x3_takes(cred, ncols, K, n_x))
+    return {RHIP_CONV_PARTS, conv_x3_splits(n_rows, cred, ncols, K)};
+  const int splits = os_splits<T>(n_rows, cred, credw, ncols, K);
+  if (cred == credw && K <= kLdsMaxK && os_lds_width<T>(cred) && n_x >= 1 &&
+      n_x * cred * static_cast<int64_t>(sizeof(T)) <= kBufMaxBytes && !(kIsF32<T> && splits > 1))
+    return {RHIP_CONV_LDS, splits};
+  if (!kIsF32<T> && cred == credw && fr_nt(cred, ncols, K, n_x, n_rows) != 0)
+    return {RHIP_CONV_RESIDENT};
+  return {RHIP_CONV_TILED, splits};
+}
+
 // Weight slices reordered for a table whose row k multiplies slice
 // perm[k]: dst[k][r][c] = src[perm[k]][r][c] ([K][rows][cols], same layout).
 template <typename T>
@@ -3107,14 +3162,14 @@ __global__ __launch_bounds__(kThreads) void permute_w_kernel(const T *__restrict
 
 // y[order[j]] = sum_k x[nbr[k][j]] @ W'[wperm[k]] with W'[k][c][n] = wt[k][n][c]
 // (wperm NULL: the identity); x has n_x rows. partial: os_partial_floats(...)
-// floats, or null to run without a split. credw: row stride of wt (cred, or
+// floats, or fewer to run without a split. credw: row stride of wt (cred, or
 // the padded reduction of red_width). The LDS-indexed kernel reads slice
 // wperm[k] itself; for the other kernels the slices are first copied in
 // table order to wperm_buf (K * ncols * credw elements; required with wperm).
 template <typename T>
 static void run_os(const T *x, int64_t n_x, int cred, const T *wt, int credw, int ncols,
                    const float *bias, const int32_t *nbr, int64_t n_rows, int K,
-                   const int32_t *order, T *y, float *partial, hipStream_t s,
+                   const int32_t *order, T *y, const PartialBuf &part, hipStream_t s,
                    bool resident = true, const int32_t *wperm = nullptr,
                    T *wperm_buf = nullptr) {
   if (n_rows == 0)
@@ -3122,7 +3177,8 @@ static void run_os(const T *x, int64_t n_x, int cred, const T *wt, int credw, in
   // the LDS-indexed kernel first: it beats the resident-weight kernel on the
   // maps that took that one (config 5 step 6.01 -> 5.86 ms), and with an
   // offset-axis split it takes the small coarse maps as well
-  const int splits = partial ? os_splits<T>(n_rows, credw, ncols, K) : 1;
+  const int splits = part.fit(os_splits<T>(n_rows, cred, credw, ncols, K), n_rows, ncols);
+  float *partial = part.p;
   if (run_os_lds(x, n_x, cred, wt, wperm, credw, ncols, bias, nbr, n_rows, K, order, y, splits,
                  partial, s)) {
     RHIP_LAUNCH_CHECK();
@@ -3663,7 +3719,7 @@ static void run_dw_rows(const __bf16 *x, int64_t n_in, int cin, const __bf16 *gy
 struct ConvWs {
   void *wt = nullptr;
   size_t wt_bytes = 0;
-  float *os_partial = nullptr;
+  PartialBuf os_partial;
   float *bias_partial = nullptr;
   // padded layers: the padded widths, both sides' rows, the weights (or dW)
   // and the bias, and the flag of a value that is not finite
@@ -3700,8 +3756,8 @@ static ConvWs carve_conv_front(Carve &cv, int32_t K, int32_t cin, int32_t cout, 
     return std::max(os_partial_floats<float>(n, cred, ncols, K),
                     sp > 1 ? static_cast<size_t>(sp) * n * ncols : size_t(0));
   };
-  w.os_partial =
-      cv.take<float>(std::max<size_t>({1, osp(n_out, w.cp, w.np), osp(n_in, w.np, w.cp)}));
+  w.os_partial.floats = std::max<size_t>({1, osp(n_out, w.cp, w.np), osp(n_in, w.np, w.cp)});
+  w.os_partial.p = cv.take<float>(w.os_partial.floats);
   w.bias_partial = cv.take<float>(static_cast<size_t>(kBiasChunks) * cout);
   if (pad) {
     w.px = cv.take<char>(n_in * w.cp * es);
@@ -3724,7 +3780,7 @@ static ConvWs carve_conv(Carve &cv, int32_t K, int32_t cin, int32_t cout, int32_
 }
 
 // The forward in workspace w: the transposed weights at w.wt (w.wt_bytes: K *
-// cin * cout elements at least), the split partial sums at w.os_partial (null:
+// cin * cout elements at least), the split partial sums in w.os_partial (none:
 // no split) and the padded copies (w.px null: none).
 template <typename T>
 static void conv_forward_into(const T *x, int64_t n_in, int32_t cin, const T *weight, int32_t K,
@@ -3733,30 +3789,29 @@ static void conv_forward_into(const T *x, int64_t n_in, int32_t cin, const T *we
                               hipStream_t stream) {
   constexpr int32_t dtype = kIsF32<T> ? RHIP_F32 : RHIP_BF16;
   const int64_t per = static_cast<int64_t>(cin) * cout;
-  if (!os_shape_of(dtype, cin, cout, K)) {
-    if (thin_runs(K, cin, n_in, sizeof(T), w.px != nullptr)) {
-      conv_thin<T>(x, n_in, cin, weight, per, cout, 1, nullptr, cout, bias, nbr, n_out, K,
-                   out_order, y, stream);
-      return;
-    }
-    if (w.px != nullptr) { // on padded copies
-      T *px = static_cast<T *>(w.px), *pw = static_cast<T *>(w.pw);
-      const bool copy = w.cp != cin || !aligned16(x);
-      pad_features<T>(x, copy ? n_in : 0, cin, w.cp, px, w.bad, nullptr, stream);
-      pad_weights<T>(weight, K, cin, cout, w.cp, w.np, pw, bias, w.pbias, w.bad, stream);
-      T *out = w.np != cout ? static_cast<T *>(w.py) : y;
-      ConvWs inner = w;
-      inner.px = nullptr;
-      conv_forward_into<T>(copy ? px : x, n_in, w.cp, pw, K, w.np, bias ? w.pbias : nullptr, nbr,
-                           out_order, n_out, out, inner, stream);
-      finish_rows<T>(out, w.np, y,
-                     PadSum<T>{x, weight, cin, cout, cout, 1, nullptr, bias, nbr, out_order, n_out,
-                               K},
-                     w.bad, stream);
-      return;
-    }
+  const int how = conv_plan<T>(n_in, cin, n_out, cout, K, w.px != nullptr).how;
+  if (how == RHIP_CONV_THIN) {
+    conv_thin<T>(x, n_in, cin, weight, per, cout, 1, nullptr, cout, bias, nbr, n_out, K, out_order,
+                 y, stream);
+    return;
   }
-  if (conv_small_takes<T>(n_out, n_in, cin, cout, K) && aligned16(x)) {
+  if (how == RHIP_CONV_PADDED) {
+    T *px = static_cast<T *>(w.px), *pw = static_cast<T *>(w.pw);
+    const bool copy = w.cp != cin || !aligned16(x);
+    pad_features<T>(x, copy ? n_in : 0, cin, w.cp, px, w.bad, nullptr, stream);
+    pad_weights<T>(weight, K, cin, cout, w.cp, w.np, pw, bias, w.pbias, w.bad, stream);
+    T *out = w.np != cout ? static_cast<T *>(w.py) : y;
+    ConvWs inner = w;
+    inner.px = nullptr;
+    conv_forward_into<T>(copy ? px : x, n_in, w.cp, pw, K, w.np, bias ? w.pbias : nullptr, nbr,
+                         out_order, n_out, out, inner, stream);
+    finish_rows<T>(out, w.np, y,
+                   PadSum<T>{x, weight, cin, cout, cout, 1, nullptr, bias, nbr, out_order, n_out,
+                             K},
+                   w.bad, stream);
+    return;
+  }
+  if (how == RHIP_CONV_SMALL && aligned16(x)) {
     const T *wn = weight;
     if constexpr (!kIsF32<T>) { // the bf16 operands hold eight channels of a column
       T *wt = static_cast<T *>(w.wt);
@@ -3771,10 +3826,10 @@ static void conv_forward_into(const T *x, int64_t n_in, int32_t cin, const T *we
     return;
   }
   if constexpr (kIsF32<T>) {
-    if (conv_x3_takes(cin, cout, K, n_in) && aligned16(x) && aligned16(y) &&
+    if (how == RHIP_CONV_PARTS && aligned16(x) && aligned16(y) &&
         w.wt_bytes >= conv_x3_weight_bytes(K, cin, cout)) {
       conv_x3(x, n_in, cin, weight, cout, 1, nullptr, cout, bias, nbr, n_out, K, out_order, y,
-              w.wt, w.os_partial, stream);
+              w.wt, w.os_partial.p, w.os_partial.floats, stream);
       return;
     }
   }
@@ -3785,9 +3840,10 @@ static void conv_forward_into(const T *x, int64_t n_in, int32_t cin, const T *we
     // the LDS-indexed kernel reads W itself where it takes the shape
     // (unpadded reductions, unsplit 128-column tiles): no transposed copy
     if (n_out > 0 && credw == cin) {
-      const int splits = w.os_partial ? os_splits<T>(n_out, cin, cout, K) : 1;
+      const int splits =
+          w.os_partial.fit(os_splits<T>(n_out, cin, cin, cout, K), n_out, cout);
       if (run_os_lds(x, n_in, cin, weight, nullptr, cin, cout, bias, nbr, n_out, K, out_order, y,
-                     splits, w.os_partial, stream, true)) {
+                     splits, w.os_partial.p, stream, true)) {
         RHIP_LAUNCH_CHECK();
         return;
       }
@@ -3812,43 +3868,43 @@ static void conv_backward_input_into(const T *grad_y, int64_t n_out, int32_t cou
                                      const ConvWs *w, hipStream_t stream) {
   constexpr int32_t dtype = kIsF32<T> ? RHIP_F32 : RHIP_BF16;
   const int64_t per = static_cast<int64_t>(cin) * cout;
-  if (w != nullptr && !os_shape_of(dtype, cout, cin, K)) {
-    if (thin_runs(K, cout, n_out, sizeof(T), w->px != nullptr)) {
-      conv_thin<T>(grad_y, n_out, cout, weight, per, 1, cout, weight_perm, cin, nullptr, nbr_t,
-                   n_in, K, in_order, grad_x, stream);
-      return;
-    }
-    if (w->px != nullptr) { // on padded copies
-      T *py = static_cast<T *>(w->py), *pw = static_cast<T *>(w->pw);
-      const bool copy = w->np != cout || !aligned16(grad_y);
-      pad_features<T>(grad_y, copy ? n_out : 0, cout, w->np, py, w->bad, nullptr, stream);
-      pad_weights<T>(weight, K, cin, cout, w->cp, w->np, pw, nullptr, nullptr, w->bad, stream);
-      T *out = w->cp != cin ? static_cast<T *>(w->px) : grad_x;
-      ConvWs inner = *w;
-      inner.px = nullptr;
-      conv_backward_input_into<T>(copy ? py : grad_y, n_out, w->np, pw, K, w->cp, nbr_t,
-                                  weight_perm, in_order, n_in, out, &inner, stream);
-      finish_rows<T>(out, w->cp, grad_x,
-                     PadSum<T>{grad_y, weight, cout, cin, 1, cout, weight_perm, nullptr, nbr_t,
-                               in_order, n_in, K},
-                     w->bad, stream);
-      return;
-    }
+  const int how =
+      conv_plan<T>(n_out, cout, n_in, cin, K, w != nullptr && w->px != nullptr).how;
+  if (how == RHIP_CONV_THIN && w != nullptr) {
+    conv_thin<T>(grad_y, n_out, cout, weight, per, 1, cout, weight_perm, cin, nullptr, nbr_t, n_in,
+                 K, in_order, grad_x, stream);
+    return;
+  }
+  if (how == RHIP_CONV_PADDED) {
+    T *py = static_cast<T *>(w->py), *pw = static_cast<T *>(w->pw);
+    const bool copy = w->np != cout || !aligned16(grad_y);
+    pad_features<T>(grad_y, copy ? n_out : 0, cout, w->np, py, w->bad, nullptr, stream);
+    pad_weights<T>(weight, K, cin, cout, w->cp, w->np, pw, nullptr, nullptr, w->bad, stream);
+    T *out = w->cp != cin ? static_cast<T *>(w->px) : grad_x;
+    ConvWs inner = *w;
+    inner.px = nullptr;
+    conv_backward_input_into<T>(copy ? py : grad_y, n_out, w->np, pw, K, w->cp, nbr_t, weight_perm,
+                                in_order, n_in, out, &inner, stream);
+    finish_rows<T>(out, w->cp, grad_x,
+                   PadSum<T>{grad_y, weight, cout, cin, 1, cout, weight_perm, nullptr, nbr_t,
+                             in_order, n_in, K},
+                   w->bad, stream);
+    return;
   }
   const T *wk = weight;
   const int32_t *wperm = weight_perm;
   int credw = cout;
-  if (conv_small_takes<T>(n_in, n_out, cout, cin, K) && aligned16(grad_y) && aligned16(weight)) {
+  if (how == RHIP_CONV_SMALL && aligned16(grad_y) && aligned16(weight)) {
     conv_small<T>(grad_y, n_out, cout, weight, false, weight_perm, cin, nullptr, nbr_t, n_in, K,
                   in_order, grad_x, stream);
     return;
   }
   if (w != nullptr) {
     if constexpr (kIsF32<T>) {
-      if (conv_x3_takes(cout, cin, K, n_out) && aligned16(grad_y) && aligned16(grad_x) &&
+      if (how == RHIP_CONV_PARTS && aligned16(grad_y) && aligned16(grad_x) &&
           w->wt_bytes >= conv_x3_weight_bytes(K, cin, cout)) {
         conv_x3(grad_y, n_out, cout, weight, 1, cout, weight_perm, cin, nullptr, nbr_t, n_in, K,
-                in_order, grad_x, w->wt, w->os_partial, stream);
+                in_order, grad_x, w->wt, w->os_partial.p, w->os_partial.floats, stream);
         return;
       }
     }
@@ -3865,7 +3921,7 @@ static void conv_backward_input_into(const T *grad_y, int64_t n_out, int32_t cou
   }
   // dX rows gather dY rows; W[k] [cin][cout] is already [n = cin][c = cout].
   run_os<T>(grad_y, n_out, cout, wk, credw, cin, nullptr, nbr_t, n_in, K, in_order, grad_x,
-            w ? w->os_partial : nullptr, stream, true, wperm,
+            w ? w->os_partial : PartialBuf{}, stream, true, wperm,
             w ? static_cast<T *>(w->wt) : nullptr);
 }
 
@@ -3960,6 +4016,22 @@ extern "C" int rhip_conv_forward_workspace_bytes(int32_t K, int32_t cin, int32_t
     Carve cv(nullptr, 0);
     carve_conv_front(cv, K, cin, cout, dtype, n_in, n_out);
     *bytes = cv.used + 256;
+  });
+}
+
+extern "C" int rhip_conv_plan(int32_t dtype, int32_t K, int32_t cred, int32_t ncols, int64_t n_x,
+                              int64_t n_rows, int32_t *kernel, int32_t *splits) {
+  return guarded([&] {
+    check_dtype(dtype);
+    RHIP_CHECK_ARG(kernel != nullptr && splits != nullptr, "kernel or splits is null");
+    RHIP_CHECK_ARG(K >= 1 && cred >= 1 && ncols >= 1, "sizes must be positive");
+    RHIP_CHECK_ARG(n_x >= 0 && n_rows >= 0, "row counts must be >= 0");
+    const bool can_pad = pads(dtype, cred, ncols, K);
+    const ConvPlan p = dtype == RHIP_F32
+                           ? conv_plan<float>(n_x, cred, n_rows, ncols, K, can_pad)
+                           : conv_plan<__bf16>(n_x, cred, n_rows, ncols, K, can_pad);
+    *kernel = p.how;
+    *splits = p.splits;
   });
 }
 

@@ -433,7 +433,7 @@ int conv_x3_splits(int64_t n_rows, int cred, int ncols, int K) {
 void conv_x3(const float *x, int64_t n_x, int cred, const float *w, int wc, int wn,
              const int32_t *wperm, int ncols, const float *bias, const int32_t *nbr,
              int64_t n_rows, int K, const int32_t *order, float *y, void *wt, float *partial,
-             hipStream_t s) {
+             size_t partial_floats, hipStream_t s) {
   if (n_rows == 0)
     return;
   __bf16 *w3 = static_cast<__bf16 *>(wt);
@@ -442,7 +442,10 @@ void conv_x3(const float *x, int64_t n_x, int cred, const float *w, int wc, int 
                      dim3(kThreads), 0, s, w, wc, wn, cred, ncols, total, w3);
   RHIP_LAUNCH_CHECK();
   const Plain plain{x, w, wc, wn, wperm, nbr, n_rows, K, cred, ncols};
-  const int splits = partial ? conv_x3_splits(n_rows, cred, ncols, K) : 1;
+  int splits = conv_x3_splits(n_rows, cred, ncols, K);
+  if (partial == nullptr || partial_floats / (static_cast<size_t>(n_rows) * ncols) <
+                                static_cast<size_t>(splits))
+    splits = 1;
   const int nt = x3_nt(ncols);
   const dim3 grid(static_cast<unsigned>(xcd_grid(ceil_div(n_rows, kWaves * x3_rg(K) * 16))),
                   static_cast<unsigned>(ncols / nt), static_cast<unsigned>(splits));

@@ -19,11 +19,11 @@ int conv_x3_splits(int64_t n_rows, int cred, int ncols, int K);
 
 // y[order[j]][n] = sum_k x[nbr[k][j]] . w[perm(k)][.][n] (+ bias[n]), the
 // weight of channel c and column n at w[k * cred * ncols + c * wc + n * wn].
-// wt: conv_x3_weight_bytes; partial: splits * n_rows * ncols floats, null
+// wt: conv_x3_weight_bytes; partial: splits * n_rows * ncols floats, or fewer
 // for no split.
 void conv_x3(const float *x, int64_t n_x, int cred, const float *w, int wc, int wn,
              const int32_t *wperm, int ncols, const float *bias, const int32_t *nbr,
              int64_t n_rows, int K, const int32_t *order, float *y, void *wt, float *partial,
-             hipStream_t s);
+             size_t partial_floats, hipStream_t s);
 
 } // namespace rhip
