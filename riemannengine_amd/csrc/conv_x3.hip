@@ -13,11 +13,14 @@
 // MFMAs': 64->64 9.6e-8 / 7.9e-8 against 3.8e-7 / 2.7e-7, 256->256 3.7e-7 /
 // 3.0e-7 against 1.1e-6 / 7.5e-7.
 //
-// Below 2^-110 the later parts reach bf16's smallest values and hold fewer
-// bits: such an operand is off by up to 2^-134 itself. Where parts cannot
-// represent a value (infinities, NaN, magnitudes that
-// round to infinity in bf16) some part is not finite, and so is every output
-// it reaches. A wave that finds such an output adds its rows up again in
+// Both operands are split after a multiplication by 2^24, and the sums are
+// multiplied by 2^-48. The parts of a float are multiples of its last bit, at
+// least 2^-149, so scaled they are normal bf16 values, exact down to the
+// smallest fp32 (unscaled, the later parts of a value below 2^-110 were bf16
+// denormals that hold fewer bits: off by 9e-6 at 2^-118, 4e-2 at 2^-130).
+// Where parts cannot represent a value or a scaled sum leaves fp32's range
+// (infinities, NaN, operands of 2^103 and sums of 2^80 and more) some part or
+// sum is not finite, and so is every output it reaches. A wave that finds such an output adds its rows up again in
 // plain fp32, over the pairs that exist (the split form: in its reduction).
 #include <algorithm>
 #include <type_traits>
@@ -31,16 +34,18 @@ namespace {
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 constexpr int kMaxK = 128;
 
+constexpr float kScale = 0x1p24f, kUnscale = 0x1p-48f; // operands, sums
+
 struct Parts {
   v8bf hi, mid, lo;
 };
 
-// the three bf16 parts of eight floats
+// the three bf16 parts of eight floats times kScale
 __device__ __forceinline__ Parts split8(const v4f &a, const v4f &b) {
   Parts p;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    const float v = j < 4 ? a[j & 3] : b[j & 3];
+    const float v = (j < 4 ? a[j & 3] : b[j & 3]) * kScale;
     const __bf16 h = static_cast<__bf16>(v);
     const float r = v - static_cast<float>(h);
     const __bf16 m = static_cast<__bf16>(r);
@@ -51,7 +56,7 @@ __device__ __forceinline__ Parts split8(const v4f &a, const v4f &b) {
   return p;
 }
 
-// Weights in three parts: wt[k][part][n][c'], the 32 channels of a step in
+// Weights times kScale in three parts: wt[k][part][n][c'], the 32 channels of a step in
 // the order the gathered rows come in: place 8g + j holds channel 4g + j of
 // the step's first 16 for j < 4, else channel 4g + j - 4 of its second 16.
 __global__ __launch_bounds__(kThreads) void x3_weights_kernel(const float *__restrict__ w, int wc,
@@ -67,7 +72,7 @@ __global__ __launch_bounds__(kThreads) void x3_weights_kernel(const float *__res
   const int n = rem / cred, cp = rem % cred;
   const int g = (cp & 31) >> 3, j = cp & 7;
   const int c = (cp & ~31) + 4 * g + (j < 4 ? j : 12 + j);
-  const float v = w[k * per + c * wc + n * wn];
+  const float v = w[k * per + c * wc + n * wn] * kScale;
   const __bf16 h = static_cast<__bf16>(v);
   const float r = v - static_cast<float>(h);
   const __bf16 m = static_cast<__bf16>(r);
@@ -308,7 +313,7 @@ conv_x3_kernel(const float *__restrict__ x, int64_t n_x, const __bf16 *__restric
   for (int r = 0; r < RG; ++r)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
-      acc[r][nb] += low[r][nb];
+      acc[r][nb] = (acc[r][nb] + low[r][nb]) * kUnscale;
 
   if constexpr (SPLIT) { // [split][position][column]
 #pragma unroll

@@ -78,3 +78,40 @@ def test_x3_keeps_values_that_are_not_finite(bad, where, n, span):
     assert (y[small] - ref[small]).norm() <= 1e-5 * scale
     big = m & ~small
     assert torch.allclose(y[big], ref[big], rtol=1e-5)
+
+
+def _device_sums(km, x, w, transpose=False):
+    """_sums on the device, in float64."""
+    rin, rout = (km.out_rows, km.in_rows) if transpose else (km.in_rows, km.out_rows)
+    y = torch.zeros(km.n_out, w.shape[1] if transpose else w.shape[2], dtype=torch.float64,
+                    device=DEV)
+    for k in range(w.shape[0]):
+        s = slice(int(km.offsets_host[k]), int(km.offsets_host[k + 1]))
+        wk = w[k].double()
+        y.index_add_(0, rout[s].long(),
+                     x[rin[s].long()].double() @ (wk.t().contiguous() if transpose else wk))
+    return y
+
+
+@pytest.mark.parametrize("n,cout", [(5000, 64), (14000, 256)])  # split, whole
+@pytest.mark.parametrize("ex,ew", [(-112, 0), (-118, 0), (-124, 12), (-130, 20), (-140, 24),
+                                   (0, -112), (10, -124), (20, -130), (-60, -50), (60, -100)])
+def test_x3_keeps_the_bits_of_small_operands(n, cout, ex, ew):
+    """Features, gradients and weights down to fp32's denormals (the inputs as
+    fp32 holds them) give sums as exact as ordinary ones."""
+    km = _map(n, oracle.region_offsets(3, 3), seed=n, span=18 if n > 9000 else 13)
+    kernel, splits = abi.conv_plan(torch.float32, 27, 64, cout, n, n)
+    assert kernel == "parts" and (splits > 1) == (n == 5000)
+    g = torch.Generator(DEV).manual_seed(ex * 7 + ew)
+    x, gy, w = (torch.randn(s, generator=g, device=DEV) for s in
+                ((n, 64), (n, cout), (27, 64, cout)))
+    x, gy, w = (torch.ldexp(t, torch.tensor(e, device=DEV)) for t, e in
+                ((x, ex), (gy, ex), (w, ew)))
+    assert all(bool((t != 0).float().mean() > 0.99) for t in (x, gy, w))
+    print(f"x3 small n={n} cout={cout} 2^{ex} 2^{ew}", flush=True)
+    for got, ref in ((abi.conv_forward(x, w, km), _device_sums(km, x, w)),
+                     (abi.conv_backward_input(gy, w, km), _device_sums(km, gy, w, True))):
+        assert float(ref.norm()) > 0
+        # fp32's smallest step where the sums are that small
+        step = 2.0 ** -149 * ref.numel() ** 0.5
+        assert float((got.double() - ref).norm()) <= 1e-6 * float(ref.norm()) + step
