@@ -20,8 +20,10 @@
 // denormals that hold fewer bits: off by 9e-6 at 2^-118, 4e-2 at 2^-130).
 // Where parts cannot represent a value or a scaled sum leaves fp32's range
 // (infinities, NaN, operands of 2^103 and sums of 2^80 and more) some part or
-// sum is not finite, and so is every output it reaches. A wave that finds such an output adds its rows up again in
-// plain fp32, over the pairs that exist (the split form: in its reduction).
+// sum is not finite, and so is every output it reaches. A wave that holds such
+// an output walks its stages once more on the fp32 matrix cores, each stage's
+// products added only to the rows that have the neighbour, and takes from that
+// the outputs that are not finite.
 #include <algorithm>
 #include <type_traits>
 
@@ -84,26 +86,13 @@ __global__ __launch_bounds__(kThreads) void x3_weights_kernel(const float *__res
 
 __device__ __forceinline__ bool finite(float v) { return v - v == 0.f; }
 
-// The plain fp32 sum of one output element over its pairs.
-struct Plain {
+// The call's operands as they came (conv_x3).
+struct Operands {
   const float *x, *w;
   int wc, wn;
   const int32_t *wperm, *nbr;
   int64_t n_rows;
   int K, cred, ncols;
-  __device__ float operator()(int64_t pos, int col) const {
-    float sum = 0.f;
-    for (int k = 0; k < K; ++k) {
-      const int32_t id = nbr[k * n_rows + pos];
-      if (id < 0)
-        continue;
-      const float *xr = x + static_cast<int64_t>(id) * cred;
-      const float *wr = w + static_cast<int64_t>(wperm ? wperm[k] : k) * cred * ncols + col * wn;
-      for (int c = 0; c < cred; ++c)
-        sum += xr[c] * wr[static_cast<int64_t>(c) * wc];
-    }
-    return sum;
-  }
 };
 
 // As conv_os_lds_kernel (indices of a wave's row groups in LDS, offsets
@@ -117,7 +106,7 @@ struct Plain {
 template <int NT, int RG, int WAVES, int CW, int KQ, bool SPLIT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(WAVES))) void
 conv_x3_kernel(const float *__restrict__ x, int64_t n_x, const __bf16 *__restrict__ wt,
-               const Plain plain, const float *__restrict__ bias, const int32_t *__restrict__ nbr,
+               const Operands ops, const float *__restrict__ bias, const int32_t *__restrict__ nbr,
                int64_t n_rows, int K, const int32_t *__restrict__ order, float *__restrict__ y,
                float *__restrict__ partial) {
   constexpr int CCH = 32; // channels per stage: one MFMA step
@@ -131,14 +120,14 @@ conv_x3_kernel(const float *__restrict__ x, int64_t n_x, const __bf16 *__restric
   constexpr int MW = KQ / 8;
   static_assert(CW % CCH == 0 && CCH % 32 == 0 && KQ % 8 == 0, "whole chunks and steps");
   __shared__ __align__(16) __bf16 sB[3 * NT * LDW];
-  __shared__ int32_t sK[kWaves][RG][KQ][kWave];
+  __shared__ __align__(16) int32_t sK[kWaves][RG][KQ][kWave];
   __shared__ uint32_t smask[kWaves * RG][MW];
 
   const int lane = threadIdx.x & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int i16 = lane & 15;
   const int g = lane >> 4;
-  const int ncols = plain.ncols;
+  const int ncols = ops.ncols;
   const int64_t tile0 = xcd_tile(blockIdx.x) * ROWS;
   if (tile0 >= n_rows)
     return; // padding workgroup (uniform)
@@ -212,16 +201,24 @@ conv_x3_kernel(const float *__restrict__ x, int64_t n_x, const __bf16 *__restric
     }
   };
   int left = 0;
-  if constexpr (SPLIT) {
+  auto to_first = [&]() { // from all stages to this split's
+    if constexpr (SPLIT) {
+      left = 0;
 #pragma unroll
-    for (int mw = 0; mw < MW; ++mw)
-      left += __builtin_popcount(m[mw]) * NCH;
-    const int s_begin = static_cast<int>(static_cast<int64_t>(left) * blockIdx.z / gridDim.z);
-    const int s_end = static_cast<int>(static_cast<int64_t>(left) * (blockIdx.z + 1) / gridDim.z);
-    for (int i = 0; i < s_begin; ++i)
-      advance(lowest());
-    left = s_end - s_begin;
-  }
+      for (int mw = 0; mw < MW; ++mw)
+        left += __builtin_popcount(m[mw]) * NCH;
+      const int s_begin = static_cast<int>(static_cast<int64_t>(left) * blockIdx.z / gridDim.z);
+      const int s_end = static_cast<int>(static_cast<int64_t>(left) * (blockIdx.z + 1) / gridDim.z);
+      for (int i = 0; i < s_begin; ++i)
+        advance(lowest());
+      left = s_end - s_begin;
+    }
+  };
+  uint32_t all[MW];
+#pragma unroll
+  for (int mw = 0; mw < MW; ++mw)
+    all[mw] = m[mw];
+  to_first();
   auto more = [&]() {
     if constexpr (SPLIT)
       return left > 0;
@@ -244,7 +241,7 @@ conv_x3_kernel(const float *__restrict__ x, int64_t n_x, const __bf16 *__restric
                             static_cast<uint32_t>(ch * CCH * sizeof(float)) + lane_byte,
                         ~(id >> 31));
     }
-    const int kw = plain.wperm ? plain.wperm[k] : k;
+    const int kw = ops.wperm ? ops.wperm[k] : k;
     const __bf16 *wk = wt + (static_cast<int64_t>(kw) * 3 * ncols + col0) * CW + ch * CCH;
     uint4 wreg[NPT];
 #pragma unroll
@@ -315,6 +312,79 @@ conv_x3_kernel(const float *__restrict__ x, int64_t n_x, const __bf16 *__restric
     for (int nb = 0; nb < NB; ++nb)
       acc[r][nb] = (acc[r][nb] + low[r][nb]) * kUnscale;
 
+  float sum = 0.f; // NaN where an output is not finite (0 * v is NaN there)
+#pragma unroll
+  for (int r = 0; r < RG; ++r)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        sum += 0.f * acc[r][nb][e];
+  if (__any(!finite(sum))) { // uniform: those outputs from the operands in fp32
+    v4f again[RG][NB];
+#pragma unroll
+    for (int r = 0; r < RG; ++r)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+        again[r][nb] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int mw = 0; mw < MW; ++mw)
+      m[mw] = all[mw];
+    cc = 0;
+    to_first();
+    while (more()) {
+      const int k = lowest(), ch = cc;
+      advance(k);
+      if constexpr (SPLIT)
+        --left;
+      if (!((wmask[k >> 5] >> (k & 31)) & 1u)) // uniform
+        continue;
+      const int kw = ops.wperm ? ops.wperm[k] : k;
+      v4f b[NB][2]; // channels 16 sub + 4g .. 4g + 3 of the stage, column i16
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            b[nb][sub][e] = ops.w[static_cast<int64_t>(kw) * CW * ncols +
+                                  (ch * CCH + 16 * sub + 4 * g + e) * ops.wc +
+                                  (col0 + nb * 16 + i16) * ops.wn];
+#pragma unroll
+      for (int r = 0; r < RG; ++r) {
+        const int32_t *ids = &sK[wv][r][k >> 2][(k & 3) * 16];
+        const int32_t id = ids[i16];
+        const uint32_t off = pick_off(
+            static_cast<uint32_t>(id) * static_cast<uint32_t>(CW * sizeof(float)) +
+                static_cast<uint32_t>(ch * CCH * sizeof(float)) + static_cast<uint32_t>(16 * g),
+            ~(id >> 31));
+        const int4 has = *reinterpret_cast<const int4 *>(ids + 4 * g); // rows 4g .. 4g + 3
+        v4f a[2];
+#pragma unroll
+        for (int sub = 0; sub < 2; ++sub)
+          a[sub] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
+                                               rx, off + static_cast<uint32_t>(sub * 64), 0, 0));
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          v4f t = again[r][nb];
+          Mfma<float>::mma(a[0], b[nb][0], t);
+          Mfma<float>::mma(a[1], b[nb][1], t);
+          again[r][nb] = v4f{has.x >= 0 ? t[0] : again[r][nb][0],
+                             has.y >= 0 ? t[1] : again[r][nb][1],
+                             has.z >= 0 ? t[2] : again[r][nb][2],
+                             has.w >= 0 ? t[3] : again[r][nb][3]};
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < RG; ++r)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          acc[r][nb][e] = finite(acc[r][nb][e]) ? acc[r][nb][e] : again[r][nb][e];
+  }
+
   if constexpr (SPLIT) { // [split][position][column]
 #pragma unroll
     for (int r = 0; r < RG; ++r)
@@ -330,15 +400,6 @@ conv_x3_kernel(const float *__restrict__ x, int64_t n_x, const __bf16 *__restric
       }
     return;
   }
-  float sum = 0.f; // NaN or infinite where an output is (0 * v is NaN there)
-#pragma unroll
-  for (int r = 0; r < RG; ++r)
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        sum += 0.f * acc[r][nb][e];
-  const bool redo = __any(sum != 0.f || !finite(sum));
 #pragma unroll
   for (int r = 0; r < RG; ++r) {
 #pragma unroll
@@ -350,8 +411,6 @@ conv_x3_kernel(const float *__restrict__ x, int64_t n_x, const __bf16 *__restric
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
           float v = acc[r][nb][e];
-          if (redo)
-            v = plain(pos, col0 + nb * 16 + i16);
           if (bias)
             v += bias[col0 + nb * 16 + i16];
           __builtin_nontemporal_store(v, &dst[nb * 16]); // as conv_os_lds_kernel's
@@ -361,16 +420,14 @@ conv_x3_kernel(const float *__restrict__ x, int64_t n_x, const __bf16 *__restric
   }
 }
 
-// The split form's sums in split order, with the bias; a sum that is not
-// finite again in plain fp32.
+// The split form's sums in split order, with the bias.
 __global__ __launch_bounds__(kThreads) void x3_reduce_kernel(const float *__restrict__ partial,
-                                                             int splits, int64_t n_rows,
-                                                             const Plain plain,
+                                                             int splits, int64_t n_rows, int ncols,
                                                              const float *__restrict__ bias,
                                                              const int32_t *__restrict__ order,
                                                              float *__restrict__ y) {
   const int64_t t = blockIdx.x * static_cast<int64_t>(kThreads) + threadIdx.x;
-  const int ncols = plain.ncols, q = ncols / 4;
+  const int q = ncols / 4;
   const int64_t pos = t / q;
   if (pos >= n_rows)
     return;
@@ -379,10 +436,6 @@ __global__ __launch_bounds__(kThreads) void x3_reduce_kernel(const float *__rest
 #pragma unroll 4
   for (int z = 1; z < splits; ++z)
     a += *reinterpret_cast<const v4f *>(partial + (z * n_rows + pos) * ncols + c);
-  if (!finite(0.f * a[0] + 0.f * a[1] + 0.f * a[2] + 0.f * a[3]))
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      a[e] = plain(pos, c + e);
   if (bias)
     a += v4f{bias[c], bias[c + 1], bias[c + 2], bias[c + 3]};
   *reinterpret_cast<v4f *>(y + (order ? order[pos] : pos) * ncols + c) = a;
@@ -397,15 +450,15 @@ constexpr int x3_rg(int K) { return K <= 32 ? 2 : 1; }
 
 template <int NT, int CW, int KQ>
 void launch(dim3 grid, bool split, const float *x, int64_t n_x, const __bf16 *wt,
-            const Plain &plain, const float *bias, const int32_t *order, float *y, float *partial,
+            const Operands &ops, const float *bias, const int32_t *order, float *y, float *partial,
             hipStream_t s) {
   constexpr int RG = x3_rg(4 * KQ), W = RG == 2 ? 4 : 3;
   if (split)
     hipLaunchKernelGGL((conv_x3_kernel<NT, RG, W, CW, KQ, true>), grid, dim3(kThreads), 0, s, x,
-                       n_x, wt, plain, bias, plain.nbr, plain.n_rows, plain.K, order, y, partial);
+                       n_x, wt, ops, bias, ops.nbr, ops.n_rows, ops.K, order, y, partial);
   else
     hipLaunchKernelGGL((conv_x3_kernel<NT, RG, W, CW, KQ, false>), grid, dim3(kThreads), 0, s, x,
-                       n_x, wt, plain, bias, plain.nbr, plain.n_rows, plain.K, order, y, nullptr);
+                       n_x, wt, ops, bias, ops.nbr, ops.n_rows, ops.K, order, y, nullptr);
 }
 
 } // namespace
@@ -446,7 +499,7 @@ void conv_x3(const float *x, int64_t n_x, int cred, const float *w, int wc, int 
   hipLaunchKernelGGL(x3_weights_kernel, dim3(static_cast<unsigned>(ceil_div(total, kThreads))),
                      dim3(kThreads), 0, s, w, wc, wn, cred, ncols, total, w3);
   RHIP_LAUNCH_CHECK();
-  const Plain plain{x, w, wc, wn, wperm, nbr, n_rows, K, cred, ncols};
+  const Operands ops{x, w, wc, wn, wperm, nbr, n_rows, K, cred, ncols};
   int splits = conv_x3_splits(n_rows, cred, ncols, K);
   if (partial == nullptr || partial_floats / (static_cast<size_t>(n_rows) * ncols) <
                                 static_cast<size_t>(splits))
@@ -456,7 +509,7 @@ void conv_x3(const float *x, int64_t n_x, int cred, const float *w, int wc, int 
                   static_cast<unsigned>(ncols / nt), static_cast<unsigned>(splits));
   auto go = [&](auto ntc, auto cwc, auto kqc) {
     launch<decltype(ntc)::value, decltype(cwc)::value, decltype(kqc)::value>(
-        grid, splits > 1, x, n_x, w3, plain, bias, order, y, partial, s);
+        grid, splits > 1, x, n_x, w3, ops, bias, order, y, partial, s);
   };
   auto pick_k = [&](auto ntc, auto cwc) {
     K <= 32   ? go(ntc, cwc, std::integral_constant<int, 8>{})
@@ -478,7 +531,7 @@ void conv_x3(const float *x, int64_t n_x, int cred, const float *w, int wc, int 
   if (splits > 1) {
     hipLaunchKernelGGL(x3_reduce_kernel,
                        dim3(static_cast<unsigned>(ceil_div(n_rows * (ncols / 4), kThreads))),
-                       dim3(kThreads), 0, s, partial, splits, n_rows, plain, bias, order, y);
+                       dim3(kThreads), 0, s, partial, splits, n_rows, ncols, bias, order, y);
     RHIP_LAUNCH_CHECK();
   }
 }
