@@ -12,6 +12,11 @@
 // Every workgroup reads the weights of its rows' offsets itself (no copy is
 // staged for others), which the L2 serves; that traffic, n_rows / 16 times the
 // weights, is what limits the rows (conv_small_takes).
+//
+// A missing neighbour's row is zeros, which a weight that is not finite turns
+// into NaN. A wave whose sums hold a value that is not finite walks its stages
+// once more in the same order, each stage's products added only to the rows
+// that have the neighbour, and takes those sums from there.
 #include <algorithm>
 #include <type_traits>
 
@@ -82,6 +87,30 @@ __global__ __launch_bounds__(kThreads) void conv_small_kernel(
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb)
     acc[nb] = v4f{0.f, 0.f, 0.f, 0.f};
+  auto load_a = [&](int k, int ch) {
+    const int32_t id = __builtin_amdgcn_ds_bpermute(((k & 3) * 16 + i16) * 4, v[k >> 2]);
+    const uint32_t off =
+        pick_off(static_cast<uint32_t>(id) * static_cast<uint32_t>(cred * sizeof(T)) +
+                     static_cast<uint32_t>((ch * CH + g * EPL) * sizeof(T)),
+                 ~(id >> 31));
+    return __builtin_bit_cast(Frag, __builtin_amdgcn_raw_buffer_load_b128(rx, off, 0, 0));
+  };
+  auto load_b = [&](int k, int ch, Frag (&b)[NB]) {
+    const int64_t kw = wperm ? wperm[k] : k;
+    const int c = ch * CH + g * EPL;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      const int n = col0 + nb * 16 + i16;
+      if constexpr (BY_CHANNEL) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          b[nb][e] = w[(kw * cred + c + e) * ncols + n];
+      } else {
+        b[nb] = *reinterpret_cast<const Frag *>(w + (kw * ncols + n) * cred + c);
+      }
+    }
+  };
+  const uint32_t all = m;
   advance(wv);
   while (m) {
     int kj[U], cj[U];
@@ -96,30 +125,11 @@ __global__ __launch_bounds__(kThreads) void conv_small_kernel(
     }
     Frag a[U], b[U][NB];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int32_t id = __builtin_amdgcn_ds_bpermute(((kj[u] & 3) * 16 + i16) * 4, v[kj[u] >> 2]);
-      const uint32_t off =
-          pick_off(static_cast<uint32_t>(id) * static_cast<uint32_t>(cred * sizeof(T)) +
-                       static_cast<uint32_t>((cj[u] * CH + g * EPL) * sizeof(T)),
-                   ~(id >> 31));
-      a[u] = __builtin_bit_cast(Frag, __builtin_amdgcn_raw_buffer_load_b128(rx, off, 0, 0));
-    }
+    for (int u = 0; u < U; ++u)
+      a[u] = load_a(kj[u], cj[u]);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t kw = wperm ? wperm[kj[u]] : kj[u];
-      const int c = cj[u] * CH + g * EPL;
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        const int n = col0 + nb * 16 + i16;
-        if constexpr (BY_CHANNEL) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            b[u][nb][e] = w[(kw * cred + c + e) * ncols + n];
-        } else {
-          b[u][nb] = *reinterpret_cast<const Frag *>(w + (kw * ncols + n) * cred + c);
-        }
-      }
-    }
+    for (int u = 0; u < U; ++u)
+      load_b(kj[u], cj[u], b[u]);
 #pragma unroll
     for (int u = 0; u < U; ++u)
       if (live[u]) { // uniform
@@ -127,6 +137,43 @@ __global__ __launch_bounds__(kThreads) void conv_small_kernel(
         for (int nb = 0; nb < NB; ++nb)
           M::mma(a[u], b[u][nb], acc[nb]);
       }
+  }
+  float check = 0.f; // NaN where a sum is not finite
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      check += 0.f * acc[nb][e];
+  if (__any(!(check == 0.f))) { // uniform
+    v4f again[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+      again[nb] = v4f{0.f, 0.f, 0.f, 0.f};
+    m = all;
+    cc = 0;
+    for (advance(wv); m; advance(kWaves)) {
+      const int k = __builtin_ctz(m);
+      const Frag a = load_a(k, cc);
+      Frag b[NB];
+      load_b(k, cc, b);
+      bool has[4]; // rows 4g .. 4g + 3
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        has[e] = __builtin_amdgcn_ds_bpermute(((k & 3) * 16 + 4 * g + e) * 4, v[k >> 2]) >= 0;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        v4f t = again[nb];
+        M::mma(a, b[nb], t);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          again[nb][e] = has[e] ? t[e] : again[nb][e];
+      }
+    }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        acc[nb][e] = acc[nb][e] - acc[nb][e] == 0.f ? acc[nb][e] : again[nb][e];
   }
   // D[4g + e][i16] of block nb
 #pragma unroll
@@ -145,22 +192,6 @@ __global__ __launch_bounds__(kThreads) void conv_small_kernel(
 #pragma unroll
       for (int q = 1; q < kWaves; ++q)
         sum += sR[q][r * LDR + c];
-      if (!(sum - sum == 0.f)) {
-        // not finite: over the pairs that exist only (a missing neighbour's
-        // zeros times a weight that is not finite would be NaN)
-        sum = 0.f;
-        for (int k = 0; k < K; ++k) {
-          const int32_t id = nbr[k * n_rows + pos];
-          if (id < 0)
-            continue;
-          const T *xr = x + static_cast<int64_t>(id) * cred;
-          const T *wr = w + static_cast<int64_t>(wperm ? wperm[k] : k) * cred * ncols;
-          for (int j = 0; j < cred; ++j)
-            sum += to_f32(xr[j]) *
-                   to_f32(BY_CHANNEL ? wr[static_cast<int64_t>(j) * ncols + col0 + c]
-                                     : wr[static_cast<int64_t>(col0 + c) * cred + j]);
-        }
-      }
       if (bias)
         sum += bias[col0 + c];
       y[(order ? order[pos] : pos) * ncols + col0 + c] = from_f32<T>(sum);

@@ -1,6 +1,6 @@
 """A value that is not finite changes the outputs it reaches, in every kernel
-that adds such outputs up a second time: fp32 operands in bf16 parts
-(whole and split). An infinity
+that adds such outputs up a second time: the small-map kernel and fp32 operands
+in bf16 parts (whole and split). An infinity
 times ordinary values is not finite, so the outputs to change are exactly
 those with a pair on it. Of the others, those in the column of a weight or
 gradient that is not finite may be sums in another order (their rows' missing
@@ -36,6 +36,8 @@ def _same_but(clean, got, hit, column=None):
 
 
 @pytest.mark.parametrize("n,span,cin,cout,dtype,kernel", [
+    (300, 5, 64, 64, torch.float32, "small"), (77, 4, 32, 48, torch.float32, "small"),
+    (300, 5, 64, 64, torch.bfloat16, "small"), (100, 4, 96, 32, torch.bfloat16, "small"),
     (6000, 12, 64, 64, torch.float32, "parts split"),
     (5000, 11, 96, 192, torch.float32, "parts split"),
     (15001, 15, 256, 256, torch.float32, "parts"), (58000, 24, 64, 64, torch.float32, "parts")])
