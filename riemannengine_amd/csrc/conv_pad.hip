@@ -9,7 +9,11 @@
 // The tiled kernels multiply a missing neighbour's zeros, which a weight (or,
 // in dW, a gradient) that is not finite turns into NaN. The copies see every
 // such value and set a flag on the device; the finishing kernels then add the
-// outputs up again over the pairs that exist, from the unpadded operands.
+// outputs that are not finite up again over the pairs that exist, from the
+// unpadded operands: one lane per output, and in dW, where a sum runs over all
+// rows, one wave per 16 x 16 tile on the fp32 matrix cores. With one infinite
+// gradient, or all NaN, dW of 64->20 bf16 on 200k rows takes 5.6 ms (one lane
+// per element 71, a wave per element 12 and 198).
 #include "conv_pad.hpp"
 
 namespace rhip {
@@ -81,6 +85,12 @@ __global__ __launch_bounds__(kThreads) void finish_rows_kernel(const T *yp, int 
       y[t] = yp[pos * np + col];
     return;
   }
+  const int64_t row = sum.order ? sum.order[pos] : pos;
+  const T v = yp[row * np + col];
+  if (finite(v)) {
+    y[row * sum.ncols + col] = v;
+    return;
+  }
   float acc = 0.f;
   for (int k = 0; k < sum.K; ++k) {
     const int32_t id = sum.nbr[k * sum.n_rows + pos];
@@ -94,34 +104,66 @@ __global__ __launch_bounds__(kThreads) void finish_rows_kernel(const T *yp, int 
   }
   if (sum.bias)
     acc += sum.bias[col];
-  y[(sum.order ? sum.order[pos] : pos) * sum.ncols + col] = from_f32<T>(acc);
+  y[row * sum.ncols + col] = from_f32<T>(acc);
 }
 
+// A wave owns 16 x 16 elements of one offset's dW, a lane four of a column.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void finish_weights_kernel(
     const T *__restrict__ dwp, int cp, int np, const T *__restrict__ x, int cin,
     const T *__restrict__ gy, int cout, const int32_t *__restrict__ nbr,
     const int32_t *__restrict__ order, int64_t n_out, int K, T *__restrict__ dw,
     const int *__restrict__ bad) {
-  const int64_t t = blockIdx.x * static_cast<int64_t>(kThreads) + threadIdx.x;
-  if (t >= static_cast<int64_t>(K) * cin * cout)
-    return;
-  const int64_t row = t / cout;
-  const int co = static_cast<int>(t - row * cout);
-  const int64_t k = row / cin;
-  const int ci = static_cast<int>(row - k * cin);
-  if (*bad == 0) {
-    dw[t] = dwp[(k * cp + ci) * np + co];
-    return;
+  const int lane = threadIdx.x & (kWave - 1), i16 = lane & 15, g = lane >> 4;
+  const int ct = (cin + 15) / 16, ot = (cout + 15) / 16;
+  const int64_t tile = blockIdx.x * static_cast<int64_t>(kWaves) + threadIdx.x / kWave;
+  const int64_t k = tile / (ct * ot);
+  if (k >= K)
+    return; // the whole wave
+  const int rem = static_cast<int>(tile - k * (ct * ot));
+  const int ci0 = rem / ot * 16, co = rem % ot * 16 + i16;
+  const bool col = co < cout;
+  T v[4];
+  bool ok = true;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int ci = ci0 + 4 * g + e;
+    v[e] = col && ci < cin ? dwp[(k * cp + ci) * np + co] : from_f32<T>(0.f);
+    ok = ok && finite(v[e]);
   }
-  float acc = 0.f;
-  for (int64_t p = 0; p < n_out; ++p) {
-    const int32_t id = nbr[k * n_out + p];
-    if (id >= 0)
-      acc += to_f32(x[static_cast<int64_t>(id) * cin + ci]) *
-             to_f32(gy[(order ? order[p] : p) * cout + co]);
+  if (*bad != 0 && __any(!ok)) { // uniform
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
+    const bool row = ci0 + i16 < cin;
+    for (int64_t p0 = 0; p0 < n_out; p0 += kWave) {
+      const int64_t p = p0 + lane;
+      const int32_t id = p < n_out ? nbr[k * n_out + p] : -1;
+      if (!__any(id >= 0)) // uniform; past here row 0 exists
+        continue;
+      const int32_t o = id < 0 ? 0 : (order ? order[p] : static_cast<int32_t>(p));
+      T a[16], b[16];
+      uint32_t has = 0;
+#pragma unroll
+      for (int s = 0; s < 16; ++s) { // positions 4s + g, at clamped places: all in flight
+        const int32_t is = __shfl(id, 4 * s + g), os = __shfl(o, 4 * s + g);
+        has |= (is >= 0 ? 1u : 0u) << s;
+        a[s] = x[static_cast<int64_t>(max(is, 0)) * cin + min(ci0 + i16, cin - 1)];
+        b[s] = gy[static_cast<int64_t>(os) * cout + min(co, cout - 1)];
+      }
+#pragma unroll
+      for (int s = 0; s < 16; ++s) { // zeros on both sides where there is no pair
+        const bool pair = (has >> s) & 1u;
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(pair && row ? to_f32(a[s]) : 0.f,
+                                                   pair && col ? to_f32(b[s]) : 0.f, acc, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      v[e] = finite(v[e]) ? v[e] : from_f32<T>(acc[e]);
   }
-  dw[t] = from_f32<T>(acc);
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (col && ci0 + 4 * g + e < cin)
+      dw[(k * cin + ci0 + 4 * g + e) * cout + co] = v[e];
 }
 
 dim3 blocks_of(int64_t threads) {
@@ -157,8 +199,9 @@ template <typename T>
 void finish_weights(const T *dwp, int cp, int np, const T *x, int cin, const T *gy, int cout,
                     const int32_t *nbr, const int32_t *order, int64_t n_out, int K, T *dw,
                     const int *bad, hipStream_t s) {
-  hipLaunchKernelGGL((finish_weights_kernel<T>), blocks_of(static_cast<int64_t>(K) * cin * cout),
-                     dim3(kThreads), 0, s, dwp, cp, np, x, cin, gy, cout, nbr, order, n_out, K, dw,
+  hipLaunchKernelGGL((finish_weights_kernel<T>),
+                     blocks_of(K * ceil_div(cin, 16) * ceil_div(cout, 16) * kWave), dim3(kThreads),
+                     0, s, dwp, cp, np, x, cin, gy, cout, nbr, order, n_out, K, dw,
                      bad);
   RHIP_LAUNCH_CHECK();
 }

@@ -15,7 +15,7 @@ inline int pad_width(int c) {
   return static_cast<int>(ceil_div(c, 64)) * 64;
 }
 
-// What the finishing kernels need to add outputs up again from the unpadded
+// What the finishing kernels need to add an output up again from the unpadded
 // operands: y[p][n] = sum_k sum_c x[nbr[k][p]][c] w[perm(k)][c * wc + n * wn]
 // (+ bias[n]), w slices of C * ncols elements.
 template <typename T> struct PadSum {
@@ -42,12 +42,13 @@ void pad_weights(const T *w, int K, int cin, int cout, int cp, int np, T *dst, c
                  float *bias_dst, int *bad, hipStream_t s);
 
 // y[r][0 .. ncols) = yp[r][0 .. ncols) of rows of np (yp == y with np ==
-// ncols: nothing to move), or where *bad the sums of `sum`.
+// ncols: nothing to move); where *bad, values that are not finite are the sums
+// of `sum`.
 template <typename T>
 void finish_rows(const T *yp, int np, T *y, const PadSum<T> &sum, const int *bad, hipStream_t s);
 
-// dw [K][cin][cout] from dwp [K][cp][np], or where *bad the sums over the
-// pairs of x[nbr[k][p]][ci] * gy[order[p]][co].
+// dw [K][cin][cout] from dwp [K][cp][np]; where *bad, values that are not
+// finite are the sums over the pairs of x[nbr[k][p]][ci] * gy[order[p]][co].
 template <typename T>
 void finish_weights(const T *dwp, int cp, int np, const T *x, int cin, const T *gy, int cout,
                     const int32_t *nbr, const int32_t *order, int64_t n_out, int K, T *dw,

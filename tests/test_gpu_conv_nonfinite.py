@@ -1,6 +1,6 @@
 """A value that is not finite changes the outputs it reaches, in every kernel
-that adds such outputs up a second time: the small-map kernel and fp32 operands
-in bf16 parts (whole and split). An infinity
+that adds such outputs up a second time: the small-map kernel, fp32 operands
+in bf16 parts (whole and split), and layers on padded copies. An infinity
 times ordinary values is not finite, so the outputs to change are exactly
 those with a pair on it. Of the others, those in the column of a weight or
 gradient that is not finite may be sums in another order (their rows' missing
@@ -40,7 +40,9 @@ def _same_but(clean, got, hit, column=None):
     (300, 5, 64, 64, torch.bfloat16, "small"), (100, 4, 96, 32, torch.bfloat16, "small"),
     (6000, 12, 64, 64, torch.float32, "parts split"),
     (5000, 11, 96, 192, torch.float32, "parts split"),
-    (15001, 15, 256, 256, torch.float32, "parts"), (58000, 24, 64, 64, torch.float32, "parts")])
+    (15001, 15, 256, 256, torch.float32, "parts"), (58000, 24, 64, 64, torch.float32, "parts"),
+    (300, 5, 24, 40, torch.float32, "padded"), (300, 5, 24, 64, torch.bfloat16, "padded"),
+    (400, 5, 64, 20, torch.bfloat16, "padded"), (6000, 12, 40, 40, torch.float32, "padded")])
 def test_other_outputs_keep_their_bits(n, span, cin, cout, dtype, kernel):
     km = _map(n, span)
     for cred, ncols in ((cin, cout), (cout, cin)):
@@ -67,3 +69,10 @@ def test_other_outputs_keep_their_bits(n, span, cin, cout, dtype, kernel):
     _same_but(y, abi.conv_forward(xb, w, km), hits(n, cout, orr[ir == n // 2], slice(None)))
     _same_but(gx, abi.conv_backward_input(gb, w, km),
               hits(n, cin, ir[orr == n // 3], slice(None)))
+    if kernel == "padded":  # dW on padded copies: the offsets that pair the row, its column
+        gw = abi.conv_weight_grad(x, gy, km, 27)
+        ks = torch.repeat_interleave(torch.arange(27, device=DEV),
+                                     torch.as_tensor(np.diff(km.offsets_host)).to(DEV))
+        hit = torch.zeros(27, cin, cout, dtype=torch.bool, device=DEV)
+        hit[ks[orr == n // 3].unique(), :, 5] = True
+        _same_but(gw, abi.conv_weight_grad(x, gb, km, 27), hit, 5)
