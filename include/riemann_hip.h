@@ -280,11 +280,21 @@ int rhip_conv_workspace_bytes(int32_t K, int32_t cin, int32_t cout,
                               int64_t n_pairs, size_t *bytes);
 
 /* Workspace of one layer's forward, input-gradient and bias-gradient calls
- * alone (no weight gradient): the front part of the rhip_conv_workspace_bytes
- * layout. */
+ * alone (no weight gradient). */
 int rhip_conv_forward_workspace_bytes(int32_t K, int32_t cin, int32_t cout,
                                       int32_t dtype, int64_t n_in, int64_t n_out,
                                       size_t *bytes);
+
+/* Workspace of the given passes alone (RHIP_PASS_ bits, one call at a time):
+ * what each uses on the kernel that the layer's shape selects. n_pairs
+ * matters to the weight gradient only. */
+#define RHIP_PASS_FORWARD 1
+#define RHIP_PASS_INPUT_GRAD 2
+#define RHIP_PASS_BIAS_GRAD 4
+#define RHIP_PASS_WEIGHT_GRAD 8
+int rhip_conv_pass_workspace_bytes(int32_t passes, int32_t K, int32_t cin, int32_t cout,
+                                   int32_t dtype, int64_t n_in, int64_t n_out,
+                                   int64_t n_pairs, size_t *bytes);
 
 /* The kernels of rhip_conv_forward and rhip_conv_backward_input. */
 typedef enum rhip_conv_kernel {

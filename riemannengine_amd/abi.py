@@ -36,8 +36,8 @@ EXPORTS = (
     "rhip_kmap_pairs_workspace_bytes", "rhip_kmap_pairs", "rhip_stencil_partners",
     "rhip_conv_backward_weight_ragged", "rhip_conv_backward_weight_ragged_supported",
     "rhip_conv_backward_weight_rows_supported",
-    "rhip_conv_workspace_bytes", "rhip_conv_forward_workspace_bytes", "rhip_conv_plan",
-    "rhip_conv_forward",
+    "rhip_conv_workspace_bytes", "rhip_conv_forward_workspace_bytes",
+    "rhip_conv_pass_workspace_bytes", "rhip_conv_plan", "rhip_conv_forward",
     "rhip_conv_forward_noalloc", "rhip_conv_bias_grad",
     "rhip_conv_backward_input", "rhip_conv_backward_weight", "rhip_conv_backward_weight_rows",
     "rhip_stride_map_workspace_bytes", "rhip_stride_map_count", "rhip_group_map_count",
@@ -91,6 +91,8 @@ def _declare(lib):
                                           _vp, _vp, _vp, _vp, _vp, _vp]),
         "rhip_conv_workspace_bytes": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i64, _i64, _i64,
                                                      _P(_sz)]),
+        "rhip_conv_pass_workspace_bytes": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i32, _i64,
+                                                          _i64, _i64, _P(_sz)]),
         "rhip_conv_plan": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i64, _i64, _P(_i32),
                                           _P(_i32)]),
         "rhip_conv_forward": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i32, _i32, _vp, _vp,
@@ -476,6 +478,15 @@ def kernel_map(in_table: CoordTable, out_table: CoordTable, offsets) -> KernelMa
 
 # ------------------------------------------------------------ convolution
 
+PASS_FORWARD, PASS_INPUT_GRAD, PASS_BIAS_GRAD, PASS_WEIGHT_GRAD = 1, 2, 4, 8  # rhip_conv passes
+
+
+def _pass_ws(passes, K, cin, cout, dtype, dev, n_in, n_out, n_pairs=0) -> torch.Tensor:
+    """Workspace of the given passes of a layer."""
+    return torch.empty(_sizeq(lib().rhip_conv_pass_workspace_bytes, passes, K, cin, cout, dtype,
+                              n_in, n_out, n_pairs), dtype=torch.uint8, device=dev)
+
+
 def _conv_ws(K, cin, cout, dtype, dev, kmap: "KernelMap") -> torch.Tensor:
     return torch.empty(_sizeq(lib().rhip_conv_workspace_bytes, K, cin, cout, dtype, kmap.n_in,
                               kmap.n_out, kmap.n_pairs), dtype=torch.uint8, device=dev)
@@ -506,9 +517,7 @@ def conv_bias_grad(grad_y: torch.Tensor) -> torch.Tensor:
     grad_y = grad_y.contiguous()
     n, C = grad_y.shape
     gb = torch.empty(C, dtype=torch.float32, device=grad_y.device)
-    ws = torch.empty(_sizeq(lib().rhip_conv_forward_workspace_bytes, 1, 1, C,
-                            _dtype_code(grad_y.dtype), 0, n), dtype=torch.uint8,
-                     device=grad_y.device)
+    ws = _pass_ws(PASS_BIAS_GRAD, 1, 1, C, _dtype_code(grad_y.dtype), grad_y.device, 0, n)
     _check(lib().rhip_conv_bias_grad(_ptr(grad_y), n, C, _dtype_code(grad_y.dtype), _ptr(gb),
                                      _ptr(ws), ws.numel(), _stream(grad_y.device)),
            "rhip_conv_bias_grad")
@@ -527,7 +536,7 @@ def conv_forward(x: torch.Tensor, weight: torch.Tensor, kmap: KernelMap,
         raise RuntimeError("shape mismatch between features, weight and kernel map")
     b = None if bias is None else bias.reshape(-1).to(torch.float32).contiguous()
     y = torch.empty((kmap.n_out, cout), dtype=x.dtype, device=x.device)
-    ws = _conv_fwd_ws(K, cin, cout, dt, x.device, kmap)
+    ws = _pass_ws(PASS_FORWARD, K, cin, cout, dt, x.device, kmap.n_in, kmap.n_out)
     _check(lib().rhip_conv_forward(_ptr(x), kmap.n_in, cin, _ptr(weight), K, cout, _ptr(b),
                                    _ptr(kmap.nbr), _ptr(kmap.out_order), kmap.n_out, _ptr(y),
                                    dt, _ptr(ws), ws.numel(), _stream(x.device)),
@@ -586,7 +595,7 @@ def conv_backward_input(grad_y: torch.Tensor, weight: torch.Tensor, kmap: Kernel
     weight = weight.to(grad_y.dtype).contiguous()
     K, cin, cout = weight.shape
     gx = torch.empty((kmap.n_in, cin), dtype=grad_y.dtype, device=grad_y.device)
-    ws = _conv_fwd_ws(K, cin, cout, dt, grad_y.device, kmap)
+    ws = _pass_ws(PASS_INPUT_GRAD, K, cin, cout, dt, grad_y.device, kmap.n_in, kmap.n_out)
     if kmap.symmetric:  # nbr with the stencil partners as weight permutation
         table, perm, order = kmap.nbr, kmap.partner, kmap.out_order
     else:
@@ -605,7 +614,8 @@ def conv_backward_weight(x: torch.Tensor, grad_y: torch.Tensor, kmap: KernelMap,
     x, grad_y = x.contiguous(), grad_y.to(x.dtype).contiguous()
     cin, cout = x.shape[1], grad_y.shape[1]
     gw = torch.empty((K, cin, cout), dtype=x.dtype, device=x.device)
-    ws = _conv_ws(K, cin, cout, dt, x.device, kmap)
+    ws = _pass_ws(PASS_WEIGHT_GRAD, K, cin, cout, dt, x.device, kmap.n_in, kmap.n_out,
+                  kmap.n_pairs)
     _check(lib().rhip_conv_backward_weight(_ptr(x), kmap.n_in, cin, _ptr(grad_y), kmap.n_out,
                                            cout, K, _ptr(kmap.offsets), kmap.n_pairs,
                                            _ptr(kmap.in_rows), _ptr(kmap.out_rows), _ptr(gw),
@@ -631,7 +641,8 @@ def conv_weight_grad(x: torch.Tensor, grad_y: torch.Tensor, kmap: KernelMap,
     x, grad_y = x.contiguous(), grad_y.to(x.dtype).contiguous()
     cin, cout = x.shape[1], grad_y.shape[1]
     gw = torch.empty((K, cin, cout), dtype=x.dtype, device=x.device)
-    ws = _conv_ws(K, cin, cout, dt, x.device, kmap)
+    ws = _pass_ws(PASS_WEIGHT_GRAD, K, cin, cout, dt, x.device, kmap.n_in, kmap.n_out,
+                  kmap.n_pairs)
     st = RHIP_ERR_UNSUPPORTED
     pair_list = x.dtype == torch.bfloat16 and K <= 8 and (
         kmap.n_pairs < 2 * kmap.n_out
@@ -665,7 +676,8 @@ def conv_backward_weight_rows(x: torch.Tensor, grad_y: torch.Tensor, kmap: Kerne
     x, grad_y = x.contiguous(), grad_y.to(x.dtype).contiguous()
     cin, cout = x.shape[1], grad_y.shape[1]
     gw = torch.empty((K, cin, cout), dtype=x.dtype, device=x.device)
-    ws = _conv_ws(K, cin, cout, dt, x.device, kmap)
+    ws = _pass_ws(PASS_WEIGHT_GRAD, K, cin, cout, dt, x.device, kmap.n_in, kmap.n_out,
+                  kmap.n_pairs)
     _check(lib().rhip_conv_backward_weight_rows(_ptr(x), kmap.n_in, cin, _ptr(grad_y),
                                                 kmap.n_out, cout, K, _ptr(kmap.nbr),
                                                 _ptr(kmap.out_order), _ptr(gw), dt, _ptr(ws),

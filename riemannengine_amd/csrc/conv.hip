@@ -2795,15 +2795,6 @@ static int os_splits(int64_t n_rows, int cred, int credw, int ncols, int K) {
       std::max<int64_t>(1, std::min<int64_t>({8, want, std::max<int64_t>(1, stages / 4)})));
 }
 
-// Floats of split partial sums run_os needs (0 without a split) for a
-// reduction of cred channels that it pads by itself.
-template <typename T>
-static size_t os_partial_floats(int64_t n_rows, int cred, int ncols, int K) {
-  const int credw = red_width(kIsF32<T> ? RHIP_F32 : RHIP_BF16, cred);
-  const int sp = os_splits<T>(n_rows, cred, credw, ncols, K);
-  return sp > 1 ? static_cast<size_t>(sp) * n_rows * ncols : 0;
-}
-
 // Partial sums of a split offset axis: `floats` of them at p (null: none).
 struct PartialBuf {
   float *p = nullptr;
@@ -3161,10 +3152,10 @@ __global__ __launch_bounds__(kThreads) void permute_w_kernel(const T *__restrict
 }
 
 // y[order[j]] = sum_k x[nbr[k][j]] @ W'[wperm[k]] with W'[k][c][n] = wt[k][n][c]
-// (wperm NULL: the identity); x has n_x rows. partial: os_partial_floats(...)
-// floats, or fewer to run without a split. credw: row stride of wt (cred, or
-// the padded reduction of red_width). The LDS-indexed kernel reads slice
-// wperm[k] itself; for the other kernels the slices are first copied in
+// (wperm NULL: the identity); x has n_x rows. part: os_splits times n_rows x
+// ncols floats, or fewer to run without a split. credw: row stride of wt
+// (cred, or the padded reduction of red_width). The LDS-indexed kernel reads
+// slice wperm[k] itself; for the other kernels the slices are first copied in
 // table order to wperm_buf (K * ncols * credw elements; required with wperm).
 template <typename T>
 static void run_os(const T *x, int64_t n_x, int cred, const T *wt, int credw, int ncols,
@@ -3709,74 +3700,121 @@ static void run_dw_rows(const __bf16 *x, int64_t n_in, int cin, const __bf16 *gy
   RHIP_LAUNCH_CHECK();
 }
 
-// One workspace serves the calls of a layer. Its front holds what the
-// forward, the input gradient and the bias gradient use: the transposed
-// weights, the split partial sums of the output-stationary kernel and the
-// bias gradient's chunk sums. Behind them, used by dW
-// only: the per-workgroup partial tiles (sized from the dW plans of this map)
-// and the fp32 accumulator of the any-shape kernel. A workspace of
-// rhip_conv_forward_workspace_bytes serves the forward and input gradient.
+// One workspace serves the calls of a layer, one call at a time: each carves
+// what it uses from the start, so a workspace is as large as the largest of
+// them. rhip_conv_forward_workspace_bytes is the forward, the input gradient
+// and the bias gradient, rhip_conv_workspace_bytes that and the weight
+// gradient, rhip_conv_pass_workspace_bytes any of them.
 struct ConvWs {
+  // a forward or input gradient: the transposed (or permuted, padded) weights,
+  // fp32 as three bf16 parts where conv_x3 takes the layer, and the split
+  // partial sums
   void *wt = nullptr;
   size_t wt_bytes = 0;
   PartialBuf os_partial;
-  float *bias_partial = nullptr;
   // padded layers: the padded widths, both sides' rows, the weights (or dW)
   // and the bias, and the flag of a value that is not finite
   int cp = 0, np = 0;
   void *px = nullptr, *py = nullptr, *pw = nullptr;
   float *pbias = nullptr;
   int *bad = nullptr;
+  // dW: the per-workgroup partial tiles and the fp32 accumulator of the
+  // any-shape kernel
   float *partial = nullptr;
   float *acc = nullptr;
 };
 
-static ConvWs carve_conv_front(Carve &cv, int32_t K, int32_t cin, int32_t cout, int32_t dtype,
-                               int64_t n_in, int64_t n_out) {
+static ConvPlan plan_of(int32_t dtype, int64_t n_x, int cred, int64_t n_rows, int ncols, int K,
+                        bool can_pad) {
+  return dtype == RHIP_F32 ? conv_plan<float>(n_x, cred, n_rows, ncols, K, can_pad)
+                           : conv_plan<__bf16>(n_x, cred, n_rows, ncols, K, can_pad);
+}
+
+// A forward (cin to cout) or an input gradient (cout to cin): what conv_plan's
+// kernel for it uses, and the copies only where that is the padded one.
+static ConvWs carve_conv_pass(Carve &cv, bool forward, int32_t K, int32_t cin, int32_t cout,
+                              int32_t dtype, int64_t n_in, int64_t n_out) {
   ConvWs w;
-  const bool f32 = dtype == RHIP_F32;
-  const size_t es = f32 ? 4 : 2;
-  // channel counts the tiled kernels see
-  const bool pad = pads(dtype, cin, cout, K);
-  w.cp = pad ? pad_width(cin) : cin;
-  w.np = pad ? pad_width(cout) : cout;
-  // transposed forward weights, or the padded copy of dX's (fp32: their three
-  // bf16 parts where conv_x3 takes the layer)
-  const size_t nw = static_cast<size_t>(K) *
-                    std::max(static_cast<size_t>(w.np) * red_width(dtype, w.cp),
-                             static_cast<size_t>(w.cp) * red_width(dtype, w.np));
-  w.wt_bytes = nw * es;
-  if (f32 && (conv_x3_takes(w.cp, w.np, K, n_in) || conv_x3_takes(w.np, w.cp, K, n_out)))
-    w.wt_bytes = std::max(w.wt_bytes, conv_x3_weight_bytes(K, w.cp, w.np));
-  w.wt = cv.take<char>(w.wt_bytes);
-  auto osp = [&](int64_t n, int cred, int ncols) {
-    if (!f32)
-      return os_partial_floats<__bf16>(n, cred, ncols, K);
-    const int sp = conv_x3_splits(n, cred, ncols, K);
-    return std::max(os_partial_floats<float>(n, cred, ncols, K),
-                    sp > 1 ? static_cast<size_t>(sp) * n * ncols : size_t(0));
-  };
-  w.os_partial.floats = std::max<size_t>({1, osp(n_out, w.cp, w.np), osp(n_in, w.np, w.cp)});
-  w.os_partial.p = cv.take<float>(w.os_partial.floats);
-  w.bias_partial = cv.take<float>(static_cast<size_t>(kBiasChunks) * cout);
-  if (pad) {
-    w.px = cv.take<char>(n_in * w.cp * es);
-    w.py = cv.take<char>(n_out * w.np * es);
+  const size_t es = dtype == RHIP_F32 ? 4 : 2;
+  int cred = forward ? cin : cout, ncols = forward ? cout : cin;
+  const int64_t n_x = forward ? n_in : n_out, n_rows = forward ? n_out : n_in;
+  ConvPlan plan = plan_of(dtype, n_x, cred, n_rows, ncols, K, pads(dtype, cin, cout, K));
+  if (plan.how == RHIP_CONV_THIN)
+    return w;
+  if (plan.how == RHIP_CONV_PADDED) {
+    w.cp = pad_width(cin);
+    w.np = pad_width(cout);
+    w.px = cv.take<char>(forward || w.cp != cin ? n_in * w.cp * es : 1);
+    w.py = cv.take<char>(!forward || w.np != cout ? n_out * w.np * es : 1);
     w.pw = cv.take<char>(static_cast<size_t>(K) * w.cp * w.np * es);
     w.pbias = cv.take<float>(w.np);
     w.bad = cv.take<int>(1);
+    cred = pad_width(cred);
+    ncols = pad_width(ncols);
+    plan = plan_of(dtype, n_x, cred, n_rows, ncols, K, false);
   }
+  w.wt_bytes = static_cast<size_t>(K) * ncols * red_width(dtype, cred) * es;
+  if (plan.how == RHIP_CONV_PARTS)
+    w.wt_bytes = std::max(w.wt_bytes, conv_x3_weight_bytes(K, cred, ncols));
+  w.wt = cv.take<char>(w.wt_bytes);
+  w.os_partial.floats = plan.splits > 1 ? static_cast<size_t>(plan.splits) * n_rows * ncols : 1;
+  w.os_partial.p = cv.take<float>(w.os_partial.floats);
   return w;
 }
 
-static ConvWs carve_conv(Carve &cv, int32_t K, int32_t cin, int32_t cout, int32_t dtype,
-                         int64_t n_in, int64_t n_out, const DwPlan &p) {
-  ConvWs w = carve_conv_front(cv, K, cin, cout, dtype, n_in, n_out);
+static ConvWs carve_conv_dw(Carve &cv, int32_t K, int32_t cin, int32_t cout, int32_t dtype,
+                            int64_t n_in, int64_t n_out, const DwPlan &p) {
+  ConvWs w;
+  const size_t es = dtype == RHIP_F32 ? 4 : 2;
+  if (dw_ragged(dtype, cin, cout, K, n_in, n_out) == Ragged::kPad) {
+    w.cp = pad_width(cin);
+    w.np = pad_width(cout);
+    w.px = cv.take<char>(n_in * w.cp * es);
+    w.py = cv.take<char>(n_out * w.np * es);
+    w.pw = cv.take<char>(static_cast<size_t>(K) * w.cp * w.np * es);
+    w.bad = cv.take<int>(1);
+  }
   w.partial = cv.take<float>(
       std::max<size_t>({1, p.partial_floats() * K, dw_table_floats(dtype, cin, cout, K, n_in, n_out),
                         dw_ragged_floats(dtype, cin, cout, K, n_in, n_out)}));
   w.acc = cv.take<float>(static_cast<size_t>(K) * cin * cout);
   return w;
+}
+
+// Chunk sums of the bias gradient.
+static float *carve_bias(Carve &cv, int32_t cout) {
+  return cv.take<float>(static_cast<size_t>(kBiasChunks) * cout);
+}
+
+// Bytes of the largest of the passes (RHIP_PASS_ bits).
+static size_t pass_bytes(int32_t passes, int32_t K, int32_t cin, int32_t cout, int32_t dtype,
+                         int64_t n_in, int64_t n_out, int64_t n_pairs) {
+  size_t most = 0;
+  auto size = [&](int32_t pass, auto &&carve) {
+    if (passes & pass) {
+      Carve cv(nullptr, 0);
+      carve(cv);
+      most = std::max(most, cv.used);
+    }
+  };
+  size(RHIP_PASS_FORWARD,
+       [&](Carve &cv) { carve_conv_pass(cv, true, K, cin, cout, dtype, n_in, n_out); });
+  size(RHIP_PASS_INPUT_GRAD,
+       [&](Carve &cv) { carve_conv_pass(cv, false, K, cin, cout, dtype, n_in, n_out); });
+  size(RHIP_PASS_BIAS_GRAD, [&](Carve &cv) { carve_bias(cv, cout); });
+  size(RHIP_PASS_WEIGHT_GRAD, [&](Carve &cv) {
+    carve_conv_dw(cv, K, cin, cout, dtype, n_in, n_out,
+                  dw_plan(dtype, cin, cout, K, n_pairs, n_in, n_out));
+  });
+  return most;
+}
+
+static void check_sizes(int32_t K, int32_t cin, int32_t cout, int32_t dtype, int64_t n_in,
+                        int64_t n_out, int64_t n_pairs, const size_t *bytes) {
+  RHIP_CHECK_ARG(bytes != nullptr, "bytes is null");
+  RHIP_CHECK_ARG(K >= 1 && cin >= 1 && cout >= 1, "sizes must be positive");
+  RHIP_CHECK_ARG(n_in >= 0 && n_out >= 0 && n_pairs >= 0, "counts must be >= 0");
+  check_dtype(dtype);
 }
 
 // The forward in workspace w: the transposed weights at w.wt (w.wt_bytes: K *
@@ -3994,14 +4032,10 @@ extern "C" int rhip_conv_workspace_bytes(int32_t K, int32_t cin, int32_t cout,
                                          int32_t dtype, int64_t n_in, int64_t n_out,
                                          int64_t n_pairs, size_t *bytes) {
   return guarded([&] {
-    RHIP_CHECK_ARG(bytes != nullptr, "bytes is null");
-    RHIP_CHECK_ARG(K >= 1 && cin >= 1 && cout >= 1, "sizes must be positive");
-    RHIP_CHECK_ARG(n_in >= 0 && n_out >= 0 && n_pairs >= 0, "counts must be >= 0");
-    check_dtype(dtype);
-    Carve cv(nullptr, 0);
-    carve_conv(cv, K, cin, cout, dtype, n_in, n_out,
-               dw_plan(dtype, cin, cout, K, n_pairs, n_in, n_out));
-    *bytes = cv.used + 256;
+    check_sizes(K, cin, cout, dtype, n_in, n_out, n_pairs, bytes);
+    auto of = [&](int32_t p) { return pass_bytes(p, K, cin, cout, dtype, n_in, n_out, n_pairs); };
+    *bytes = of(RHIP_PASS_FORWARD | RHIP_PASS_INPUT_GRAD) + of(RHIP_PASS_BIAS_GRAD) +
+             of(RHIP_PASS_WEIGHT_GRAD) + 256;
   });
 }
 
@@ -4009,13 +4043,19 @@ extern "C" int rhip_conv_forward_workspace_bytes(int32_t K, int32_t cin, int32_t
                                                  int32_t dtype, int64_t n_in, int64_t n_out,
                                                  size_t *bytes) {
   return guarded([&] {
-    RHIP_CHECK_ARG(bytes != nullptr, "bytes is null");
-    RHIP_CHECK_ARG(K >= 1 && cin >= 1 && cout >= 1, "sizes must be positive");
-    RHIP_CHECK_ARG(n_in >= 0 && n_out >= 0, "counts must be >= 0");
-    check_dtype(dtype);
-    Carve cv(nullptr, 0);
-    carve_conv_front(cv, K, cin, cout, dtype, n_in, n_out);
-    *bytes = cv.used + 256;
+    check_sizes(K, cin, cout, dtype, n_in, n_out, 0, bytes);
+    auto of = [&](int32_t p) { return pass_bytes(p, K, cin, cout, dtype, n_in, n_out, 0); };
+    *bytes = of(RHIP_PASS_FORWARD | RHIP_PASS_INPUT_GRAD) + of(RHIP_PASS_BIAS_GRAD) + 256;
+  });
+}
+
+extern "C" int rhip_conv_pass_workspace_bytes(int32_t passes, int32_t K, int32_t cin, int32_t cout,
+                                              int32_t dtype, int64_t n_in, int64_t n_out,
+                                              int64_t n_pairs, size_t *bytes) {
+  return guarded([&] {
+    check_sizes(K, cin, cout, dtype, n_in, n_out, n_pairs, bytes);
+    RHIP_CHECK_ARG(passes >= 1 && passes < 2 * RHIP_PASS_WEIGHT_GRAD, "unknown passes");
+    *bytes = pass_bytes(passes, K, cin, cout, dtype, n_in, n_out, n_pairs) + 256;
   });
 }
 
@@ -4027,9 +4067,7 @@ extern "C" int rhip_conv_plan(int32_t dtype, int32_t K, int32_t cred, int32_t nc
     RHIP_CHECK_ARG(K >= 1 && cred >= 1 && ncols >= 1, "sizes must be positive");
     RHIP_CHECK_ARG(n_x >= 0 && n_rows >= 0, "row counts must be >= 0");
     const bool can_pad = pads(dtype, cred, ncols, K);
-    const ConvPlan p = dtype == RHIP_F32
-                           ? conv_plan<float>(n_x, cred, n_rows, ncols, K, can_pad)
-                           : conv_plan<__bf16>(n_x, cred, n_rows, ncols, K, can_pad);
+    const ConvPlan p = plan_of(dtype, n_x, cred, n_rows, ncols, K, can_pad);
     *kernel = p.how;
     *splits = p.splits;
   });
@@ -4050,10 +4088,8 @@ extern "C" int rhip_conv_forward(const void *x, int64_t n_in, int32_t cin,
     RHIP_CHECK_ARG(y && weight && nbr, "y, weight and nbr are required");
     RHIP_CHECK_ARG(n_in == 0 || x != nullptr, "x is null");
     RHIP_CHECK_ARG(workspace != nullptr, "workspace is null");
-    // the workspace was sized for this layer's map (n_in, n_out); the dW
-    // plan does not change the forward's pieces
     Carve cv(workspace, workspace_bytes);
-    const ConvWs w = carve_conv_front(cv, K, cin, cout, dtype, n_in, n_out);
+    const ConvWs w = carve_conv_pass(cv, true, K, cin, cout, dtype, n_in, n_out);
     if (dtype == RHIP_F32)
       conv_forward_into<float>(static_cast<const float *>(x), n_in, cin,
                                static_cast<const float *>(weight), K, cout, bias, nbr, out_order,
@@ -4112,10 +4148,8 @@ extern "C" int rhip_conv_bias_grad(const void *grad_y, int64_t n_out, int32_t co
     RHIP_CHECK_ARG(grad_bias != nullptr, "grad_bias is null");
     RHIP_CHECK_ARG(n_out == 0 || grad_y != nullptr, "grad_y is null");
     RHIP_CHECK_ARG(workspace != nullptr, "workspace is null");
-    // the chunk sums go to the front of the layer workspace, whose forward
-    // part reserves room for them
     Carve cv(workspace, workspace_bytes);
-    float *partial = cv.take<float>(static_cast<size_t>(kBiasChunks) * cout);
+    float *partial = carve_bias(cv, cout);
     const int64_t rpc = ceil_div(std::max<int64_t>(n_out, 1), kBiasChunks);
     const int chunks = static_cast<int>(ceil_div(std::max<int64_t>(n_out, 1), rpc));
     if (dtype == RHIP_F32)
@@ -4151,7 +4185,7 @@ extern "C" int rhip_conv_backward_input(const void *grad_y, int64_t n_out,
     ConvWs w;
     if (workspace != nullptr) {
       Carve cv(workspace, workspace_bytes);
-      w = carve_conv_front(cv, K, cin, cout, dtype, n_in, n_out);
+      w = carve_conv_pass(cv, false, K, cin, cout, dtype, n_in, n_out);
     }
     const ConvWs *pw = workspace != nullptr ? &w : nullptr;
     if (dtype == RHIP_F32)
@@ -4183,7 +4217,7 @@ extern "C" int rhip_conv_backward_weight(
     // an offset pairs each input and each output row at most once
     const DwPlan plan = dw_plan(dtype, cin, cout, K, n_pairs, n_in, n_out);
     Carve cv(workspace, workspace_bytes);
-    const ConvWs w = carve_conv(cv, K, cin, cout, dtype, n_in, n_out, plan);
+    const ConvWs w = carve_conv_dw(cv, K, cin, cout, dtype, n_in, n_out, plan);
     if (dtype == RHIP_F32)
       run_dw<float>(static_cast<const float *>(x), n_in, cin,
                     static_cast<const float *>(grad_y), n_out, cout, kmap_offsets, K, in_rows,
@@ -4217,7 +4251,7 @@ extern "C" int rhip_conv_backward_weight_rows(
     RHIP_CHECK_ARG(workspace != nullptr, "workspace is null");
     RHIP_CHECK_ARG(aligned16(x) && aligned16(grad_y), "x and grad_y must be 16-byte aligned");
     Carve cv(workspace, workspace_bytes);
-    const ConvWs w = carve_conv(cv, K, cin, cout, dtype, n_in, n_out, DwPlan{});
+    const ConvWs w = carve_conv_dw(cv, K, cin, cout, dtype, n_in, n_out, DwPlan{});
     if (dtype == RHIP_F32)
       run_dw_pos(static_cast<const float *>(x), n_in, cin, static_cast<const float *>(grad_y),
                  n_out, cout, K, nbr, out_order, w.partial, static_cast<float *>(grad_w), stream);
@@ -4274,7 +4308,7 @@ extern "C" int rhip_conv_backward_weight_ragged(
     RHIP_CHECK_ARG(n_in == 0 || n_out == 0 || x, "x is null");
     RHIP_CHECK_ARG(workspace != nullptr, "workspace is null");
     Carve cv(workspace, workspace_bytes);
-    const ConvWs w = carve_conv(cv, K, cin, cout, dtype, n_in, n_out, DwPlan{});
+    const ConvWs w = carve_conv_dw(cv, K, cin, cout, dtype, n_in, n_out, DwPlan{});
     auto run = [&](auto *dw) {
       using T = std::remove_pointer_t<decltype(dw)>;
       const T *xt = static_cast<const T *>(x), *gt = static_cast<const T *>(grad_y);

@@ -21,20 +21,14 @@ int32_t rhip_dtype(const at::Tensor &t) {
               t.scalar_type());
 }
 
-// Workspace of a layer's calls; with_dw false: the forward, input-gradient
-// and bias-gradient calls only (the front of the full layout).
-at::Tensor conv_workspace(int32_t K, int64_t cin, int64_t cout, int32_t dt, int64_t n_in,
-                          int64_t n_out, int64_t n_pairs, bool with_dw, const at::Device &dev) {
+// Workspace of a layer's passes (RHIP_PASS_ bits), one call at a time.
+at::Tensor conv_workspace(int32_t passes, int32_t K, int64_t cin, int64_t cout, int32_t dt,
+                          int64_t n_in, int64_t n_out, int64_t n_pairs, const at::Device &dev) {
   size_t bytes = 0;
-  if (with_dw)
-    check_rhip(rhip_conv_workspace_bytes(K, static_cast<int32_t>(cin), static_cast<int32_t>(cout),
-                                         dt, n_in, n_out, n_pairs, &bytes),
-               "rhip_conv_workspace_bytes");
-  else
-    check_rhip(rhip_conv_forward_workspace_bytes(K, static_cast<int32_t>(cin),
-                                                 static_cast<int32_t>(cout), dt, n_in, n_out,
-                                                 &bytes),
-               "rhip_conv_forward_workspace_bytes");
+  check_rhip(rhip_conv_pass_workspace_bytes(passes, K, static_cast<int32_t>(cin),
+                                            static_cast<int32_t>(cout), dt, n_in, n_out, n_pairs,
+                                            &bytes),
+             "rhip_conv_pass_workspace_bytes");
   return torch::empty({static_cast<int64_t>(bytes)},
                       torch::TensorOptions().dtype(torch::kUInt8).device(dev));
 }
@@ -72,7 +66,7 @@ struct HipConvolutionFunction : public torch::autograd::Function<HipConvolutionF
     TORCH_CHECK(x.size(1) == cin, "feature channels ", x.size(1), " != kernel in-channels ", cin);
     const int32_t dt = rhip_dtype(x);
     auto y = torch::empty({n_out, cout}, x.options());
-    auto ws = conv_workspace(K, cin, cout, dt, n_in, n_out, n_pairs, false, dev);
+    auto ws = conv_workspace(RHIP_PASS_FORWARD, K, cin, cout, dt, n_in, n_out, n_pairs, dev);
     const bool has_bias = bias.numel() > 0;
     if (has_bias)
       TORCH_CHECK(bias.is_cuda() && bias.scalar_type() == torch::kFloat &&
@@ -110,16 +104,22 @@ struct HipConvolutionFunction : public torch::autograd::Function<HipConvolutionF
     const int32_t K = static_cast<int32_t>(w.size(0));
     const int64_t cin = w.size(1), cout = w.size(2), n_in = x.size(0);
     const int32_t dt = rhip_dtype(x);
-    const bool need_dw = ctx->needs_input_grad(1);
-    auto ws = conv_workspace(K, cin, cout, dt, n_in, n_out, n_pairs, need_dw, dev);
+    const bool need_dx = ctx->needs_input_grad(0), need_dw = ctx->needs_input_grad(1);
+    const bool need_db = ctx->saved_data["has_bias"].toBool() && ctx->needs_input_grad(2);
     at::Tensor gx, gw, gb;
-    if (ctx->saved_data["has_bias"].toBool() && ctx->needs_input_grad(2)) {
+    if (!need_dx && !need_dw && !need_db)
+      return {gx, gw, gb, {}, {}, {}, {}, {}, {}, {}, {}, {}, {}, {}};
+    auto ws = conv_workspace((need_dx ? RHIP_PASS_INPUT_GRAD : 0) |
+                                 (need_dw ? RHIP_PASS_WEIGHT_GRAD : 0) |
+                                 (need_db ? RHIP_PASS_BIAS_GRAD : 0),
+                             K, cin, cout, dt, n_in, n_out, n_pairs, dev);
+    if (need_db) {
       gb = torch::empty({cout}, x.options().dtype(torch::kFloat));
       check_rhip(rhip_conv_bias_grad(gy.data_ptr(), n_out, static_cast<int32_t>(cout), dt,
                                      gb.data_ptr<float>(), ws.data_ptr(), ws.numel(), st),
                  "rhip_conv_bias_grad");
     }
-    if (ctx->needs_input_grad(0)) {
+    if (need_dx) {
       gx = torch::empty_like(x);
       check_rhip(rhip_conv_backward_input(gy.data_ptr(), n_out, static_cast<int32_t>(cout),
                                           w.data_ptr(), K, static_cast<int32_t>(cin),
