@@ -175,6 +175,12 @@ int rhip_expand_coords(const int32_t *coords, int64_t n, int32_t ncol,
 int rhip_kmap_workspace_bytes(int64_t n_in, int64_t n_out, int32_t K,
                               size_t *bytes);
 
+/* The same for maps over this input table, which may need less: a table with
+ * a brick grid (rhip_spatial_order) reserves no room for the neighbours that
+ * the mask pass of other tables keeps (4 bytes per row and offset). */
+int rhip_kmap_table_workspace_bytes(const rhip_table *in_table, int64_t n_out,
+                                    int32_t K, size_t *bytes);
+
 /* Set by rhip_kmap_count for a map of a coordinate set onto itself (out_coords
  * are in_table's own rows, in order) whose stencil offsets are distinct and
  * closed under negation: one offset of each +/- pair is probed and the

@@ -32,7 +32,8 @@ EXPORTS = (
     "rhip_hash_workspace_bytes", "rhip_hash_build", "rhip_hash_lookup",
     "rhip_order_workspace_bytes", "rhip_brick_bytes", "rhip_spatial_order",
     "rhip_stride_coords",
-    "rhip_expand_coords", "rhip_kmap_workspace_bytes", "rhip_kmap_count", "rhip_kmap_fill",
+    "rhip_expand_coords", "rhip_kmap_workspace_bytes",
+    "rhip_kmap_table_workspace_bytes", "rhip_kmap_count", "rhip_kmap_fill",
     "rhip_kmap_pairs_workspace_bytes", "rhip_kmap_pairs", "rhip_stencil_partners",
     "rhip_conv_backward_weight_ragged", "rhip_conv_backward_weight_ragged_supported",
     "rhip_conv_backward_weight_rows_supported",
@@ -84,6 +85,7 @@ def _declare(lib):
         "rhip_stride_coords": (ctypes.c_int, [_vp, _i64, _i32, _P(_i32), _vp, _vp]),
         "rhip_expand_coords": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i32, _vp, _vp]),
         "rhip_kmap_workspace_bytes": (ctypes.c_int, [_i64, _i64, _i32, _P(_sz)]),
+        "rhip_kmap_table_workspace_bytes": (ctypes.c_int, [_P(RhipTable), _i64, _i32, _P(_sz)]),
         "rhip_kmap_count": (ctypes.c_int, [_P(RhipTable), _vp, _vp, _i64, _i32, _P(_i32),
                                            _vp, _sz, _vp, _vp, _vp, _P(_i64), _P(_i32),
                                            _vp]),
@@ -439,8 +441,8 @@ def kernel_map(in_table: CoordTable, out_table: CoordTable, offsets) -> KernelMa
     st = _stream(dev)
     nbr = torch.empty((K, max(n_out, 1)), dtype=torch.int32, device=dev)
     out_order = torch.empty(max(n_out, 1), dtype=torch.int32, device=dev)
-    ws = torch.empty(_sizeq(L.rhip_kmap_workspace_bytes, n_in, n_out, K), dtype=torch.uint8,
-                     device=dev)
+    ws = torch.empty(_sizeq(L.rhip_kmap_table_workspace_bytes, ctypes.byref(in_table.struct),
+                            n_out, K), dtype=torch.uint8, device=dev)
     kofs = torch.empty(K + 1, dtype=torch.int64, device=dev)
     flags = ctypes.c_int32(0)
     off_host = offsets.numpy()

@@ -585,7 +585,8 @@ HipKernelMap CoordinateManager::generate(const CoordinateMapHIP &in_map,
   m.n_in = n_in;
   m.n_out = n_out;
   size_t ws_bytes = 0;
-  check_rhip(rhip_kmap_workspace_bytes(n_in, n_out, K, &ws_bytes), "rhip_kmap_workspace_bytes");
+  check_rhip(rhip_kmap_table_workspace_bytes(&in_map.table, n_out, K, &ws_bytes),
+             "rhip_kmap_table_workspace_bytes");
   auto ws = device_bytes(ws_bytes, dev);
   // the map's table, processing order and CSR offsets in one block
   const int64_t rows_out = std::max<int64_t>(n_out, 1);

@@ -826,7 +826,7 @@ struct KmapWs {
   int32_t *vals_a, *vals_b;
   void *sort_tmp;
   size_t sort_bytes;
-  int32_t *rows; // the mask pass's neighbours (tables without bricks)
+  int32_t *rows; // the mask pass's neighbours (where it keeps them)
   // phase 2
   unsigned long long *mask_t;
   uint32_t *tkeys_a, *tkeys_b;
@@ -835,7 +835,13 @@ struct KmapWs {
   size_t tsort_bytes;
 };
 
-static KmapWs carve_kmap(Carve &cv, int64_t n_in, int64_t n_out, int32_t K, int32_t D) {
+// Whether the mask pass of a map over this table keeps its neighbours (a
+// missing table: one of any kind).
+static bool keeps_rows(const rhip_table *t, int32_t K) {
+  return K <= kKeptK && (t == nullptr || t->bricks == nullptr);
+}
+
+static KmapWs carve_kmap(Carve &cv, int64_t n_in, int64_t n_out, int32_t K, int32_t D, bool keep) {
   const int64_t nw = map_waves(n_out);
   const int64_t mo = std::max<int64_t>(n_out, 1), mi = std::max<int64_t>(n_in, 1);
   KmapWs w{};
@@ -852,7 +858,7 @@ static KmapWs carve_kmap(Carve &cv, int64_t n_in, int64_t n_out, int32_t K, int3
   w.vals_b = cv.take<int32_t>(mo);
   w.sort_bytes = sort_pairs_u32_bytes(mo);
   w.sort_tmp = cv.take<char>(w.sort_bytes);
-  w.rows = cv.take<int32_t>(K <= kKeptK ? static_cast<size_t>(mo) * kept_stride(K) : 1);
+  w.rows = cv.take<int32_t>(keep ? static_cast<size_t>(mo) * kept_stride(K) : 1);
   const size_t end1 = cv.used;
   cv.used = base;
   w.mask_t = cv.take<unsigned long long>(2 * mi);
@@ -960,7 +966,18 @@ extern "C" int rhip_kmap_workspace_bytes(int64_t n_in, int64_t n_out, int32_t K,
     RHIP_CHECK_ARG(bytes != nullptr, "bytes is null");
     RHIP_CHECK_ARG(n_in >= 0 && n_out >= 0 && K >= 1, "need n_in, n_out >= 0 and K >= 1");
     Carve cv(nullptr, 0);
-    carve_kmap(cv, n_in, n_out, K, RHIP_MAX_COLS - 1);
+    carve_kmap(cv, n_in, n_out, K, RHIP_MAX_COLS - 1, keeps_rows(nullptr, K));
+    *bytes = cv.used + 256;
+  });
+}
+
+extern "C" int rhip_kmap_table_workspace_bytes(const rhip_table *in_table, int64_t n_out,
+                                               int32_t K, size_t *bytes) {
+  return guarded([&] {
+    RHIP_CHECK_ARG(in_table != nullptr && bytes != nullptr, "in_table or bytes is null");
+    RHIP_CHECK_ARG(n_out >= 0 && K >= 1, "need n_out >= 0 and K >= 1");
+    Carve cv(nullptr, 0);
+    carve_kmap(cv, in_table->n_unique, n_out, K, RHIP_MAX_COLS - 1, keeps_rows(in_table, K));
     *bytes = cv.used + 256;
   });
 }
@@ -979,7 +996,8 @@ extern "C" int rhip_kmap_count(const rhip_table *in_table, const int32_t *out_co
                    "offsets_host, kmap_offsets and workspace are required");
     const int D = in_table->ncol - 1;
     Carve cv(workspace, workspace_bytes);
-    KmapWs w = carve_kmap(cv, in_table->n_unique, n_out, K, RHIP_MAX_COLS - 1);
+    KmapWs w = carve_kmap(cv, in_table->n_unique, n_out, K, RHIP_MAX_COLS - 1,
+                          keeps_rows(in_table, K));
     const int64_t nb = std::max<int64_t>(1, ceil_div(n_out, kMapBlock));
     const int64_t nw = map_waves(n_out);
     const std::vector<int32_t> partner =
@@ -1066,7 +1084,7 @@ extern "C" int rhip_kmap_count(const rhip_table *in_table, const int32_t *out_co
             return;
           }
         }
-        if (masks && K <= kKeptK && tv.bricks == nullptr) {
+        if (masks && keeps_rows(in_table, K)) {
           int lp = 0;
           while (kKeptU << lp < K)
             ++lp;
@@ -1153,7 +1171,8 @@ extern "C" int rhip_kmap_fill(const int32_t *nbr, const int32_t *out_order, int6
     const bool sym = (flags & RHIP_KMAP_SYMMETRIC) != 0;
     RHIP_CHECK_ARG(!sym || n_in == n_out, "a symmetric map has n_in == n_out");
     Carve cv(workspace, workspace_bytes);
-    KmapWs w = carve_kmap(cv, n_in, n_out, K, RHIP_MAX_COLS - 1);
+    // phase 1 is done with the neighbours it kept
+    KmapWs w = carve_kmap(cv, n_in, n_out, K, RHIP_MAX_COLS - 1, false);
     const int64_t nb = std::max<int64_t>(1, ceil_div(n_out, kMapBlock));
     const int64_t nw = map_waves(n_out);
     const bool want_t = nbr_t != nullptr && n_in > 0;

@@ -2,13 +2,14 @@
 one), whose neighbours the mask pass keeps and a permutation reads back:
 bit-exact pairs and tables against the oracle for the strides of the kept rows
 (1 to 32 offsets), strided and symmetric maps, two rows to several waves."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import oracle
+from riemannengine_amd import abi
 from helpers import gpu_canonical, gpu_tables_and_map, random_coords
-
-pytestmark = pytest.mark.gpu
 
 
 def _spread(c, D):
@@ -18,6 +19,7 @@ def _spread(c, D):
     return np.unique(far, axis=0).astype(np.int32)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("D,ks,n", [(3, 3, 2), (3, 3, 63), (3, 3, 700), (3, 2, 300), (2, 3, 300),
                                     (2, 5, 200), (1, 3, 65), (5, 2, 129), (4, 2, 64), (3, 1, 100)])
 def test_spread_clouds_match_oracle(D, ks, n):
@@ -36,6 +38,7 @@ def test_spread_clouds_match_oracle(D, ks, n):
     assert got == want
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("stride", [2, 3])
 def test_spread_strided_maps_match_oracle(stride):
     rng = np.random.default_rng(stride)
@@ -45,3 +48,20 @@ def test_spread_strided_maps_match_oracle(stride):
     kofs, ir, orr = oracle.kernel_map(c, out, off)
     _, _, km = gpu_tables_and_map(c, out, off)
     np.testing.assert_array_equal(gpu_canonical(km), oracle.canonical_pairs(kofs, ir, orr))
+
+
+def test_tables_with_bricks_reserve_no_kept_neighbours():
+    """Host sizes only: 28 entries a row less for 27 offsets where the table has a
+    brick grid, and the general query covers both."""
+    def ws(fn, *a):
+        return abi._sizeq(getattr(abi.lib(), fn), *a)
+
+    t = abi.RhipTable()
+    t.n_unique, t.ncol = 100000, 4
+    plain = ws("rhip_kmap_table_workspace_bytes", ctypes.byref(t), 50000, 27)
+    assert plain <= ws("rhip_kmap_workspace_bytes", 100000, 50000, 27)
+    t.n_unique = 1000  # the second phase, sized by the input rows, no longer the larger
+    plain = ws("rhip_kmap_table_workspace_bytes", ctypes.byref(t), 50000, 27)
+    t.bricks = 256  # any address: not read
+    bricks = ws("rhip_kmap_table_workspace_bytes", ctypes.byref(t), 50000, 27)
+    assert plain - bricks >= 28 * 4 * 50000 - 4096
