@@ -3455,19 +3455,31 @@ static int dw_pos_ranges(int K, int cin, int cout, int vb, int waves, int64_t n_
 // at most 8 offsets and channel counts that are not multiples of 64 keep
 // conv_dw_pos_bf16_kernel.
 constexpr int kDwShxKPW = 7;
-// Output channels that are not a multiple of 64 (96 above all) take it too,
-// the last tile part empty: conv_dw_pos_bf16_kernel has them in 32-channel
-// tiles, which read the X rows once each. Measured per call: 128->96 on 48k
-// rows 110 -> 74 us. Where the last input chunk is part empty as well, only on
-// large maps: 96->96 on 101k rows 149 -> 129, but on 10k 41 -> 54; with whole
-// output tiles never (96->128 on 48k 64 -> 72).
-constexpr int64_t kDwShxPartRows = 65536;
+static int dw_shx_units(int K, int cin, int cout) {
+  return static_cast<int>(ceil_div(cin, 64) * ceil_div(cout, 64) * ceil_div(K, kDwShxKPW));
+}
+// Output channels that are not a multiple of 64 (96 above all) may take it
+// too, the last tile (and input chunk) part empty. A workgroup of either
+// kernel streams its range of the rows in about the same time, so the one that
+// runs more ranges at once is faster, conv_dw_pos_bf16_kernel (32-channel
+// tiles) by 0 to 20 % where both run as many; with more workgroups than fit at
+// once it takes a second round. Measured per call on MI355X, 3^3, the other
+// kernel / this one: 96->96 (24 / 32 ranges) on 101k rows 156 / 134 us, on 48k
+// 90 / 81, but on 29k (24 each) 66 / 71 and on 10k (8 each) 49 / 61; 64->96 on
+// 101k (40 / 64) 108 / 85, on 23k (16 each) 54 / 66; 160->96 on 101k (16 each)
+// 222 / 236; 192->96 on 48k (8 / 16) 218 / 133; 224->160 on 10k (8 each, 560
+// workgroups / 384) 98 / 77.
 static bool dw_shx_bf16(int K, int cin, int cout, int64_t n_out) {
   if (K <= kDwPosMaxKSmall || cin % 16 != 0 || cout % 32 != 0)
     return false;
   if (cout % 64 == 0)
     return cin % 64 == 0;
-  return cout > 64 && (cin % 64 == 0 || (cin > 64 && n_out >= kDwShxPartRows));
+  if (cin < 64 || cout < 64)
+    return false;
+  const int pos = dw_pos_ranges(K, cin, cout, 2, 2, n_out, 16);
+  const int groups = static_cast<int>(ceil_div(K, kWaves * dw_pos_kpw(K)));
+  return dw_ranges_for(dw_shx_units(K, cin, cout), 2, n_out, 16) > pos ||
+         pos * (cin / 16) * (cout / 32) * groups > 256 * 2;
 }
 
 // Ranges of conv_dw_pos_bf16_kernel (or conv_dw_shx_bf16_kernel) and
@@ -3475,9 +3487,7 @@ static bool dw_shx_bf16(int K, int cin, int cout, int64_t n_out) {
 // them).
 static int dw_pos_bf16_ranges(int K, int cin, int cout, int64_t n_out) {
   if (dw_shx_bf16(K, cin, cout, n_out))
-    return dw_ranges_for(static_cast<int>(ceil_div(cin, 64) * ceil_div(cout, 64) *
-                                          ceil_div(K, kDwShxKPW)),
-                         2, n_out, 16);
+    return dw_ranges_for(dw_shx_units(K, cin, cout), 2, n_out, 16);
   const int waves = K <= kDwPosMaxKSmall ? 4 : 2;
   return dw_pos_ranges(K, cin, cout, cout % 64 == 0 ? 4 : 2, waves, n_out, 16);
 }

@@ -34,16 +34,19 @@ def test_96_channel_layers_match_oracle(n, ks, cin, cout):
         assert_rel(got.float().cpu().numpy(), ref, TOL[torch.bfloat16], name)
 
 
-def test_96_channel_weight_gradient_of_a_large_map():
-    """Enough rows for the shared-row kernel with its last input chunk part
-    empty, against the pair-list kernel (the same products in another order;
-    both sum in fp32, the result rounds to bf16 once: 2^-8)."""
+@pytest.mark.parametrize("n,cin,cout", [
+    (66001, 96, 96), (30000, 192, 96), (5000, 224, 160), (40001, 80, 224), (30001, 160, 96),
+    (9000, 96, 96), (70000, 64, 96)])
+def test_weight_gradient_with_part_empty_tiles(n, cin, cout):
+    """Channel counts that are no multiples of 64, on either side of where the
+    shared-row kernel takes over, against the pair-list kernel (the same
+    products in another order; both sum in fp32, the result rounds to bf16
+    once: 2^-8)."""
     rng = np.random.default_rng(1)
     c, _, _ = oracle.insert_and_map(random_coords(rng, 100000, 3, 30))
-    n = 66001
     km = gpu_tables_and_map(c[:n], c[:n], oracle.region_offsets(3, 3), same=True)[2]
-    x, gy = (to_dev(rng.standard_normal((n, 96)).astype(np.float32), torch.bfloat16)
-             for _ in range(2))
+    x, gy = (to_dev(rng.standard_normal((n, k)).astype(np.float32), torch.bfloat16)
+             for k in (cin, cout))
     got, ref = abi.conv_weight_grad(x, gy, km, 27), abi.conv_backward_weight(x, gy, km, 27)
     assert_rel(got.float().cpu().numpy(), ref.float().cpu().numpy(), 2 ** -8, "dW")
     assert torch.equal(got, abi.conv_weight_grad(x, gy, km, 27))
