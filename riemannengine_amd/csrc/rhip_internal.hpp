@@ -260,21 +260,22 @@ struct StrideArg {
 // runs throughout, a map of 17 tiles ran on two XCDs and left six idle: the
 // 256-channel fp32 forward on 2,057 rows 285 us, dealt evenly 126; bf16 89
 // and 44; with four or eight runs per XCD, bf16 96->96 on 101k rows 142 / 141
-// us against 139-142, 64->64 on 48k rows 35.4 / 34.9 against 34.1.) The grid is padded to a multiple of 8 runs (padding ids map past
-// the last tile). The run follows from the padded grid, which the padding
-// lifts to the next run's threshold only where it is a multiple of that run
-// too.
+// us against 139-142, 64->64 on 48k rows 35.4 / 34.9 against 34.1.) The grid
+// is padded to a multiple of 8 runs (padding ids map past the last tile). The
+// run follows from the padded grid, which the padding lifts to the next run's
+// threshold only where it is a multiple of that run too.
 constexpr int kXcds = 8;
 constexpr int kXcdRunLog = 4;
 __host__ __device__ __forceinline__ int xcd_run_log(uint32_t tiles) {
   const uint32_t runs = tiles / (2 * kXcds);
   return runs < 1 ? 0 : (runs >> kXcdRunLog ? kXcdRunLog : 31 - __builtin_clz(runs));
 }
-__device__ __forceinline__ int64_t xcd_tile(uint32_t b) {
-  const int lg = xcd_run_log(gridDim.x);
+__host__ __device__ __forceinline__ int64_t xcd_tile(uint32_t b, uint32_t grid) {
+  const int lg = xcd_run_log(grid);
   const uint32_t x = b % kXcds, m = b / kXcds;
   return ((((m >> lg) * kXcds + x) << lg) + (m & ((1u << lg) - 1)));
 }
+__device__ __forceinline__ int64_t xcd_tile(uint32_t b) { return xcd_tile(b, gridDim.x); }
 inline int64_t xcd_grid(int64_t tiles) {
   const int64_t n = static_cast<int64_t>(kXcds)
                     << xcd_run_log(static_cast<uint32_t>(std::min<int64_t>(tiles, UINT32_MAX)));

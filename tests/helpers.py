@@ -40,6 +40,21 @@ def gpu_canonical(km):
                                   km.out_rows.cpu().numpy())
 
 
+def reference_passes(km, x, gy, w):
+    """(Y, dX, dW) of a convolution as one fp32 product per offset on the
+    device."""
+    y = torch.zeros(km.n_out, w.shape[2], device=DEV)
+    gx, gw = torch.zeros(x.shape, device=DEV), torch.zeros(w.shape, device=DEV)
+    for k in range(w.shape[0]):
+        s = slice(int(km.offsets_host[k]), int(km.offsets_host[k + 1]))
+        ir, orr, wk = km.in_rows[s].long(), km.out_rows[s].long(), w[k].float()
+        xk, gk = x[ir].float(), gy[orr].float()
+        y.index_add_(0, orr, xk @ wk)
+        gx.index_add_(0, ir, gk @ wk.t().contiguous())
+        gw[k] = xk.t().contiguous() @ gk
+    return y, gx, gw
+
+
 def random_coords(rng, n, D=3, span=20, batch=2):
     c = np.concatenate([rng.integers(0, batch, (n, 1)), rng.integers(-span, span, (n, D))], 1)
     return c.astype(np.int32)

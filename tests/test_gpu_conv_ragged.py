@@ -2,7 +2,8 @@
 forward with bias, input gradient and weight gradient at the edges of the
 thin kernels' tiles (64 positions, 96 im2col columns, 16 / 32 / 64 output
 columns; rows of 2-, 4- and 16-byte pieces) and of the padded widths (32, 64,
-128, 192, 256), and with weights or gradients that are not finite. Tolerance:
+128, 192, 256; copies that run on the small-map kernel, on larger maps and on
+more than 32 offsets on the tiled ones), and with weights or gradients that are not finite. Tolerance:
 norm-wise rel 1e-4 for fp32 and 2e-2 for bf16 (helpers.TOL)."""
 import numpy as np
 import pytest
@@ -55,7 +56,8 @@ def _ragged_dw(x, gy, km):
     (700, 3, 4, 80), (129, 3, 6, 13), (300, 5, 1, 20), (300, 5, 6, 40), (257, 1, 64, 20),
     (1000, 1, 256, 10), (500, 1, 13, 21), (200, 2, 12, 100), (130, 3, 24, 24), (90, 3, 37, 5),
     (400, 3, 64, 20), (400, 3, 20, 64), (257, 3, 33, 65), (129, 2, 40, 129), (300, 3, 200, 72),
-    (200, 5, 24, 40), (150, 3, 300, 8), (3000, 3, 40, 40)])
+    (200, 5, 24, 40), (150, 3, 300, 8), (3000, 3, 40, 40), (5000, 3, 72, 129),
+    (5001, 3, 24, 100)])
 def test_ragged_layers_match_oracle(n, ks, cin, cout, dtype):
     km = _map(n, ks, seed=n + ks)
     rng = np.random.default_rng(cin * 31 + cout)
@@ -64,6 +66,8 @@ def test_ragged_layers_match_oracle(n, ks, cin, cout, dtype):
     b = rng.standard_normal(cout).astype(np.float32)
     xt, wt, gyt = (to_dev(a.astype(np.float32), dtype) for a in (x, w, gy))
     print(f"ragged n={n} ks={ks} {cin}->{cout} {dtype}", flush=True)
+    assert all(abi.conv_plan(dtype, km.K, *s, n, n)[0] in ("thin", "padded")
+               for s in ((cin, cout), (cout, cin)))
     y = abi.conv_forward(xt, wt, km, bias=to_dev(b))
     gx = abi.conv_backward_input(gyt, wt, km)
     ry, rgx, rgw = _reference(km, *(t.float().cpu().numpy() for t in (xt, wt, gyt)))

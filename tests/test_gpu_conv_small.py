@@ -1,7 +1,8 @@
 """Maps with few rows: forward with bias and input gradient of the kernel
 whose waves share out a 16-row tile's stages, against the oracle at its edges
 (16 rows, 16 / 32 / 64 columns, one chunk or several, fewer stages than waves,
-1 to 32 offsets, both weight layouts). Tolerance: norm-wise rel 1e-4 for fp32
+1 to 32 offsets, both weight layouts; in bf16 a direction that reduces an odd
+multiple of 16 channels runs on the general kernel). Tolerance: norm-wise rel 1e-4 for fp32
 and 2e-2 for bf16 (helpers.TOL)."""
 import numpy as np
 import pytest
@@ -28,6 +29,9 @@ def test_small_map_layers_match_oracle(n, off, cin, cout, dtype):
     x, gy = (to_dev(rng.standard_normal((n, k)).astype(np.float32), dtype) for k in (cin, cout))
     w = to_dev((rng.standard_normal((km.K, cin, cout)) / 20).astype(np.float32), dtype)
     b = rng.standard_normal(cout).astype(np.float32)
+    plans = [abi.conv_plan(dtype, km.K, *s, n, n)[0] for s in ((cin, cout), (cout, cin))]
+    odd = [dtype == torch.bfloat16 and c % 32 != 0 for c in (cin, cout)]
+    assert plans == ["tiled" if o else "small" for o in odd]
     print(f"small n={n} K={km.K} {cin}->{cout} {dtype}", flush=True)
     y, gx = abi.conv_forward(x, w, km, bias=to_dev(b)), abi.conv_backward_input(gy, w, km)
     kofs, ir, orr = km.offsets_host, km.in_rows.cpu().numpy(), km.out_rows.cpu().numpy()

@@ -9,7 +9,7 @@ import torch
 
 import oracle
 from riemannengine_amd import abi
-from helpers import DEV, TOL, gpu_tables_and_map, random_coords, to_dev
+from helpers import DEV, TOL, gpu_tables_and_map, random_coords, reference_passes, to_dev
 
 WIDTHS = (16, 32, 48, 64, 80, 96, 112, 128, 144, 160, 176, 192, 240, 256, 288, 384)
 
@@ -118,13 +118,5 @@ def test_calls_stay_in_their_workspace(n, cin, cout, dtype, kernel):
                   (p(x), n, cin, p(gy), n, cout, 27, p(km.offsets), km.n_pairs, p(km.in_rows),
                    p(km.out_rows), p(gw)))
     abi._check(rc, "dW")
-    ry, rgx, rgw = (torch.zeros(t.shape, device=DEV) for t in (y, gx, gw))
-    for k in range(27):
-        s = slice(int(km.offsets_host[k]), int(km.offsets_host[k + 1]))
-        ir, orr, wk = km.in_rows[s].long(), km.out_rows[s].long(), w[k].float()
-        xk, gk = x[ir].float(), gy[orr].float()
-        ry.index_add_(0, orr, xk @ wk)
-        rgx.index_add_(0, ir, gk @ wk.t().contiguous())
-        rgw[k] = xk.t().contiguous() @ gk
-    for got, ref in ((y, ry), (gx, rgx), (gw, rgw)):
+    for got, ref in zip((y, gx, gw), reference_passes(km, x, gy, w)):
         assert float((got.float() - ref).abs().max()) <= TOL[dtype] * float(ref.abs().max())
