@@ -55,6 +55,8 @@ if ROOT not in sys.path:
 # MI355X published peaks (dense): HBM3E bandwidth and MFMA throughput.
 PEAK_HBM_GBS = 8000.0
 PEAK_TFLOPS = {"f32": 157.3, "bf16": 2500.0}
+# fp32 operands as three bf16 parts each: six bf16 products per multiplication
+PEAK_PARTS_TFLOPS = PEAK_TFLOPS["bf16"] / 6
 
 
 def parse_args():
@@ -319,15 +321,28 @@ def _map_time(build, reps, warmup=5):
     return out, statistics.median(ms)
 
 
-def _roof(F, B, ms, dtype):
+def conv_kernels(dtype, K, cin, cout, n_in, n_out):
+    """The kernel rhip_conv_plan names for a layer's forward and input gradient."""
+    from riemannengine_amd import abi
+    return {"forward": abi.conv_plan(dtype, K, cin, cout, n_in, n_out)[0],
+            "backward_input": abi.conv_plan(dtype, K, cout, cin, n_out, n_in)[0]}
+
+
+def _peak(dtype, kernel=None):
+    """TFLOP/s of algorithmic work that a pass's matrix instructions reach at most."""
+    return PEAK_PARTS_TFLOPS if kernel == "parts" else PEAK_TFLOPS[dtype]
+
+
+def _roof(F, B, ms, dtype, kernel=None):
     """(bound, achieved, peak, unit, frac, t_roof_ms) of one pass: bound by
-    whichever of the MFMA peak (the dtype's) and the HBM peak would take
+    whichever of the MFMA peak (its kernel's) and the HBM peak would take
     longer on its algorithmic work."""
-    t_f = F / (PEAK_TFLOPS[dtype] * 1e12)
+    peak = _peak(dtype, kernel)
+    t_f = F / (peak * 1e12)
     t_b = B / (PEAK_HBM_GBS * 1e9)
     dur = ms * 1e-3
     if t_f >= t_b:
-        rec = {"bound": "mfma", "achieved": round(F / dur / 1e12, 3), "peak": PEAK_TFLOPS[dtype],
+        rec = {"bound": "mfma", "achieved": round(F / dur / 1e12, 3), "peak": round(peak, 1),
                "unit": "TFLOP/s"}
     else:
         rec = {"bound": "hbm", "achieved": round(B / dur / 1e9, 1), "peak": PEAK_HBM_GBS,
@@ -381,6 +396,7 @@ def config5_per_kernel(stage_in, stage_out, chans, dt, s, reps=10):
             x, gy = rnd(km.n_in, cin), rnd(km.n_out, cout)
             w = rnd(km.K, cin, cout) * 0.05
             work = conv_traffic(km.n_in, km.n_out, km.n_pairs, km.K, cin, cout, s)
+            kern = conv_kernels(dt, km.K, cin, cout, km.n_in, km.n_out)
             for pname, fn in (("forward", lambda: abi.conv_forward(x, w, km)),
                               ("backward_input", lambda: abi.conv_backward_input(gy, w, km)),
                               ("backward_weight", lambda: abi.conv_weight_grad(x, gy, km, km.K))):
@@ -389,7 +405,7 @@ def config5_per_kernel(stage_in, stage_out, chans, dt, s, reps=10):
                 rec = {"stage": i + 1, "op": f"{op} C{cin}->{cout}", "pass": pname,
                        "rows_in": km.n_in, "rows_out": km.n_out, "pairs": km.n_pairs,
                        "per_step": count}
-                rec.update(_roof(F, B, ms, dname))
+                rec.update(_roof(F, B, ms, dname, kern.get(pname)))
                 out.append(rec)
             del x, gy, w
         x, r, gy = rnd(n, C), rnd(n, C), rnd(n, C)
@@ -923,6 +939,8 @@ def conv_step_record(args, dtype, km, n_in, n_out, P, K, cin, cout):
     per = {n: statistics.mean(e[j].elapsed_time(e[j + 1]) for e in bev)
            for j, n in enumerate(names)}
     work = conv_traffic(n_in, n_out, P, K, cin, cout, s)
+    kernels = conv_kernels(dt, K, cin, cout, n_in, n_out)
+    peak = {n: _peak(dtype, kernels.get(n)) for n in names}
     dom = max(names, key=lambda n: per[n])
     F, B = work[dom]
     # the dominant pass's duration from the timed steps where that is dW
@@ -930,29 +948,29 @@ def conv_step_record(args, dtype, km, n_in, n_out, P, K, cin, cout):
     dur_s = kernel_ms * 1e-3
     if dtype == "f32":
         roof = {"bound": "mfma", "achieved": round(F / dur_s / 1e12, 3),
-                "peak": PEAK_TFLOPS["f32"], "unit": "TFLOP/s"}
+                "peak": round(peak[dom], 1), "unit": "TFLOP/s"}
     else:
         roof = {"bound": "hbm", "achieved": round(B / dur_s / 1e9, 1),
                 "peak": PEAK_HBM_GBS, "unit": "GB/s"}
     roof["frac"] = round(roof["achieved"] / roof["peak"], 4)
     roof["traffic"], roof["traffic_source"] = measured_traffic(dtype, dom)
     roof["mfma"] = measured_mfma(dtype, dom, F)
-    roof["kernel"] = {"forward": "conv_os_lds_kernel (forward)",
-                      "backward_input": "conv_os_lds_kernel (dX)",
-                      "backward_weight": (
-                          "conv_dw_pos64_kernel + conv_dw_rows_reduce_kernel (dW pass)"
-                          if dtype == "f32" else
-                          "conv_dw_shx_bf16_kernel + conv_dw_rows_reduce_kernel (dW pass)")}[dom]
+    os_names = {"parts": "conv_x3_kernel", "lds": "conv_os_lds_kernel"}
+    roof["kernel"] = (
+        ("conv_dw_pos64_kernel" if dtype == "f32" else "conv_dw_shx_bf16_kernel") +
+        " + conv_dw_rows_reduce_kernel (dW pass)" if dom == "backward_weight" else
+        "%s (%s)" % (os_names.get(kernels[dom], kernels[dom]), dom))
     roof["kernel_ms"] = round(kernel_ms, 4)
     roof["kernel_ms_source"] = ("events around dW in every %dth timed step" % every
                                 if dom == "backward_weight"
                                 else "events in %d untimed steps after the timed ones" % nb)
     roof["algorithmic"] = {"flop": F, "bytes": B}
 
-    # whole-step roofline: max(compute, memory) time at peak / measured
+    # whole-step roofline: max(compute, memory) time at peak / measured, each
+    # pass's compute at the rate of its own kernel
     Ft = sum(v[0] for v in work.values())
     Bt = sum(v[1] for v in work.values())
-    t_roof = max(Ft / (PEAK_TFLOPS[dtype] * 1e12), Bt / (PEAK_HBM_GBS * 1e9))
+    t_roof = max(sum(work[n][0] / (peak[n] * 1e12) for n in names), Bt / (PEAK_HBM_GBS * 1e9))
     return {
         "value": round(n_in / (ms_per_step * 1e-3) / 1e6, 3),
         "unit": "Mvoxels/s",
@@ -963,6 +981,7 @@ def conv_step_record(args, dtype, km, n_in, n_out, P, K, cin, cout):
         "step_roofline": {"t_roof_ms": round(t_roof * 1e3, 4),
                           "frac": round(t_roof * 1e3 / ms_per_step, 4),
                           "frac_source": "t_roof / timed ms_per_step",
+                          "mfma_peak_tflops": {n: round(peak[n], 1) for n in names},
                           "flop": Ft, "bytes": Bt},
         "roofline": roof,
     }
