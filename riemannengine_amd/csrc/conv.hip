@@ -323,10 +323,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(WAVES)
 
 // conv_os_kernel's fast form for stencils of at most 4 * KQ offsets (KQ = 8:
 // 32 offsets, one mask word; KQ = 24: 96, three words), reduction widths of
-// 1, 2 or 4 channel chunks (CW = cred = credw, a compile-time
-// constant), no split of the offset axis and inputs addressable by 32-bit
-// buffer offsets. It computes the same sums in the same order; what differs
-// is the control around them:
+// 1, 2 or 4 chunks of CSUB 16- or 32-channel loads (bf16 also 3 loads a chunk:
+// 96 and 192 channels; CW = cred = credw, a compile-time constant) and inputs
+// addressable by 32-bit buffer offsets; a split offset axis in bf16 only. It
+// computes the same sums in the same order; what differs is the control around
+// them:
 //  * each wave stores its row groups' neighbour indices (offsets 4q + g in
 //    lane (i16, g) of slot q) in LDS once, and a stage reads its row's index
 //    with one ds_read instead of a register select chain and a ds_bpermute;
@@ -2989,9 +2990,10 @@ static bool run_os_lds_nt(const T *x, int64_t n_x, int cred, const T *wt, const 
                                 splits, partial, s, wtr);
 }
 
-// The fast forward/dX kernel where it applies: at most 96 offsets, no split,
-// unpadded reductions of one, two or four chunks (bf16 also three and six)
-// and inputs that 32-bit buffer offsets reach. Returns whether it launched.
+// The fast forward/dX kernel where it applies: at most 96 offsets, no fp32 split,
+// unpadded reductions of one, two or four chunks (bf16 also three and six; the
+// widths are template arguments, and 288 or 384 channels are not built) and
+// inputs that 32-bit buffer offsets reach. Returns whether it launched.
 template <typename T>
 static bool run_os_lds(const T *x, int64_t n_x, int cred, const T *wt, const int32_t *wperm,
                        int credw, int ncols, const float *bias, const int32_t *nbr,

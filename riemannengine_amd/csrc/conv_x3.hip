@@ -2,16 +2,17 @@
 // output-stationary gather GEMM of conv_os_lds_kernel with each fp32 operand
 // as the sum of three bf16 parts.
 //
-// A float is hi + mid + lo exactly enough: hi rounds it to bf16 (8 bits), mid
-// rounds the rest, lo rounds what is left, so what is lost is under 2^-25 of
-// it. Of the nine products of two such sums the six largest are kept (hi hi,
-// hi mid, mid hi, mid mid, hi lo, lo hi); the dropped ones are under 2^-25 of
-// the product, below the rounding of one fp32 multiplication. All sums stay
-// fp32 in the MFMA accumulators. Six v_mfma_f32_16x16x32_bf16 take 96 cycles
-// for 32 channels where eight v_mfma_f32_16x16x4_f32 take 256. The error
-// against 64-bit sums (2-norm, 3^3, normal / ReLU features) is below the fp32
-// MFMAs': 64->64 9.6e-8 / 7.9e-8 against 3.8e-7 / 2.7e-7, 256->256 3.7e-7 /
-// 3.0e-7 against 1.1e-6 / 7.5e-7.
+// A float is hi + mid + lo: hi rounds it to bf16 (8 bits), mid rounds the
+// rest, lo is what is left. Of the nine products of two such sums the six
+// largest are kept (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi); the dropped
+// ones are under 2^-25 of the product, below the rounding of one fp32
+// multiplication (the method: G. Henry, P. T. P. Tang, A. Heinecke, "Leveraging
+// the bfloat16 Artificial Intelligence Datatype For Higher-Precision
+// Computations", ARITH 2019). All sums stay fp32 in the MFMA accumulators. Six
+// v_mfma_f32_16x16x32_bf16 take 96 cycles for 32 channels where eight
+// v_mfma_f32_16x16x4_f32 take 256. The error against 64-bit sums (2-norm, 3^3,
+// normal / ReLU features) is below the fp32 MFMAs': 64->64 9.6e-8 / 7.9e-8
+// against 3.8e-7 / 2.7e-7, 256->256 3.7e-7 / 3.0e-7 against 1.1e-6 / 7.5e-7.
 //
 // Both operands are split after a multiplication by 2^24, and the sums are
 // multiplied by 2^-48. The parts of a float are multiples of its last bit, at
@@ -33,7 +34,6 @@ namespace rhip {
 
 namespace {
 
-typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 constexpr int kMaxK = 128;
 
 constexpr float kScale = 0x1p24f, kUnscale = 0x1p-48f; // operands, sums
@@ -99,9 +99,11 @@ struct Operands {
 // walked as a bit mask, quad-order gathers, missing neighbours as loads past
 // the buffer), RG 16-row groups per wave so that each weight fragment read
 // from LDS (three parts, 1.5 times the bytes of fp32) serves RG groups.
-// Bound by no single unit: on 410k rows, 64->64 (284 us with one sum), a
-// variant without the gathers took 218 us, one without the split into parts
-// 253, one with the hi hi product alone 172. Stages of 64 channels at 3 waves
+// Bound by no single unit: on 410k rows, 64->64, the matrix pipes are busy 0.39
+// of the time, the VALU 0.40, LDS 0.15 and 0.21 more in bank conflicts; of 284
+// us (with one sum, operands not scaled) a variant without the gathers took
+// 218, one without the split into parts 253, one with the hi hi product alone
+// 172. Stages of 64 channels at 3 waves
 // per SIMD took 293, one row group per wave 309-334, three or four 298.
 template <int NT, int RG, int WAVES, int CW, int KQ, bool SPLIT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(WAVES))) void
@@ -470,7 +472,11 @@ void launch(dim3 grid, bool split, const float *x, int64_t n_x, const __bf16 *wt
 // 43 / 33, on 2k 24 / 25; 96->96 on 101k rows 339 / 260; 128->128 on 10k rows
 // 120 / 79; 256->256 on 2k rows 122 / 84; 81 offsets, 64->64, 233k rows 1007 /
 // 718; but 32->32 on 200k rows 70 / 67, 64->32 on 200k rows 121 / 125, 64->16
-// on 101k rows 46 / 70.
+// on 101k rows 46 / 70. (Scaling the operands came after these and costs 1 to
+// 3 %: 64->64 on 410k rows 293, 256->256 on 48k 743 -> 758.) The width is a
+// template argument, of which each value adds 12 kernels; the five are those
+// that networks have most, and other multiples of 32 (160, 224, 320 and on)
+// stay on the fp32 MFMAs, where they were not compared.
 bool conv_x3_takes(int cred, int ncols, int K, int64_t n_x) {
   const bool width = cred == 64 || cred == 96 || cred == 128 || cred == 192 ||
                      cred == 256;
