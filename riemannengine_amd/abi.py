@@ -654,7 +654,8 @@ def conv_weight_grad(x: torch.Tensor, grad_y: torch.Tensor, kmap: KernelMap,
                                                   kmap.n_out, cout, K, _ptr(kmap.nbr),
                                                   _ptr(kmap.out_order), _ptr(gw), dt, _ptr(ws),
                                                   ws.numel(), _stream(x.device))
-    if st == RHIP_ERR_UNSUPPORTED:
+    if st == RHIP_ERR_UNSUPPORTED and lib().rhip_conv_backward_weight_ragged_supported(
+            dt, cin, cout, K, kmap.n_in, kmap.n_out):
         st = lib().rhip_conv_backward_weight_ragged(_ptr(x), kmap.n_in, cin, _ptr(grad_y),
                                                   kmap.n_out, cout, K, _ptr(kmap.nbr),
                                                   _ptr(kmap.out_order), _ptr(gw), dt, _ptr(ws),

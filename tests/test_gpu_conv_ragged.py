@@ -23,6 +23,22 @@ def test_ragged_weight_gradient_query_without_a_gpu():
     assert q(7, 3, 32, 27, 1000, 1000) == 0 and q(abi.F32, 3, 32, 27, -1, 1000) == 0
 
 
+@pytest.mark.gpu
+def test_a_pair_list_weight_gradient_asks_for_no_ragged_kernel(monkeypatch):
+    """Neither thin nor padded (216 offsets of 40 channels): the query says so,
+    and no call is made to be refused."""
+    km, lib = _map(60, 6, seed=3, span=3), abi.lib()
+    x, gy = (to_dev(np.ones((60, c), np.float32)) for c in (40, 8))
+
+    def refused(*args):
+        raise AssertionError("called for a shape its query refuses")
+
+    monkeypatch.setattr(lib, "rhip_conv_backward_weight_ragged", refused)
+    got = abi.conv_weight_grad(x, gy, km, km.K)
+    pairs = torch.from_numpy(np.diff(km.offsets_host).astype(np.float32))
+    assert torch.equal(got.cpu(), pairs[:, None, None].expand(km.K, 40, 8))
+
+
 def _map(n, ks, seed, span=7):
     c, _, _ = oracle.insert_and_map(random_coords(np.random.default_rng(seed), 4 * n + 8, 3, span))
     c = c[:n]
