@@ -2678,8 +2678,6 @@ static void launch_os(const T *x, int cred, const T *wt, int credw, int ncols,
 template <typename T> static int os_nt(int ncols) {
   if (!kIsF32<T> && ncols % 128 == 0)
     return 128;
-  if (!kIsF32<T> && ncols % 96 == 0)
-    return 96;
   return ncols % 64 == 0 ? 64 : (ncols % 32 == 0 ? 32 : 16);
 }
 
@@ -2771,27 +2769,51 @@ static bool thin_runs(int K, int C, int64_t n_x, int elem_bytes, bool can_pad) {
          (!can_pad || C <= kThinChannels || K * C <= kThinCols || (K == 1 && C <= kThinCols1));
 }
 
+// Rows of a workgroup's tile (bf16 128-column tiles hold kWideRG row groups
+// per wave, 96-column ones too where a stage has two chunks or more).
+template <typename T> static int os_tile_rows(int nt, int cred) {
+  const bool wide = !kIsF32<T> && (nt >= 128 || (nt == 96 && cred >= 64));
+  return kWaves * 16 * (wide ? kWideRG : 1);
+}
+
+// Workgroups that a launch aims at with splits of the offset axis.
+constexpr int64_t kSplitBlocks = 640;
+
+// Whether a bf16 layer takes 96-column tiles (the LDS-indexed kernel alone has
+// them). They gather a row once where 32-column tiles do so three times, but
+// are a third of the workgroups, and where those would be split, the partial
+// sums of a short reduction cost more than the gathers: stride-2 maps (8
+// offsets, and one neighbour per row in their transposes), 32 channels, and 64
+// into one tile keep the narrower tiles there. Per call on MI355X, 32- or
+// 64-column tiles / 96 split: transposed 2^3 192->96 on 23k rows 12.6 / 23.7
+// us, 192->192 16.3 / 26.1; 3^3 32->96 on 23k 18.0 / 27.0 (on 101k, unsplit,
+// 38.5 / 32.0), 64->96 26.5 / 29.8; but 96->96 on 10k 59 / 29, 64->192 34 / 28.
+template <typename T>
+static bool os_nt96(int cred, int credw, int ncols, int64_t n_rows, int K) {
+  if (kIsF32<T> || ncols % 128 == 0 || ncols % 96 != 0 || cred != credw || K > kLdsMaxK ||
+      !os_lds_width<T>(cred))
+    return false;
+  const bool narrow = K <= 8 || cred == 32 || (cred == 64 && ncols == 96);
+  const int64_t blocks = ceil_div(n_rows, os_tile_rows<T>(96, cred)) * (ncols / 96);
+  return !narrow || (kSplitBlocks + blocks / 2) / blocks <= 1;
+}
+
 // Splits of the offset axis for the MFMA kernel: a map with few rows and
 // wide channels gives too few workgroups to hide the gathers (one per CU
 // for 9k rows at 256 channels), so the (offset, channel chunk) stages are
 // shared among up to 8 workgroups per tile, aiming at ~640 workgroups
 // (measured on the config-5 stages), each keeping at least 4 stages on
-// average. 1 = no split. The tiles counted are those the reduction runs in:
-// bf16 128-column tiles hold kWideRG row groups per wave, and 96-column tiles
-// exist in the LDS-indexed kernel alone (32-column tiles elsewhere). credw:
-// the width red_width pads cred to, which is what the stages are counted in.
+// average. 1 = no split. The tiles counted are those the reduction runs in.
+// credw: the width red_width pads cred to, which is what the stages are counted
+// in.
 template <typename T>
 static int os_splits(int64_t n_rows, int cred, int credw, int ncols, int K) {
   if (n_rows <= 0 || ncols % 16 != 0)
     return 1;
-  int nt = os_nt<T>(ncols);
-  if (nt == 96 && !(cred == credw && K <= kLdsMaxK && os_lds_width<T>(cred)))
-    nt = 32;
-  const bool wide = !kIsF32<T> && (nt >= 128 || (nt == 96 && cred >= 64));
-  const int rows = kWaves * 16 * (wide ? kWideRG : 1);
-  const int64_t blocks = ceil_div(n_rows, rows) * (ncols / nt);
+  const int nt = os_nt96<T>(cred, credw, ncols, n_rows, K) ? 96 : os_nt<T>(ncols);
+  const int64_t blocks = ceil_div(n_rows, os_tile_rows<T>(nt, cred)) * (ncols / nt);
   const int64_t stages = static_cast<int64_t>(K) * std::max(1, credw / 64);
-  const int64_t want = (640 + blocks / 2) / blocks; // nearest
+  const int64_t want = (kSplitBlocks + blocks / 2) / blocks; // nearest
   return static_cast<int>(
       std::max<int64_t>(1, std::min<int64_t>({8, want, std::max<int64_t>(1, stages / 4)})));
 }
@@ -2971,7 +2993,7 @@ static bool run_os_lds_nt(const T *x, int64_t n_x, int cred, const T *wt, const 
                           int ncols, const float *bias, const int32_t *nbr, int64_t n_rows,
                           int K, const int32_t *order, T *y, int splits, float *partial,
                           hipStream_t s, bool wtr = false) {
-  const int nt = os_nt<T>(ncols);
+  const int nt = os_nt96<T>(cred, cred, ncols, n_rows, K) ? 96 : os_nt<T>(ncols);
   if constexpr (!kIsF32<T>) {
     if (nt == 128)
       return os_lds_csub<T, 128, KQ>(x, n_x, cred, wt, wperm, ncols, bias, nbr, n_rows, K, order,

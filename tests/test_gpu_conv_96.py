@@ -13,14 +13,13 @@ import oracle
 from riemannengine_amd import abi
 from helpers import TOL, assert_rel, gpu_tables_and_map, random_coords, reference_passes, to_dev
 
-pytestmark = pytest.mark.gpu
-
 
 def _kernel(K, cred, ncols, n):
     name, splits = abi.conv_plan(torch.bfloat16, K, cred, ncols, n, n)
     return name + (" split" if splits > 1 else "")
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,ks,cin,cout,fwd,dx", [
     # split, 3^3: rows at and around 64- and 128-row tiles
     (1343, 3, 96, 96, "lds split", "lds split"), (1344, 3, 96, 96, "lds split", "lds split"),
@@ -59,6 +58,7 @@ def test_96_channel_layers_match_products(n, ks, cin, cout, fwd, dx):
         assert_rel(a.float().cpu().numpy(), ref.cpu().numpy(), TOL[torch.bfloat16], name)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,cin,cout", [
     (66001, 96, 96), (30000, 192, 96), (5000, 224, 160), (40001, 80, 224), (30001, 160, 96),
     (9000, 96, 96), (70000, 64, 96)])
@@ -75,3 +75,18 @@ def test_weight_gradient_with_part_empty_tiles(n, cin, cout):
     got, ref = abi.conv_weight_grad(x, gy, km, 27), abi.conv_backward_weight(x, gy, km, 27)
     assert_rel(got.float().cpu().numpy(), ref.float().cpu().numpy(), 2 ** -8, "dW")
     assert torch.equal(got, abi.conv_weight_grad(x, gy, km, 27))
+
+
+def test_96_column_tiles_without_a_gpu():
+    """Short reductions take the narrower tiles where 96-column ones would be
+    split; 192 columns that the kernel with 96-column tiles does not take run
+    in 64-column ones."""
+    bf16 = torch.bfloat16
+    for n in (10000, 23086):
+        assert abi.conv_plan(bf16, 27, 32, 96, n, n) == ("lds", 1)
+    assert abi.conv_plan(bf16, 27, 64, 96, 23086, 23086) == ("lds", 1)
+    assert abi.conv_plan(bf16, 27, 96, 96, 10000, 10000)[1] > 1
+    assert abi.conv_plan(bf16, 27, 64, 192, 10000, 10000)[1] > 1
+    for cred, ncols in ((192, 96), (96, 192), (192, 192)):  # a transposed stride-2 map
+        assert abi.conv_plan(bf16, 8, cred, ncols, 5100, 23086) == ("lds", 1)
+    assert abi.conv_plan(bf16, 27, 48, 192, 5036, 5036) == ("tiled", 3)
