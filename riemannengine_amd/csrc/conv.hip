@@ -2953,6 +2953,10 @@ static bool os_lds_shape(const T *x, int64_t n_x, int cred, const T *wt, const i
     return launch_os_lds<T, NT, 1, CSUB, G, W, KQ>(x, n_x, cred, wt, wperm, ncols, bias, nbr,
                                                    n_rows, K, order, y, splits, partial, s);
   } else { // bf16 128-column tiles: 4 waves per SIMD, one stage per barrier group
+    // two 96-channel chunks take the transposed copy: 192->256 on 101k rows 231
+    // us with it, 305 from untransposed weights (conv_os_kernel 273)
+    if (wtr && CSUB == 3 && cred != CSUB * kChOf<T>)
+      return false;
     if (splits <= 1) // without a split: one row group, twice the workgroups
       return launch_os_lds<T, NT, 1, CSUB, 1, 4, KQ>(x, n_x, cred, wt, wperm, ncols, bias, nbr,
                                                      n_rows, K, order, y, splits, partial, s, wtr);

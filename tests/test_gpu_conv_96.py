@@ -33,7 +33,8 @@ def _kernel(K, cred, ncols, n):
     (54657, 3, 96, 96, "lds", "lds"), (54655, 3, 128, 96, "lds", "lds"),
     (54656, 3, 64, 96, "lds", "lds"), (27329, 3, 32, 96, "lds", "lds"),
     (27327, 3, 192, 192, "lds", "lds"), (13697, 3, 32, 192, "lds", "lds split"),
-    (35009, 1, 96, 96, "lds", "lds"),
+    (35009, 1, 96, 96, "lds", "lds"), (54657, 3, 192, 128, "lds", "lds"),
+    (27329, 3, 192, 256, "lds", "lds"),
     # three mask words
     (200, 4, 96, 96, "lds split", "lds split"), (129, 4, 192, 64, "lds split", "lds split"),
     # padded and odd reductions into 96 columns
