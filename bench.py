@@ -325,7 +325,7 @@ def conv_kernels(dtype, K, cin, cout, n_in, n_out):
     """The kernel rhip_conv_plan names for a layer's forward and input gradient."""
     from riemannengine_amd import abi
     return {"forward": abi.conv_plan(dtype, K, cin, cout, n_in, n_out)[0],
-            "backward_input": abi.conv_plan(dtype, K, cout, cin, n_out, n_in)[0]}
+            "backward_input": abi.conv_plan(dtype, K, cout, cin, n_out, n_in, True)[0]}
 
 
 def _peak(dtype, kernel=None):

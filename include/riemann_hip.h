@@ -317,12 +317,13 @@ typedef enum rhip_conv_kernel {
 /*
  * Which kernel a call with a workspace and 16-byte aligned operands runs, and
  * into how many parts it splits the (offset, channel) stages (1: no split;
- * parts keep fp32 partial sums of n_rows x ncols in the workspace). A forward
- * reduces cred = cin channels of n_x = n_in rows to ncols = cout columns of
- * n_rows = n_out rows; an input gradient cout channels of n_out rows to cin
- * columns of n_in rows. Host only, for tests and tools.
+ * parts keep fp32 partial sums of n_rows x ncols in the workspace). pass:
+ * RHIP_PASS_FORWARD, which reduces cred = cin channels of n_x = n_in rows to
+ * ncols = cout columns of n_rows = n_out rows, or RHIP_PASS_INPUT_GRAD, which
+ * reduces cout channels of n_out rows to cin columns of n_in rows. Host only,
+ * for tests and tools.
  */
-int rhip_conv_plan(int32_t dtype, int32_t K, int32_t cred, int32_t ncols,
+int rhip_conv_plan(int32_t pass, int32_t dtype, int32_t K, int32_t cred, int32_t ncols,
                    int64_t n_x, int64_t n_rows, int32_t *kernel, int32_t *splits);
 
 /*

@@ -95,7 +95,7 @@ def _declare(lib):
                                                      _P(_sz)]),
         "rhip_conv_pass_workspace_bytes": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i32, _i64,
                                                           _i64, _i64, _P(_sz)]),
-        "rhip_conv_plan": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i64, _i64, _P(_i32),
+        "rhip_conv_plan": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i32, _i64, _i64, _P(_i32),
                                           _P(_i32)]),
         "rhip_conv_forward": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i32, _i32, _vp, _vp,
                                              _vp, _i64, _vp, _i32, _vp, _sz, _vp]),
@@ -503,12 +503,14 @@ def _conv_fwd_ws(K, cin, cout, dtype, dev, kmap: "KernelMap") -> torch.Tensor:
 CONV_KERNELS = ("rows", "thin", "padded", "small", "parts", "lds", "resident", "tiled")
 
 
-def conv_plan(dtype: torch.dtype, K: int, cred: int, ncols: int, n_x: int, n_rows: int):
+def conv_plan(dtype: torch.dtype, K: int, cred: int, ncols: int, n_x: int, n_rows: int,
+              input_grad: bool = False):
     """(kernel name, splits) of a forward or input gradient with a workspace
     and aligned operands, from rhip_conv_plan: cred channels of n_x rows to
     ncols columns of n_rows rows."""
     kernel, splits = _i32(0), _i32(0)
-    _check(lib().rhip_conv_plan(_dtype_code(dtype), K, cred, ncols, n_x, n_rows,
+    _check(lib().rhip_conv_plan(PASS_INPUT_GRAD if input_grad else PASS_FORWARD,
+                                _dtype_code(dtype), K, cred, ncols, n_x, n_rows,
                                 ctypes.byref(kernel), ctypes.byref(splits)), "rhip_conv_plan")
     return CONV_KERNELS[kernel.value], splits.value
 

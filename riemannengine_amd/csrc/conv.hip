@@ -3145,14 +3145,15 @@ struct ConvPlan {
   int how = RHIP_CONV_ROWS, splits = 1;
 };
 template <typename T>
-static ConvPlan conv_plan(int64_t n_x, int cred, int64_t n_rows, int ncols, int K, bool can_pad) {
+static ConvPlan conv_plan(bool forward, int64_t n_x, int cred, int64_t n_rows, int ncols, int K,
+                          bool can_pad) {
   const int credw = red_width(kIsF32<T> ? RHIP_F32 : RHIP_BF16, cred);
   if (!os_shape<T>(cred, credw, ncols, K)) {
     if (thin_runs(K, cred, n_x, sizeof(T), can_pad))
       return {RHIP_CONV_THIN};
     return {can_pad ? RHIP_CONV_PADDED : RHIP_CONV_ROWS};
   }
-  if (conv_small_takes<T>(n_rows, n_x, cred, ncols, K))
+  if (conv_small_takes<T>(forward, n_rows, n_x, cred, ncols, K))
     return {RHIP_CONV_SMALL};
   if (kIsF32<T> && conv_x3_takes(cred, ncols, K, n_x))
     return {RHIP_CONV_PARTS, conv_x3_splits(n_rows, cred, ncols, K)};
@@ -3762,10 +3763,10 @@ struct ConvWs {
   float *acc = nullptr;
 };
 
-static ConvPlan plan_of(int32_t dtype, int64_t n_x, int cred, int64_t n_rows, int ncols, int K,
-                        bool can_pad) {
-  return dtype == RHIP_F32 ? conv_plan<float>(n_x, cred, n_rows, ncols, K, can_pad)
-                           : conv_plan<__bf16>(n_x, cred, n_rows, ncols, K, can_pad);
+static ConvPlan plan_of(int32_t dtype, bool forward, int64_t n_x, int cred, int64_t n_rows,
+                        int ncols, int K, bool can_pad) {
+  return dtype == RHIP_F32 ? conv_plan<float>(forward, n_x, cred, n_rows, ncols, K, can_pad)
+                           : conv_plan<__bf16>(forward, n_x, cred, n_rows, ncols, K, can_pad);
 }
 
 // A forward (cin to cout) or an input gradient (cout to cin): what conv_plan's
@@ -3776,7 +3777,8 @@ static ConvWs carve_conv_pass(Carve &cv, bool forward, int32_t K, int32_t cin, i
   const size_t es = dtype == RHIP_F32 ? 4 : 2;
   int cred = forward ? cin : cout, ncols = forward ? cout : cin;
   const int64_t n_x = forward ? n_in : n_out, n_rows = forward ? n_out : n_in;
-  ConvPlan plan = plan_of(dtype, n_x, cred, n_rows, ncols, K, pads(dtype, cin, cout, K));
+  ConvPlan plan =
+      plan_of(dtype, forward, n_x, cred, n_rows, ncols, K, pads(dtype, cin, cout, K));
   if (plan.how == RHIP_CONV_THIN)
     return w;
   if (plan.how == RHIP_CONV_PADDED) {
@@ -3789,7 +3791,7 @@ static ConvWs carve_conv_pass(Carve &cv, bool forward, int32_t K, int32_t cin, i
     w.bad = cv.take<int>(1);
     cred = pad_width(cred);
     ncols = pad_width(ncols);
-    plan = plan_of(dtype, n_x, cred, n_rows, ncols, K, false);
+    plan = plan_of(dtype, forward, n_x, cred, n_rows, ncols, K, false);
   }
   w.wt_bytes = static_cast<size_t>(K) * ncols * red_width(dtype, cred) * es;
   if (plan.how == RHIP_CONV_PARTS)
@@ -3865,7 +3867,7 @@ static void conv_forward_into(const T *x, int64_t n_in, int32_t cin, const T *we
                               hipStream_t stream) {
   constexpr int32_t dtype = kIsF32<T> ? RHIP_F32 : RHIP_BF16;
   const int64_t per = static_cast<int64_t>(cin) * cout;
-  const int how = conv_plan<T>(n_in, cin, n_out, cout, K, w.px != nullptr).how;
+  const int how = conv_plan<T>(true, n_in, cin, n_out, cout, K, w.px != nullptr).how;
   if (how == RHIP_CONV_THIN) {
     conv_thin<T>(x, n_in, cin, weight, per, cout, 1, nullptr, cout, bias, nbr, n_out, K, out_order,
                  y, stream);
@@ -3945,7 +3947,7 @@ static void conv_backward_input_into(const T *grad_y, int64_t n_out, int32_t cou
   constexpr int32_t dtype = kIsF32<T> ? RHIP_F32 : RHIP_BF16;
   const int64_t per = static_cast<int64_t>(cin) * cout;
   const int how =
-      conv_plan<T>(n_out, cout, n_in, cin, K, w != nullptr && w->px != nullptr).how;
+      conv_plan<T>(false, n_out, cout, n_in, cin, K, w != nullptr && w->px != nullptr).how;
   if (how == RHIP_CONV_THIN && w != nullptr) {
     conv_thin<T>(grad_y, n_out, cout, weight, per, 1, cout, weight_perm, cin, nullptr, nbr_t, n_in,
                  K, in_order, grad_x, stream);
@@ -4097,15 +4099,18 @@ extern "C" int rhip_conv_pass_workspace_bytes(int32_t passes, int32_t K, int32_t
   });
 }
 
-extern "C" int rhip_conv_plan(int32_t dtype, int32_t K, int32_t cred, int32_t ncols, int64_t n_x,
-                              int64_t n_rows, int32_t *kernel, int32_t *splits) {
+extern "C" int rhip_conv_plan(int32_t pass, int32_t dtype, int32_t K, int32_t cred, int32_t ncols,
+                              int64_t n_x, int64_t n_rows, int32_t *kernel, int32_t *splits) {
   return guarded([&] {
     check_dtype(dtype);
+    RHIP_CHECK_ARG(pass == RHIP_PASS_FORWARD || pass == RHIP_PASS_INPUT_GRAD,
+                   "a forward or an input gradient");
     RHIP_CHECK_ARG(kernel != nullptr && splits != nullptr, "kernel or splits is null");
     RHIP_CHECK_ARG(K >= 1 && cred >= 1 && ncols >= 1, "sizes must be positive");
     RHIP_CHECK_ARG(n_x >= 0 && n_rows >= 0, "row counts must be >= 0");
     const bool can_pad = pads(dtype, cred, ncols, K);
-    const ConvPlan p = plan_of(dtype, n_x, cred, n_rows, ncols, K, can_pad);
+    const ConvPlan p =
+        plan_of(dtype, pass == RHIP_PASS_FORWARD, n_x, cred, n_rows, ncols, K, can_pad);
     *kernel = p.how;
     *splits = p.splits;
   });

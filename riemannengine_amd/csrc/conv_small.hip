@@ -87,8 +87,10 @@ __global__ __launch_bounds__(kThreads) void conv_small_kernel(
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb)
     acc[nb] = v4f{0.f, 0.f, 0.f, 0.f};
-  auto load_a = [&](int k, int ch) {
-    const int32_t id = __builtin_amdgcn_ds_bpermute(((k & 3) * 16 + i16) * 4, v[k >> 2]);
+  auto row_of = [&](int k) { // offset k's row for lane row i16
+    return __builtin_amdgcn_ds_bpermute(((k & 3) * 16 + i16) * 4, v[k >> 2]);
+  };
+  auto load_a = [&](int32_t id, int ch) {
     const uint32_t off =
         pick_off(static_cast<uint32_t>(id) * static_cast<uint32_t>(cred * sizeof(T)) +
                      static_cast<uint32_t>((ch * CH + g * EPL) * sizeof(T)),
@@ -97,16 +99,16 @@ __global__ __launch_bounds__(kThreads) void conv_small_kernel(
   };
   auto load_b = [&](int k, int ch, Frag (&b)[NB]) {
     const int64_t kw = wperm ? wperm[k] : k;
-    const int c = ch * CH + g * EPL;
+    const int c = ch * CH + g * EPL, n = col0 + i16;
+    const T *wk = w + kw * cred * ncols + (BY_CHANNEL ? c * ncols + n : n * cred + c);
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-      const int n = col0 + nb * 16 + i16;
       if constexpr (BY_CHANNEL) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          b[nb][e] = w[(kw * cred + c + e) * ncols + n];
+          b[nb][e] = wk[e * ncols + nb * 16];
       } else {
-        b[nb] = *reinterpret_cast<const Frag *>(w + (kw * ncols + n) * cred + c);
+        b[nb] = *reinterpret_cast<const Frag *>(wk + nb * 16 * cred);
       }
     }
   };
@@ -124,9 +126,13 @@ __global__ __launch_bounds__(kThreads) void conv_small_kernel(
         advance(kWaves);
     }
     Frag a[U], b[U][NB];
+    int32_t id[U];
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      a[u] = load_a(kj[u], cj[u]);
+      id[u] = row_of(kj[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      a[u] = load_a(id[u], cj[u]);
 #pragma unroll
     for (int u = 0; u < U; ++u)
       load_b(kj[u], cj[u], b[u]);
@@ -153,7 +159,7 @@ __global__ __launch_bounds__(kThreads) void conv_small_kernel(
     cc = 0;
     for (advance(wv); m; advance(kWaves)) {
       const int k = __builtin_ctz(m);
-      const Frag a = load_a(k, cc);
+      const Frag a = load_a(row_of(k), cc);
       Frag b[NB];
       load_b(k, cc, b);
       bool has[4]; // rows 4g .. 4g + 3
@@ -206,7 +212,7 @@ template <typename T> int small_nt(int ncols) {
 } // namespace
 
 template <typename T>
-bool conv_small_takes(int64_t n_rows, int64_t n_x, int cred, int ncols, int K) {
+bool conv_small_takes(bool forward, int64_t n_rows, int64_t n_x, int cred, int ncols, int K) {
   if (n_rows < 1 || n_x < 1 || K > 32 || cred % Mfma<T>::kCh != 0 || ncols % 16 != 0 ||
       n_x * cred * static_cast<int64_t>(sizeof(T)) > kBufMaxBytes)
     return false;
@@ -218,8 +224,25 @@ bool conv_small_takes(int64_t n_rows, int64_t n_x, int cred, int ncols, int K) {
   // 27.9 against 25.7 / 32.0 and 16->32 on 48k (167 MB) 19.4 / 21.4 against
   // 22.6 / 29.8; bf16 32->32 on 10k (36 MB) 18.1 / 15.3 against 14.2 / 11.5, but
   // 64->64 on 4.9k (67 MB) 19.0 / 15.5 against 22.0 / 19.2.
+  const bool f32 = std::is_same<T, float>::value;
   const int64_t read = ceil_div(n_rows, kRows) * K * cred * ncols * static_cast<int64_t>(sizeof(T));
-  return read <= (std::is_same<T, float>::value ? 100'000'000 : 40'000'000);
+  // Of 16 channels that is up to 58k rows, where many short workgroups cost
+  // more: fp32 16->16 on 23k rows 20.3 / 20.0 against 13.4 / 13.5, on 37k 13.1
+  // against 13.9 (dX), on 48k 16.2 / 14.4 against 17.2 / 16.0, transposed 2^3 on
+  // 101k 16.2 / 12 against 14.5 / 15.
+  if (n_rows > (f32 && forward && K <= 8 ? 70000 : 40000))
+    return false;
+  // With a few offsets the other kernels have no chain to shorten, and read
+  // the weights a fraction as often. 1^3 in fp32: dX 128->64 on 48k rows (99
+  // MB) 13 us against 65, 256->128 on 5k (41 MB) 12 against 19, but 192->192 on
+  // 3.1k (29 MB) 16 against 12. The forward, whose weights lie along the lanes
+  // and need no transposed copy here, gains longer: 256->128 on 5k 15 against
+  // 12, 64->64 on 23k (24 MB) 15 against 13, on 48k (49 MB) 15 against 23. bf16
+  // gains nothing there (128->256 on 3.1k 12 against 18).
+  if (K < 8)
+    return f32 && read <= (forward ? (n_rows <= 10000 ? 45'000'000 : 24'000'000)
+                                   : (n_rows <= 4096 ? 33'000'000 : 8'000'000));
+  return read <= (f32 ? 100'000'000 : 40'000'000);
 }
 
 template <typename T>
@@ -252,8 +275,8 @@ void conv_small(const T *x, int64_t n_x, int cred, const T *w, bool by_channel,
   RHIP_LAUNCH_CHECK();
 }
 
-template bool conv_small_takes<float>(int64_t, int64_t, int, int, int);
-template bool conv_small_takes<__bf16>(int64_t, int64_t, int, int, int);
+template bool conv_small_takes<float>(bool, int64_t, int64_t, int, int, int);
+template bool conv_small_takes<__bf16>(bool, int64_t, int64_t, int, int, int);
 template void conv_small<float>(const float *, int64_t, int, const float *, bool, const int32_t *,
                                 int, const float *, const int32_t *, int64_t, int,
                                 const int32_t *, float *, hipStream_t);

@@ -5,9 +5,9 @@
 
 namespace rhip {
 
-// Whether the small-map kernel runs this layer.
+// Whether the small-map kernel runs this pass (forward, else input gradient).
 template <typename T>
-bool conv_small_takes(int64_t n_rows, int64_t n_x, int cred, int ncols, int K);
+bool conv_small_takes(bool forward, int64_t n_rows, int64_t n_x, int cred, int ncols, int K);
 
 // y[order[j]][n] = sum_k x[nbr[k][j]] . w[perm(k)][.][n] (+ bias[n]); w slices
 // as [cred][ncols] (by_channel, fp32 only) or [ncols][cred].

@@ -14,8 +14,8 @@ from riemannengine_amd import abi
 from helpers import TOL, assert_rel, gpu_tables_and_map, random_coords, reference_passes, to_dev
 
 
-def _kernel(K, cred, ncols, n):
-    name, splits = abi.conv_plan(torch.bfloat16, K, cred, ncols, n, n)
+def _kernel(K, cred, ncols, n, dx=False):
+    name, splits = abi.conv_plan(torch.bfloat16, K, cred, ncols, n, n, dx)
     return name + (" split" if splits > 1 else "")
 
 
@@ -49,7 +49,7 @@ def test_96_channel_layers_match_products(n, ks, cin, cout, fwd, dx):
     c, _, _ = oracle.insert_and_map(random_coords(rng, 4 * n + 8, 3, span))
     km = gpu_tables_and_map(c[:n], c[:n], oracle.region_offsets(3, ks), same=True)[2]
     assert km.n_in == n
-    assert (_kernel(km.K, cin, cout, n), _kernel(km.K, cout, cin, n)) == (fwd, dx)
+    assert (_kernel(km.K, cin, cout, n), _kernel(km.K, cout, cin, n, True)) == (fwd, dx)
     x, gy, w = (to_dev(rng.standard_normal(s).astype(np.float32), torch.bfloat16)
                 for s in ((n, cin), (n, cout), (km.K, cin, cout)))
     print(f"96 n={n} ks={ks} {cin}->{cout} {fwd} / {dx}", flush=True)

@@ -45,8 +45,8 @@ def _same_but(clean, got, hit, column=None):
     (400, 5, 64, 20, torch.bfloat16, "padded"), (6000, 12, 40, 40, torch.float32, "padded")])
 def test_other_outputs_keep_their_bits(n, span, cin, cout, dtype, kernel):
     km = _map(n, span)
-    for cred, ncols in ((cin, cout), (cout, cin)):
-        name, splits = abi.conv_plan(dtype, 27, cred, ncols, n, n)
+    for cred, ncols, dx in ((cin, cout, False), (cout, cin, True)):
+        name, splits = abi.conv_plan(dtype, 27, cred, ncols, n, n, dx)
         assert name + (" split" if splits > 1 else "") == kernel
     g = torch.Generator(DEV).manual_seed(n)
     x, gy, w = (torch.randn(s, generator=g, device=DEV).to(dtype)

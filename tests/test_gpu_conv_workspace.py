@@ -27,8 +27,9 @@ def test_workspace_holds_the_split_sums(dtype):
                 for n in (500, 8000, 20000, 30000, 50000, 90000):
                     m = n // 3
                     room = _forward_bytes(K, cin, cout, dt, n, m)
-                    for n_rows, cred, ncols, n_x in ((m, cin, cout, n), (n, cout, cin, m)):
-                        _, sp = abi.conv_plan(dtype, K, cred, ncols, n_x, n_rows)
+                    for dx, n_rows, cred, ncols, n_x in ((False, m, cin, cout, n),
+                                                         (True, n, cout, cin, m)):
+                        _, sp = abi.conv_plan(dtype, K, cred, ncols, n_x, n_rows, dx)
                         assert sp == 1 or sp * n_rows * ncols * 4 <= room, (K, cin, cout, n)
 
 
