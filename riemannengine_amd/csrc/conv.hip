@@ -3155,7 +3155,7 @@ static ConvPlan conv_plan(bool forward, int64_t n_x, int cred, int64_t n_rows, i
   }
   if (conv_small_takes<T>(forward, n_rows, n_x, cred, ncols, K))
     return {RHIP_CONV_SMALL};
-  if (kIsF32<T> && conv_x3_takes(cred, ncols, K, n_x))
+  if (kIsF32<T> && conv_x3_takes(forward, cred, ncols, K, n_x, n_rows))
     return {RHIP_CONV_PARTS, conv_x3_splits(n_rows, cred, ncols, K)};
   const int splits = os_splits<T>(n_rows, cred, credw, ncols, K);
   if (cred == credw && K <= kLdsMaxK && os_lds_width<T>(cred) && n_x >= 1 &&

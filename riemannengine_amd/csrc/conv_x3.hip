@@ -477,17 +477,44 @@ void launch(dim3 grid, bool split, const float *x, int64_t n_x, const __bf16 *wt
 // template argument, of which each value adds 12 kernels; the five are those
 // that networks have most, and other multiples of 32 (160, 224, 320 and on)
 // stay on the fp32 MFMAs, where they were not compared.
-bool conv_x3_takes(int cred, int ncols, int K, int64_t n_x) {
+//
+// 32-column tiles split every row's operand again per tile: reductions that
+// the fp32 kernel has whole 64-channel stages for take them on maps of up to
+// 20,480 rows, where the splits below fill the chip (64->96 on 10k rows 46
+// against 45 us on the fp32 MFMAs, 128->96 71 / 89, 256->160 193 / 221; on 29k
+// rows 81 / 72, 144 / 140, 499 / 412). 96 and 192 channels it has not.
+//
+// Maps of up to 8 offsets with about one pair per row of the finer side
+// (stride-2 maps, their transposes, 1^D): the staged weights serve few
+// products. Measured on stride-2 maps, fp32 MFMA / this kernel: reductions of
+// 64 channels never gained (64->64 on 48k rows 14 / 17-24 us, transposed; 64->128
+// to 24k rows 27 / 32); the rest gain from about 4e8 pairs x channels x
+// columns (192->192 from 15,770 rows 38 / 33, 96->192 from 23k 33 / 28;
+// 128->128 from 23k 26.5 / 27), with one neighbour per row also from 40k rows
+// only (256->128 to 37k rows 36 / 40, to 48k 43 / 39), or, in the forward, for
+// which the fp32 kernel needs a transposed copy, from 20k to 192 columns and
+// more (192->192 to 23k 37 / 33, but dX 96->192 21 / 27).
+bool conv_x3_takes(bool forward, int cred, int ncols, int K, int64_t n_x, int64_t n_rows) {
   const bool width = cred == 64 || cred == 96 || cred == 128 || cred == 192 ||
                      cred == 256;
-  return width && ncols >= 64 && ncols % 32 == 0 && K <= kMaxK && n_x >= 1 &&
-         n_x * cred * static_cast<int64_t>(sizeof(float)) <= kBufMaxBytes;
+  if (!width || ncols < 64 || ncols % 32 != 0 || K > kMaxK || n_x < 1 ||
+      n_x * cred * static_cast<int64_t>(sizeof(float)) > kBufMaxBytes)
+    return false;
+  if (ncols % 64 != 0 && cred % 64 == 0 && cred != 192 && n_rows > 20480)
+    return false;
+  const int64_t fine = std::max(n_x, n_rows);
+  if (K <= 8 && K * std::min(n_x, n_rows) < 4 * fine) // under two pairs a row at best
+    return cred > 64 && fine * cred * ncols >= 400'000'000 &&
+           (n_rows <= n_x || n_rows >= 40000 || (forward && ncols >= 192 && n_rows >= 20000));
+  return true;
 }
 
 int conv_x3_splits(int64_t n_rows, int cred, int ncols, int K) {
   if (n_rows <= 0 || ncols % 32 != 0)
     return 1;
-  const int64_t blocks = ceil_div(n_rows, kWaves * x3_rg(K) * 16) * (ncols / x3_nt(ncols));
+  // a 32-column tile is half the work of a 64-column one
+  const int64_t blocks = std::max<int64_t>(
+      1, ceil_div(n_rows, kWaves * x3_rg(K) * 16) * (ncols / 32) / 2);
   const int64_t stages = static_cast<int64_t>(K) * (cred / 32);
   const int64_t want = (640 + blocks / 2) / blocks; // nearest
   return static_cast<int>(

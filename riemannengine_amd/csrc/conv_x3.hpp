@@ -5,9 +5,9 @@
 
 namespace rhip {
 
-// Whether the kernel takes a reduction of cred channels to ncols columns
-// over K offsets of n_x rows.
-bool conv_x3_takes(int cred, int ncols, int K, int64_t n_x);
+// Whether the kernel takes a reduction of cred channels to ncols columns over
+// K offsets, from n_x to n_rows rows (a forward, else an input gradient).
+bool conv_x3_takes(bool forward, int cred, int ncols, int K, int64_t n_x, int64_t n_rows);
 
 // Bytes of the three-part weights for K offsets.
 inline size_t conv_x3_weight_bytes(int K, int cred, int ncols) {

@@ -15,8 +15,6 @@ import oracle
 from riemannengine_amd import abi
 from helpers import DEV, gpu_tables_and_map, random_coords
 
-pytestmark = pytest.mark.gpu
-
 
 def _map(n, off, seed, span):
     c, _, _ = oracle.insert_and_map(random_coords(np.random.default_rng(seed), 6 * n + 8, 3, span))
@@ -37,12 +35,13 @@ def _device_sums(km, x, w, transpose=False):
     return y
 
 
-def _kernel(K, cred, ncols, n):
-    name, splits = abi.conv_plan(torch.float32, K, cred, ncols, n, n)
+def _kernel(K, cred, ncols, n, dx=False):
+    name, splits = abi.conv_plan(torch.float32, K, cred, ncols, n, n, dx)
     return name + (" split" if splits > 1 else "")
 
 
 # fwd, dx: the kernels of the forward and of the input gradient
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,ks,cin,cout,span,fwd,dx", [
     # split: rows at and around a 128-row tile's edges, both column tiles, every width
     (3711, 3, 64, 64, 11, "parts split", "parts split"),
@@ -54,11 +53,13 @@ def _kernel(K, cred, ncols, n):
     (640, 3, 256, 160, 7, "parts split", "tiled split"),
     (1000, 3, 160, 128, 8, "tiled split", "parts split"),
     (6145, 2, 64, 128, 13, "parts split", "parts split"),
+    (11009, 3, 64, 160, 15, "parts split", "tiled split"),
+    (18303, 3, 192, 96, 17, "parts split", "parts"),
     # whole
-    (55041, 3, 64, 64, 24, "parts", "parts"), (11009, 3, 64, 160, 15, "parts", "tiled split"),
-    (18303, 3, 96, 192, 17, "parts", "parts"), (13825, 3, 128, 256, 15, "parts", "parts split"),
+    (55041, 3, 64, 64, 24, "parts", "parts"), (22017, 3, 96, 160, 18, "parts", "tiled"),
+    (36481, 3, 96, 192, 21, "parts", "parts"), (13825, 3, 128, 256, 15, "parts", "parts split"),
     (13697, 3, 192, 256, 15, "parts", "parts split"), (13696, 3, 256, 256, 15, "parts", "parts"),
-    (98433, 1, 64, 64, 29, "parts", "parts"),
+    (98433, 1, 128, 128, 29, "parts", "parts"),
     # three and four mask words: 64-row tiles
     (191, 4, 64, 64, 5, "parts split", "parts split"),
     (192, 4, 128, 64, 5, "parts split", "parts split"),
@@ -72,7 +73,7 @@ def _kernel(K, cred, ncols, n):
     (260, 1, 64, 64, 5, "small", "small"), (300, 3, 192, 64, 5, "small", "small")])
 def test_x3_matches_64_bit_sums(n, ks, cin, cout, span, fwd, dx):
     km = _map(n, oracle.region_offsets(3, ks), seed=n + ks, span=span)
-    assert (_kernel(km.K, cin, cout, n), _kernel(km.K, cout, cin, n)) == (fwd, dx)
+    assert (_kernel(km.K, cin, cout, n), _kernel(km.K, cout, cin, n, True)) == (fwd, dx)
     g = torch.Generator(DEV).manual_seed(cin + cout)
     x, gy, w, b = (torch.randn(s, generator=g, device=DEV) for s in
                    ((n, cin), (n, cout), (km.K, cin, cout), (cout,)))
@@ -87,6 +88,7 @@ def test_x3_matches_64_bit_sums(n, ks, cin, cout, span, fwd, dx):
     assert float((gx - rgx).norm()) <= tol[1] * float(rgx.norm())
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,span,kernel", [(300, 5, "small"), (20000, 17, "parts split"),
                                            (55041, 24, "parts")])
 @pytest.mark.parametrize("where", ["x", "w"])
@@ -117,6 +119,7 @@ def test_x3_keeps_values_that_are_not_finite(bad, where, n, span, kernel):
     assert torch.allclose(y[big], ref[big], rtol=1e-5)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,cout", [(5000, 64), (14000, 256)])  # split, whole
 @pytest.mark.parametrize("ex,ew", [(-112, 0), (-118, 0), (-124, 12), (-130, 20), (-140, 24),
                                    (0, -112), (10, -124), (20, -130), (-60, -50), (60, -100)])
@@ -138,3 +141,24 @@ def test_x3_keeps_the_bits_of_small_operands(n, cout, ex, ew):
         # fp32's smallest step where the sums are that small
         step = 2.0 ** -149 * ref.numel() ** 0.5
         assert float((got.double() - ref).norm()) <= 1e-6 * float(ref.norm()) + step
+
+
+def test_x3_dispatch_without_a_gpu():
+    """Where the three-part kernel stops: narrow layers, part-empty column tiles
+    on large maps, stride-2 maps and 1^3 layers with little work."""
+    f32 = torch.float32
+
+    def name(*a):
+        return abi.conv_plan(f32, *a)[0]
+
+    assert name(27, 64, 64, 10000, 10000) == "parts" and name(27, 32, 64, 10000, 10000) != "parts"
+    assert name(27, 64, 48, 99999, 99999) != "parts"
+    assert name(27, 64, 96, 20480, 20480) == "parts" and name(27, 64, 96, 20481, 20481) != "parts"
+    assert name(27, 96, 96, 99999, 99999) == "parts" and name(27, 160, 64, 9999, 9999) != "parts"
+    # a stride-2 map and its transpose: channels, work, one neighbour a row
+    assert name(8, 128, 128, 48231, 10850) == "parts" and name(8, 64, 128, 48231, 10850) != "parts"
+    assert name(8, 128, 128, 23086, 5100) != "parts"
+    assert name(8, 256, 128, 10850, 48231) == "parts" and name(8, 256, 128, 8663, 37452) != "parts"
+    assert name(8, 192, 192, 5100, 23086) == "parts" != name(8, 192, 192, 5100, 23086, True)
+    assert name(1, 128, 128, 50000, 50000) == "parts" and name(1, 64, 64, 409553, 409553) != "parts"
+    assert name(8, 64, 64, 50000, 50000) == "parts"  # 2^3 at stride 1: several pairs a row

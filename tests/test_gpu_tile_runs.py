@@ -62,7 +62,7 @@ def _rows(n, step=1):
 @pytest.mark.parametrize("K,rows,width,dtype,kernels", [
     (33, 64, 16, torch.float32, ("tiled", "lds")), (33, 64, 16, torch.bfloat16, ("tiled",)),
     (33, 64, 32, torch.bfloat16, ("lds",)), (1, 16, 16, torch.float32, ("small",)),
-    (33, 64, 64, torch.float32, ("parts",)), (1, 128, 64, torch.float32, ("parts",))])
+    (33, 64, 64, torch.float32, ("parts",)), (1, 128, 128, torch.float32, ("parts",))])
 def test_every_tile_of_a_convolution_runs_once(K, rows, width, dtype, kernels):
     offsets = np.zeros((K, 3), np.int32)
     offsets[:, 2] = np.arange(K)
