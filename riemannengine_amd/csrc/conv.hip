@@ -2798,6 +2798,20 @@ static bool os_nt96(int cred, int credw, int ncols, int64_t n_rows, int K) {
   return !narrow || (kSplitBlocks + blocks / 2) / blocks <= 1;
 }
 
+// Whether a layer that no tiled kernel takes stays on one lane per output:
+// stride-2 maps and their transposes (2 to 8 offsets, about one pair per row of
+// the finer side) with little work. The padded copies are four launches, and
+// more than 96 im2col columns stage their weights for every 64 rows. Per call
+// on MI355X, here / thin or padded: transposed 2^3 13->13 (104 columns) on 23k
+// rows 12 / 21 us, on 101k 27 / 43, 20->20 (padded) on 23k 14 / 20, on 48k 22.5
+// / 21; not transposed 13->13 to 2k rows 13 / 24, 20->20 to 5k 19 / 21, to 11k 31
+// / 23.
+static bool rows_run(int K, int cred, int ncols, int64_t n_x, int64_t n_rows, bool thin) {
+  const int64_t fine = std::max(n_x, n_rows);
+  return K > 1 && K <= 8 && K * std::min(n_x, n_rows) < 4 * fine && (!thin || K * cred > 96) &&
+         fine * cred * ncols <= (n_rows > n_x ? 20'000'000 : 10'000'000);
+}
+
 // Splits of the offset axis for the MFMA kernel: a map with few rows and
 // wide channels gives too few workgroups to hide the gathers (one per CU
 // for 9k rows at 256 channels), so the (offset, channel chunk) stages are
@@ -3149,9 +3163,10 @@ static ConvPlan conv_plan(bool forward, int64_t n_x, int cred, int64_t n_rows, i
                           bool can_pad) {
   const int credw = red_width(kIsF32<T> ? RHIP_F32 : RHIP_BF16, cred);
   if (!os_shape<T>(cred, credw, ncols, K)) {
-    if (thin_runs(K, cred, n_x, sizeof(T), can_pad))
-      return {RHIP_CONV_THIN};
-    return {can_pad ? RHIP_CONV_PADDED : RHIP_CONV_ROWS};
+    const bool thin = thin_runs(K, cred, n_x, sizeof(T), can_pad);
+    if (rows_run(K, cred, ncols, n_x, n_rows, thin))
+      return {RHIP_CONV_ROWS};
+    return {thin ? RHIP_CONV_THIN : (can_pad ? RHIP_CONV_PADDED : RHIP_CONV_ROWS)};
   }
   if (conv_small_takes<T>(forward, n_rows, n_x, cred, ncols, K))
     return {RHIP_CONV_SMALL};

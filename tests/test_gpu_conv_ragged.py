@@ -11,7 +11,8 @@ import torch
 
 import oracle
 from riemannengine_amd import abi
-from helpers import DEV, TOL, assert_rel, gpu_tables_and_map, random_coords, to_dev
+from helpers import (DEV, TOL, assert_rel, gpu_tables_and_map, random_coords, reference_passes,
+                     to_dev)
 
 
 def test_ragged_weight_gradient_query_without_a_gpu():
@@ -141,3 +142,31 @@ def test_ragged_layers_keep_non_finite_values_to_their_pairs(cin, cout, dtype, b
             m = np.isfinite(r)
             assert m.any(), name
             assert_rel(a[m], r[m], TOL[dtype], name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,cin,cout,fwd,dx", [
+    (700, 13, 13, "rows", "rows"), (3000, 20, 24, "rows", "rows"), (900, 48, 20, "rows", "rows"),
+    (900, 3, 40, "thin", "rows"), (20000, 24, 40, "padded", "rows"),
+    (20000, 40, 64, "padded", "padded"), (700, 6, 12, "thin", "thin")])
+def test_ragged_layers_on_stride_maps(n, cin, cout, fwd, dx, dtype):
+    """2^3 stride-2 maps: with little work one lane per output, else thin or
+    padded, in both directions."""
+    rng = np.random.default_rng(n + cin)
+    side = int(np.ceil(n ** (1 / 3)))
+    grid = np.indices((1, side, side, side)).reshape(4, -1).T[:n]
+    c = rng.permutation(grid).astype(np.int32)
+    out = np.unique(oracle.stride(c, [2, 2, 2]), axis=0).astype(np.int32)
+    km = gpu_tables_and_map(c, out, oracle.region_offsets(3, 2))[2]
+    m = km.n_out
+    assert km.n_in == n and 8 * m < 4 * n
+    assert (abi.conv_plan(dtype, 8, cin, cout, n, m)[0],
+            abi.conv_plan(dtype, 8, cout, cin, m, n, True)[0]) == (fwd, dx)
+    x, gy = (to_dev(rng.standard_normal(s).astype(np.float32), dtype) for s in ((n, cin), (m, cout)))
+    w = to_dev((rng.standard_normal((8, cin, cout)) / 4).astype(np.float32), dtype)
+    print(f"ragged stride n={n} {cin}->{cout} {dtype}", flush=True)
+    got = (abi.conv_forward(x, w, km), abi.conv_backward_input(gy, w, km),
+           abi.conv_weight_grad(x, gy, km, 8))
+    for name, a, ref in zip(("Y", "dX", "dW"), got, reference_passes(km, x, gy, w)):
+        assert_rel(a.float().cpu().numpy(), ref.cpu().numpy(), TOL[dtype], name)
