@@ -3,8 +3,9 @@ forward with bias, input gradient and weight gradient at the edges of the
 thin kernels' tiles (64 positions, 96 im2col columns, 16 / 32 / 64 output
 columns; rows of 2-, 4- and 16-byte pieces) and of the padded widths (32, 64,
 128, 192, 256; copies that run on the small-map kernel, on larger maps and on
-more than 32 offsets on the tiled ones), and with weights or gradients that are not finite. Tolerance:
-norm-wise rel 1e-4 for fp32 and 2e-2 for bf16 (helpers.TOL)."""
+more than 32 offsets on the tiled ones), on stride-2 maps, and with weights or
+gradients that are not finite. Tolerance: norm-wise rel 1e-4 for fp32 and 2e-2
+for bf16 (helpers.TOL)."""
 import numpy as np
 import pytest
 import torch
